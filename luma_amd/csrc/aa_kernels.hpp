@@ -86,10 +86,24 @@ struct ChildRef {
     size_t ncell;
 };
 
+// n / d for n < 2^31 as one multiply-high, one add and one shift
+struct FastDiv {
+    uint32_t d, mul, sh;
+};
+inline FastDiv fast_div_of(uint32_t d) {
+    uint32_t sh = 0;
+    while ((uint64_t(1) << sh) < d) ++sh;
+    return FastDiv{d, (uint32_t)((((uint64_t(1) << sh) - d) << 32) / d + 1), sh};
+}
+__device__ __forceinline__ uint32_t fast_div(uint32_t n, const FastDiv &f) {
+    return (__umulhi(n, f.mul) + n) >> f.sh;
+}
+
 struct StepArgs {
     void *f;                      // population array
     size_t ps;                    // population stride in elements
     int nx, ny, nz;               // x = LUMA i (N_lim), y = j (M_lim), z = k (K_lim)
+    FastDiv dx, dy;               // division by nx, ny (kernels that take cells in linear order)
     const uint8_t *flags;         // per-cell flag byte (masked kernels only)
     const uint32_t *plain;        // plain-site bitmap of a labelled grid (k_plain_bits), or null
     // The double arrays below hold P::M elements: FP64, or (value, derivative) pairs in the
@@ -761,20 +775,50 @@ constexpr int periodic_waves() {
     return (std::is_same_v<P, P64> && !ODD && !STORE) ? 5 : 1;
 }
 
-template <int Q, class P, bool ODD, bool STORE, bool O32 = false>
+// FLAT: how the threads take the cells.
+//   kRows     one block per row segment (block sizes that divide the row leave no lane idle)
+//   kFlat     cells in linear order, rows starting on cache lines
+//   kFlatOdd  cells in linear order, rows starting anywhere: a population row shifted by c_y or
+//             c_z then shares its first and last line with other waves, so every access of the
+//             odd kernel is cached; the even kernel's stay line-aligned and non-temporal
+// With rows of 250 or 200 cells the row blocks leave lanes idle, and each row's non-temporal
+// accesses start and end inside a line that the neighbouring block fetches or writes again.
+enum CellOrder : int { kRows = 0, kFlat = 1, kFlatOdd = 2 };
+
+// the coordinates of linear cell index c
+__device__ __forceinline__ void cell_coords(const StepArgs &a, uint32_t c, int &x, int &y, int &z) {
+    const uint32_t row = fast_div(c, a.dx), pl = fast_div(row, a.dy);
+    x = (int)(c - row * (uint32_t)a.nx);
+    y = (int)(row - pl * (uint32_t)a.ny);
+    z = (int)pl;
+}
+
+template <int Q, class P, bool ODD, bool STORE, bool O32 = false, int FLAT = kRows>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(periodic_waves<P, ODD, STORE>())))
 void k_aa_periodic(StepArgs a) {
     using L = Lattice<Q>;
     using S = typename P::S;
     using T = typename P::T;
-    const int x = blockIdx.x * blockDim.x + threadIdx.x;
-    const int y = blockIdx.y, z = blockIdx.z + a.zoff;
-    if (x >= a.nx) return;
+    int x = 0, y = 0, z = 0;
+    uint32_t lin = 0;
+    if constexpr (FLAT != kRows) {
+        const uint32_t pl = (uint32_t)a.nx * (uint32_t)a.ny;
+        lin = blockIdx.x * 256u + threadIdx.x + pl * (uint32_t)a.zoff;
+        if (lin >= pl * (uint32_t)(a.nz - a.zoff)) return;
+        if constexpr (ODD) cell_coords(a, lin, x, y, z);
+    } else {
+        x = blockIdx.x * blockDim.x + threadIdx.x;
+        y = blockIdx.y;
+        z = blockIdx.z + a.zoff;
+        if (x >= a.nx) return;
+    }
     S *__restrict__ f = static_cast<S *>(a.f);
     const size_t ps = a.ps;
     const int nx = a.nx, ny = a.ny;
-    const size_t cell = O32 ? (size_t)((uint32_t)x + (uint32_t)nx * ((uint32_t)y + (uint32_t)ny * (uint32_t)z))
-                            : cell_of(x, y, z, nx, ny);
+    constexpr bool kNT = FLAT != kFlatOdd;   // row-aligned accesses of the odd kernel
+    const size_t cell = FLAT != kRows ? (size_t)lin
+                        : O32         ? (size_t)((uint32_t)x + (uint32_t)nx * ((uint32_t)y + (uint32_t)ny * (uint32_t)z))
+                                      : cell_of(x, y, z, nx, ny);
     Nbr nb;
     if constexpr (ODD) nb.init(x, y, z, nx, ny, a.nz);
     auto nbr = [&](int dx, int dy, int dz) -> size_t {
@@ -787,7 +831,7 @@ void k_aa_periodic(StepArgs a) {
         constexpr int v = decltype(vc)::value;
         constexpr int cx = L::c(v, 0), cy = L::c(v, 1), cz = L::c(v, 2);
         if constexpr (ODD)
-            fin[v] = ld<P, cx == 0>(elem_at<S, O32>(f + (size_t)L::opp(v) * ps, nbr(-cx, -cy, -cz)));
+            fin[v] = ld<P, kNT && cx == 0>(elem_at<S, O32>(f + (size_t)L::opp(v) * ps, nbr(-cx, -cy, -cz)));
         else
             fin[v] = ld<P>(elem_at<S, O32>(f + (size_t)v * ps, cell));
     });
@@ -799,7 +843,7 @@ void k_aa_periodic(StepArgs a) {
         constexpr int v = decltype(vc)::value;
         constexpr int cx = L::c(v, 0), cy = L::c(v, 1), cz = L::c(v, 2);
         if constexpr (ODD)
-            st<P, cx == 0>(elem_at<S, O32>(f + (size_t)v * ps, nbr(cx, cy, cz)), o);
+            st<P, kNT && cx == 0>(elem_at<S, O32>(f + (size_t)v * ps, nbr(cx, cy, cz)), o);
         else
             st<P>(elem_at<S, O32>(f + (size_t)L::opp(v) * ps, cell), o);
     };
@@ -949,7 +993,7 @@ __device__ __forceinline__ void gather_in(const StepArgs &a, int x, int y, int z
 }
 
 // gather_in for a plain site: every source is a regular pull, so no neighbour flag is read.
-template <int Q, class P, bool ODD>
+template <int Q, class P, bool ODD, bool NT = true>
 __device__ __forceinline__ void gather_plain(const StepArgs &a, size_t cell, const Nbr &nb, typename P::T *fin) {
     using L = Lattice<Q>;
     using S = typename P::S;
@@ -958,7 +1002,7 @@ __device__ __forceinline__ void gather_plain(const StepArgs &a, size_t cell, con
     static_for<Q>([&](auto vc) {
         constexpr int v = decltype(vc)::value;
         constexpr int cx = L::c(v, 0), cy = L::c(v, 1), cz = L::c(v, 2);
-        if constexpr (ODD) fin[v] = ld<P, cx == 0>(f + (size_t)L::opp(v) * ps + nb.at(-cx, -cy, -cz, a.nx, a.ny));
+        if constexpr (ODD) fin[v] = ld<P, NT && cx == 0>(f + (size_t)L::opp(v) * ps + nb.at(-cx, -cy, -cz, a.nx, a.ny));
         else fin[v] = ld<P>(f + (size_t)v * ps + cell);
     });
 }
@@ -1144,31 +1188,42 @@ __global__ __launch_bounds__(256) void k_aa_masked_list(StepArgs a, const int *c
 // k_aa_masked_list: the unlabelled kernel's pulls and pushes plus the body force where the
 // site carries one, with the arithmetic of masked_site.  It keeps the register use (and so the
 // occupancy) of the unlabelled kernel, which the boundary branches of masked_site would not.
-template <int Q, class P, bool ODD, bool STORE, bool FORCED>
+template <int Q, class P, bool ODD, bool STORE, bool FORCED, int FLAT = kRows>
 __global__ __launch_bounds__(256) void k_aa_plain(StepArgs a) {
     using L = Lattice<Q>;
     using S = typename P::S;
     using T = typename P::T;
     using M = typename P::M;
-    const int x = blockIdx.x * blockDim.x + threadIdx.x;
-    const int y = blockIdx.y, z = blockIdx.z;
-    if (x >= a.nx) return;
+    int x, y, z;
+    size_t cell;
     const int nx = a.nx, ny = a.ny;
-    const size_t cell = cell_of(x, y, z, nx, ny);
-    if (!((a.plain[cell >> 5] >> (cell & 31)) & 1u)) return;
+    if constexpr (FLAT != kRows) {
+        cell = blockIdx.x * 256u + threadIdx.x;
+        if (cell >= a.ncell) return;
+        if (!((a.plain[cell >> 5] >> (cell & 31)) & 1u)) return;
+        cell_coords(a, (uint32_t)cell, x, y, z);
+    } else {
+        x = blockIdx.x * blockDim.x + threadIdx.x;
+        y = blockIdx.y;
+        z = blockIdx.z;
+        if (x >= a.nx) return;
+        cell = cell_of(x, y, z, nx, ny);
+        if (!((a.plain[cell >> 5] >> (cell & 31)) & 1u)) return;
+    }
+    constexpr bool kNT = FLAT != kFlatOdd;
     S *__restrict__ f = static_cast<S *>(a.f);
     const size_t ps = a.ps;
     Nbr nb;
     nb.init(x, y, z, nx, ny, a.nz);
     T fin[Q];
-    gather_plain<Q, P, ODD>(a, cell, nb, fin);
+    gather_plain<Q, P, ODD, kNT>(a, cell, nb, fin);
     // the outlet side buffer of the next step (see StepArgs::xr_next)
     M *xr_row = (a.xr_next && x == nx - 3) ? mv<M>(a.xr_next) + (size_t)y + (size_t)ny * z : nullptr;
     const size_t xr_plane = (size_t)ny * a.nz;
     auto put = [&](auto vc, T o) {
         constexpr int v = decltype(vc)::value;
         constexpr int cx = L::c(v, 0), cy = L::c(v, 1), cz = L::c(v, 2);
-        if constexpr (ODD) st<P, cx == 0>(f + (size_t)v * ps + nb.at(cx, cy, cz, nx, ny), o);
+        if constexpr (ODD) st<P, kNT && cx == 0>(f + (size_t)v * ps + nb.at(cx, cy, cz, nx, ny), o);
         else st<P>(f + (size_t)L::opp(v) * ps + cell, o);
         if (xr_row) xr_row[(size_t)v * xr_plane] = M(static_cast<T>(static_cast<S>(o)));
     };

@@ -105,6 +105,8 @@ inline StepArgs make_args(const lumagpu_grid *g) {
     a.nx = g->d.N;
     a.ny = g->d.M;
     a.nz = g->d.K;
+    a.dx = fast_div_of((uint32_t)g->d.N);
+    a.dy = fast_div_of((uint32_t)g->d.M);
     a.flags = g->flags;
     a.plain = g->plain;
     a.force = g->force;

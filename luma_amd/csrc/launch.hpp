@@ -217,64 +217,80 @@ inline dim3 cell_grid(int nx, int ny, int nz) {
     return dim3((nx + b.x - 1) / b.x, ny, nz);
 }
 
+// How the grid kernels of a step take the cells.  Row blocks where one of cell_block's sizes
+// divides the row; else linear order, which leaves no lane idle and no line split between two
+// non-temporal accesses.  Even / odd kernel, us per step, by rows -> linear: 250 x 190 x 175 FP16
+// 217 / 166 -> 102 / 146; 200 x 171 x 150 FP64 334 / 262 -> 279 / 268; labelled plain sites
+// 180 x 131 x 150 FP32 130 / 116 -> 95 / 114, 288 x 96 x 96 FP32 (aligned rows, a block of 32
+// lanes at the end of each) 105 / 107 -> 77 / 75.
+template <class P>
+CellOrder cell_order(const StepArgs &a) {
+    // 2^31 cells bound the linear index; the tangent forms step small grids
+    if (a.nx % 128 == 0 || a.ncell >= (size_t(1) << 31) || std::is_same_v<typename P::M, Dual>) return kRows;
+    return (a.nx * sizeof(typename P::S)) % 128 == 0 ? kFlat : kFlatOdd;
+}
+// f(std::integral_constant<int, order>) for the run-time order
+template <class P, class F>
+void with_order(CellOrder o, F &&f) {
+    if constexpr (!std::is_same_v<typename P::M, Dual>) {
+        if (o == kFlat) return f(std::integral_constant<int, kFlat>{});
+        if (o == kFlatOdd) return f(std::integral_constant<int, kFlatOdd>{});
+    }
+    f(std::integral_constant<int, kRows>{});
+}
+// f(std::bool_constant<b>) for a run-time b
+template <class F>
+void with_bool(bool b, F &&f) {
+    if (b) f(std::true_type{});
+    else f(std::false_type{});
+}
+
 template <int Q, class P>
 hipError_t launch_step_q(const LaunchSpec &ls, const StepArgs &a, hipStream_t s) {
     const dim3 b = cell_block(a.nx), g = cell_grid(a.nx, a.ny, a.nz - 2 * a.zoff);
+    const CellOrder order = cell_order<P>(a);
+    const size_t cells = (size_t)a.nx * a.ny * (a.nz - 2 * a.zoff);
+    const dim3 fb(256), fg((unsigned)((cells + 255) / 256));
     if (ls.masked && ls.nmlist >= 0) {
         // AA steps touch only a site's own set of slots, so the two disjoint site sets can run
         // one after the other
         const dim3 lg((unsigned)((ls.nmlist + 255) / 256));
-        if (ls.odd) {
-            if (ls.forced) {
-                if (ls.store) k_aa_plain<Q, P, true, true, true><<<g, b, 0, s>>>(a);
-                else k_aa_plain<Q, P, true, false, true><<<g, b, 0, s>>>(a);
-            } else {
-                if (ls.store) k_aa_plain<Q, P, true, true, false><<<g, b, 0, s>>>(a);
-                else k_aa_plain<Q, P, true, false, false><<<g, b, 0, s>>>(a);
-            }
-            if (ls.nmlist > 0) {
-                if (ls.store) k_aa_masked_list<Q, P, true, true><<<lg, 256, 0, s>>>(a, ls.mlist, ls.nmlist);
-                else k_aa_masked_list<Q, P, true, false><<<lg, 256, 0, s>>>(a, ls.mlist, ls.nmlist);
-            }
-        } else {
-            if (ls.forced) {
-                if (ls.store) k_aa_plain<Q, P, false, true, true><<<g, b, 0, s>>>(a);
-                else k_aa_plain<Q, P, false, false, true><<<g, b, 0, s>>>(a);
-            } else {
-                if (ls.store) k_aa_plain<Q, P, false, true, false><<<g, b, 0, s>>>(a);
-                else k_aa_plain<Q, P, false, false, false><<<g, b, 0, s>>>(a);
-            }
-            if (ls.nmlist > 0) {
-                if (ls.store) k_aa_masked_list<Q, P, false, true><<<lg, 256, 0, s>>>(a, ls.mlist, ls.nmlist);
-                else k_aa_masked_list<Q, P, false, false><<<lg, 256, 0, s>>>(a, ls.mlist, ls.nmlist);
-            }
-        }
+        with_bool(ls.odd, [&](auto odd) {
+            with_bool(ls.store, [&](auto store) {
+                constexpr bool ODD = decltype(odd)::value, ST = decltype(store)::value;
+                with_bool(ls.forced, [&](auto forced) {
+                    with_order<P>(order, [&](auto fl) {
+                        constexpr int FL = decltype(fl)::value;
+                        k_aa_plain<Q, P, ODD, ST, decltype(forced)::value, FL>
+                            <<<FL == kRows ? g : fg, FL == kRows ? b : fb, 0, s>>>(a);
+                    });
+                });
+                if (ls.nmlist > 0) k_aa_masked_list<Q, P, ODD, ST><<<lg, 256, 0, s>>>(a, ls.mlist, ls.nmlist);
+            });
+        });
     } else if (ls.masked) {
-        if (ls.odd) {
-            if (ls.store) k_aa_masked<Q, P, true, true><<<g, b, 0, s>>>(a);
-            else k_aa_masked<Q, P, true, false><<<g, b, 0, s>>>(a);
-        } else {
-            if (ls.store) k_aa_masked<Q, P, false, true><<<g, b, 0, s>>>(a);
-            else k_aa_masked<Q, P, false, false><<<g, b, 0, s>>>(a);
-        }
-    } else if (!P::kShift && a.ncell * sizeof(typename P::S) < (size_t(1) << 32)) {
+        with_bool(ls.odd, [&](auto odd) {
+            with_bool(ls.store, [&](auto store) {
+                k_aa_masked<Q, P, decltype(odd)::value, decltype(store)::value><<<g, b, 0, s>>>(a);
+            });
+        });
+    } else {
         // FP64 planes below 4 GiB: 32-bit offsets from the plane bases (measured at 256^3:
         // 920 us against 947 us; the shifted forms are faster with 64-bit addresses)
-        if (ls.odd) {
-            if (ls.store) k_aa_periodic<Q, P, true, true, true><<<g, b, 0, s>>>(a);
-            else k_aa_periodic<Q, P, true, false, true><<<g, b, 0, s>>>(a);
-        } else {
-            if (ls.store) k_aa_periodic<Q, P, false, true, true><<<g, b, 0, s>>>(a);
-            else k_aa_periodic<Q, P, false, false, true><<<g, b, 0, s>>>(a);
-        }
-    } else {
-        if (ls.odd) {
-            if (ls.store) k_aa_periodic<Q, P, true, true><<<g, b, 0, s>>>(a);
-            else k_aa_periodic<Q, P, true, false><<<g, b, 0, s>>>(a);
-        } else {
-            if (ls.store) k_aa_periodic<Q, P, false, true><<<g, b, 0, s>>>(a);
-            else k_aa_periodic<Q, P, false, false><<<g, b, 0, s>>>(a);
-        }
+        const bool o32 = !P::kShift && a.ncell * sizeof(typename P::S) < (size_t(1) << 32);
+        with_bool(ls.odd, [&](auto odd) {
+            with_bool(ls.store, [&](auto store) {
+                with_order<P>(order, [&](auto fl) {
+                    constexpr bool ODD = decltype(odd)::value, ST = decltype(store)::value;
+                    constexpr int FL = decltype(fl)::value;
+                    const dim3 gg = FL == kRows ? g : fg, bb = FL == kRows ? b : fb;
+                    if constexpr (!P::kShift) {
+                        if (o32) return (void)(k_aa_periodic<Q, P, ODD, ST, true, FL><<<gg, bb, 0, s>>>(a));
+                    }
+                    k_aa_periodic<Q, P, ODD, ST, false, FL><<<gg, bb, 0, s>>>(a);
+                });
+            });
+        });
     }
     return hipGetLastError();
 }
