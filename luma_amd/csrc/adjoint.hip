@@ -398,7 +398,7 @@ int adj_run(lumagpu_grid *g, int nsteps, int every, const double dir[3], int bac
                 hipError_t e = g->nedge ? launch_edges(g, a, 0) : hipSuccess;
                 if (e == hipSuccess) e = launch_adj_collide<P>(g, a, ab);
                 if (e == hipSuccess && nface) {
-                    const dim3 fb(64), fg((unsigned)((nface + 63) / 64));
+                    const dim3 fb(64), fg((unsigned)((nface + 63) / 64), (unsigned)(g->Q + 2));
                     const int *fcp = static_cast<const int *>(face_cells.p);
                     double *fp = static_cast<double *>(fpart.p);
                     const bool odd = g->parity == 0;
@@ -416,7 +416,7 @@ int adj_run(lumagpu_grid *g, int nsteps, int every, const double dir[3], int bac
                     }
                 }
                 if (e == hipSuccess && g->nedge) {
-                    const dim3 eb(64), eg((unsigned)((g->nedge + 63) / 64));
+                    const dim3 eb(64), eg((unsigned)((g->nedge + 63) / 64), (unsigned)(g->Q + 4));
                     double *db = static_cast<double *>(dbar.p), *tb = static_cast<double *>(tbar.p);
                     double *ep = static_cast<double *>(epart.p);
                     const int *nc_p = static_cast<const int *>(enb_cell.p), *np_p = static_cast<const int *>(enb_ptr.p);

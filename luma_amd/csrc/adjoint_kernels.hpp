@@ -61,33 +61,31 @@ __device__ __forceinline__ bool regularised_boundary_site(const StepArgs &a, uns
     return a.regularised && (ty == kVelocity || ty == kPressure);
 }
 
-// Transposed Jacobian of a regularised velocity face site's update (regularised_face, :313-510,
-// then BGK, :765-790) at its streamed populations g (absolute): one forward-mode (Dual) pass per
-// population, one for omega and one for the inlet profile scale (u_in -> s u_in at s = 1).
-// gbar_v = sum_w lam_w d f'_w / d g_v; omb and inb the two parameter derivatives.  The site
-// carries no body force (the adjoint refuses IB supports on velocity sites).
+// One forward-mode (Dual) pass of the transposed Jacobian of a regularised velocity face site's
+// update (regularised_face, :313-510, then BGK, :765-790) at its streamed populations g
+// (absolute): lam . d f' / d p for seed s, p = population s for s < Q, omega for s = Q and the
+// inlet profile scale (u_in -> p u_in at p = 1) for s = Q + 1.  The site carries no body force
+// (the adjoint refuses IB supports on velocity sites).
 template <int Q>
-__device__ void adj_regularised_face(const StepArgs &a, unsigned fl, int y, const double *g, const double *lam,
-                                     double *gbar, double &omb, double &inb) {
+__device__ double adj_regularised_face(const StepArgs &a, unsigned fl, int y, const double *g, const double *lam,
+                                       int s) {
     using L = Lattice<Q>;
     const int ncode = (fl >> kNormalShift) & 7;
     const double r = a.ramp_reg;
     const double vin0[3] = {a.uin[y] * r, a.uin[a.ny + y] * r, (L::D == 3) ? a.uin[2 * a.ny + y] * r : 0.0};
-    for (int s = 0; s < Q + 2; ++s) {
-        Dual ga[Q];
-        for (int v = 0; v < Q; ++v) ga[v] = Dual(g[v], v == s ? 1.0 : 0.0);
-        Dual vin[3];
-        for (int d = 0; d < 3; ++d) vin[d] = Dual(vin0[d], s == Q + 1 ? vin0[d] : 0.0);
-        Dual rr, uu[3];
-        regularised_face<Q, Dual>(ga, ncode, vin, Dual(a.rho_in), Dual(a.cs2), Dual(a.den2), rr, uu);
-        const CollideExact<Q, Dual> col{rr, {uu[0], uu[1], uu[2]}, Dual(a.omega, s == Q ? 1.0 : 0.0),
-                                        Dual(a.cs2), Dual(a.den2), nullptr};
-        double acc = 0.0;
-        for (int w = 0; w < Q; ++w) acc += lam[w] * col(w, ga[w]).d;
-        if (s < Q) gbar[s] = acc;
-        else if (s == Q) omb = acc;
-        else inb = acc;
-    }
+    Dual ga[Q];
+#pragma unroll
+    for (int v = 0; v < Q; ++v) ga[v] = Dual(g[v], v == s ? 1.0 : 0.0);
+    Dual vin[3];
+    for (int d = 0; d < 3; ++d) vin[d] = Dual(vin0[d], s == Q + 1 ? vin0[d] : 0.0);
+    Dual rr, uu[3];
+    regularised_face<Q, Dual>(ga, ncode, vin, Dual(a.rho_in), Dual(a.cs2), Dual(a.den2), rr, uu);
+    const CollideExact<Q, Dual> col{rr, {uu[0], uu[1], uu[2]}, Dual(a.omega, s == Q ? 1.0 : 0.0),
+                                    Dual(a.cs2), Dual(a.den2), nullptr};
+    double acc = 0.0;
+#pragma unroll
+    for (int w = 0; w < Q; ++w) acc += lam[w] * col(w, ga[w]).d;
+    return acc;
 }
 
 // Transposed collision Jacobian at every fluid site: gbar = (d f'/d g)^T lam, fbar =
@@ -198,14 +196,17 @@ __global__ __launch_bounds__(256, (sizeof(typename P::T) == 8 && Q == 19) ? 2 : 
     if (threadIdx.x == 0) b.part[block_linear()] = s;
 }
 
-// Regularised velocity face sites, one thread per listed site (cells[i]): gbar from
-// adj_regularised_face at the site's streamed populations; the omega and inlet-scale
-// derivatives per site in fpart[i] and fpart[n + i].
+// Regularised velocity face sites (cells[i]): gbar from adj_regularised_face at the site's
+// streamed populations; the omega and inlet-scale derivatives per site in fpart[i] and
+// fpart[n + i].  One thread per (site, seed), the sites of one seed side by side: a face is a
+// few dozen to a few thousand sites, and the Q + 2 passes of a site one after another made one
+// wave's chain the kernel's whole time (58 sites of a 220 x 60 FP64 channel: 113 -> 14 us).
 template <int Q, class P, bool ODD>
-__global__ void k_adj_faces(StepArgs a, AdjArgs<typename P::T> b, const int *cells, int n, double *fpart) {
+__global__ __launch_bounds__(64) void k_adj_faces(StepArgs a, AdjArgs<typename P::T> b, const int *cells, int n,
+                                                  double *fpart) {
     using L = Lattice<Q>;
     using T = typename P::T;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const int i = blockIdx.x * blockDim.x + threadIdx.x, s = blockIdx.y;
     if (i >= n) return;
     const size_t cell = (size_t)cells[i];
     const int nx = a.nx, ny = a.ny;
@@ -214,32 +215,31 @@ __global__ void k_adj_faces(StepArgs a, AdjArgs<typename P::T> b, const int *cel
     nb.init(x, y, z, nx, ny, a.nz);
     T fin[Q];
     gather_in<Q, P, ODD>(a, x, y, z, cell, nb, kVelocity, fin);
-    double g[Q], lam[Q], gb[Q];
+    double g[Q], lam[Q];
+#pragma unroll
     for (int v = 0; v < Q; ++v) {
         g[v] = double(fin[v]) + (P::kShift ? L::w(v) * a.rho0 : 0.0);
         lam[v] = double(b.lam[(size_t)v * a.ncell + cell]);
     }
-    double om = 0.0, in = 0.0;
-    adj_regularised_face<Q>(a, a.flags[cell], y, g, lam, gb, om, in);
-    for (int v = 0; v < Q; ++v) b.gbar[(size_t)v * a.ncell + cell] = T(gb[v]);
-    fpart[i] = om;
-    fpart[n + i] = in;
+    const double d = adj_regularised_face<Q>(a, a.flags[cell], y, g, lam, s);
+    if (s < Q) b.gbar[(size_t)s * a.ncell + cell] = T(d);
+    else fpart[(s - Q) * n + i] = d;
 }
 
-// Sites that extrapolate from their two inward neighbours (k_edge_sites), one thread per site:
-// edge and corner velocity sites (regularised_edge with the density 2 rho(x+n) - rho(x+2n) from
-// the neighbours' sweep-1 values) and pressure faces (regularised_pressure with the tangential
-// velocity 2 u(x+n) - u(x+2n)), then BGK.  The site's own gbar comes from forward-mode passes
+// Sites that extrapolate from their two inward neighbours (k_edge_sites), one thread per (site,
+// seed) as in k_adj_faces: edge and corner velocity sites (regularised_edge with the density
+// 2 rho(x+n) - rho(x+2n) from the neighbours' sweep-1 values) and pressure faces
+// (regularised_pressure with the tangential velocity 2 u(x+n) - u(x+2n)), then BGK.  The site's own gbar comes from forward-mode passes
 // over its populations; the extrapolated quantities' adjoints (dbar[i], or tbar[3 i + d] for
 // the velocity components) reach the neighbours' streamed populations through
 // d rho / d g_v = 1 and d u_d / d g_v = (c_vd - u_d) / rho (k_adj_edge_nbrs); omega and
 // inlet-scale derivatives per site in epart[i] and epart[n + i].
 template <int Q, class P, bool ODD>
-__global__ void k_adj_edges(StepArgs a, EdgeArgs e, AdjArgs<typename P::T> b, double *dbar, double *tbar,
-                            double *epart) {
+__global__ __launch_bounds__(64) void k_adj_edges(StepArgs a, EdgeArgs e, AdjArgs<typename P::T> b,
+                                                  double *dbar, double *tbar, double *epart) {
     using L = Lattice<Q>;
     using T = typename P::T;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const int i = blockIdx.x * blockDim.x + threadIdx.x, s = blockIdx.y;
     if (i >= e.n) return;
     const size_t cell = (size_t)e.cell[i];
     const int nx = a.nx, ny = a.ny;
@@ -263,37 +263,35 @@ __global__ void k_adj_edges(StepArgs a, EdgeArgs e, AdjArgs<typename P::T> b, do
     const double r = a.ramp_reg;
     const double vin0[3] = {a.uin[y] * r, a.uin[ny + y] * r, (L::D == 3) ? a.uin[2 * ny + y] * r : 0.0};
     // seeds: populations 0..Q-1, then omega, then the extrapolated density and the inlet scale
-    // (velocity edges) or the three extrapolated velocity components (pressure faces)
-    double omb = 0.0, inb = 0.0, db = 0.0, tb[3] = {0.0, 0.0, 0.0};
-    const int ns = Q + (pressure ? 4 : 3);
-    for (int s = 0; s < ns; ++s) {
-        Dual fa[Q];
-        for (int v = 0; v < Q; ++v) fa[v] = Dual(g[v], v == s ? 1.0 : 0.0);
-        Dual rr, uu[3], fout[Q];
-        if (pressure) {
-            Dual vt[3];
-            for (int d = 0; d < 3; ++d) vt[d] = Dual(vt0[d], s == Q + 1 + d ? 1.0 : 0.0);
-            regularised_pressure<Q, Dual>(fa, ncode, vt, Dual(a.rho_p), Dual(a.cs2), Dual(a.den2), rr, uu);
-        } else {
-            Dual vin[3];
-            for (int d = 0; d < 3; ++d) vin[d] = Dual(vin0[d], s == Q + 2 ? vin0[d] : 0.0);
-            regularised_edge<Q, Dual>(fa, n, vin, Dual(dens0, s == Q + 1 ? 1.0 : 0.0), Dual(a.cs2), Dual(a.den2), rr,
-                                      uu);
-        }
-        collide_exact<Q, Dual>(fa, rr, uu, static_cast<const Dual *>(nullptr), Dual(a.omega, s == Q ? 1.0 : 0.0),
-                               Dual(a.cs2), Dual(a.den2), fout);
-        double acc = 0.0;
-        for (int w = 0; w < Q; ++w) acc += lam[w] * fout[w].d;
-        if (s < Q) b.gbar[(size_t)s * a.ncell + cell] = T(acc);
-        else if (s == Q) omb = acc;
-        else if (pressure) tb[s - Q - 1] = acc;
-        else if (s == Q + 1) db = acc;
-        else inb = acc;
+    // (velocity edges, s = Q + 3 idle) or the three extrapolated velocity components (pressure
+    // faces)
+    Dual fa[Q];
+#pragma unroll
+    for (int v = 0; v < Q; ++v) fa[v] = Dual(g[v], v == s ? 1.0 : 0.0);
+    Dual rr, uu[3], fout[Q];
+    if (pressure) {
+        Dual vt[3];
+        for (int d = 0; d < 3; ++d) vt[d] = Dual(vt0[d], s == Q + 1 + d ? 1.0 : 0.0);
+        regularised_pressure<Q, Dual>(fa, ncode, vt, Dual(a.rho_p), Dual(a.cs2), Dual(a.den2), rr, uu);
+    } else {
+        Dual vin[3];
+        for (int d = 0; d < 3; ++d) vin[d] = Dual(vin0[d], s == Q + 2 ? vin0[d] : 0.0);
+        regularised_edge<Q, Dual>(fa, n, vin, Dual(dens0, s == Q + 1 ? 1.0 : 0.0), Dual(a.cs2), Dual(a.den2), rr, uu);
     }
-    dbar[i] = db;
-    for (int d = 0; d < 3; ++d) tbar[3 * (size_t)i + d] = tb[d];
-    epart[i] = omb;
-    epart[e.n + i] = inb;
+    collide_exact<Q, Dual>(fa, rr, uu, static_cast<const Dual *>(nullptr), Dual(a.omega, s == Q ? 1.0 : 0.0),
+                           Dual(a.cs2), Dual(a.den2), fout);
+    double acc = 0.0;
+#pragma unroll
+    for (int w = 0; w < Q; ++w) acc += lam[w] * fout[w].d;
+    // every output of the site has one seed that writes it; the other kind's are zero
+    if (s < Q) b.gbar[(size_t)s * a.ncell + cell] = T(acc);
+    else if (s == Q) epart[i] = acc;
+    else if (pressure) tbar[3 * (size_t)i + (s - Q - 1)] = acc;
+    else if (s == Q + 1) dbar[i] = acc;
+    else if (s == Q + 2) epart[e.n + i] = acc;
+    if (pressure && s == Q) dbar[i] = epart[e.n + i] = 0.0;
+    if (!pressure && s == Q)
+        for (int d = 0; d < 3; ++d) tbar[3 * (size_t)i + d] = 0.0;
 }
 
 // The extrapolation's reach into the neighbours: gbar_v(x) += sum over the sites that
