@@ -106,6 +106,7 @@ struct StepArgs {
     FastDiv dx, dy;               // division by nx, ny (kernels that take cells in linear order)
     const uint8_t *flags;         // per-cell flag byte (masked kernels only)
     const uint32_t *plain;        // plain-site bitmap of a labelled grid (k_plain_bits), or null
+    const uint64_t *link;         // link word of every cell of a small labelled grid (k_links)
     // The double arrays below hold P::M elements: FP64, or (value, derivative) pairs in the
     // tangent form; kernels address them through mv<M>.
     const double *force;          // force_xyz, SoA [d*ncell + cell], read where flagged
@@ -1036,6 +1037,94 @@ __global__ void k_plain_bits(const uint8_t *flags, int nx, int ny, int nz, size_
     plain[w] = bits;
 }
 
+// The link word of a site: where each of its pulls comes from, so that a boundary site's step
+// reads one word instead of its neighbours' flag bytes one dependent round trip later.
+//   bits 0..17    the source x - c_v is solid (halfway bounce-back); a push along v ends in a
+//                 solid cell exactly when the pull of opp v starts in one
+//   bits 18..35   the source is a forced-equilibrium velocity site
+//   bits 36..53   the source is an ExtrapolateRight site
+//   bit  54       some source is a refined or transition site: the flags decide (gather_in)
+//   bits 55..58   the site's type, bits 59..61 its wall-normal code
+// k_aa_masked on the 256 x 256 FP32 cavity, even / odd: 6.6 / 10.1 -> 4.3 / 5.6 us.
+constexpr int kLinkVel = 18, kLinkExt = 36, kLinkOther = 54, kLinkType = 55, kLinkNormal = 59;
+constexpr uint64_t kLinkMask = (uint64_t(1) << 18) - 1;
+
+template <int Q>
+__global__ __launch_bounds__(256) void k_links(const uint8_t *flags, int nx, int ny, int nz, int regularised,
+                                               const int *cells, size_t n, uint64_t *link) {
+    using L = Lattice<Q>;
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const size_t cell = cells ? (size_t)cells[i] : i;
+    const int x = (int)(cell % nx), y = (int)((cell / nx) % ny), z = (int)(cell / ((size_t)nx * ny));
+    Nbr nb;
+    nb.init(x, y, z, nx, ny, nz);
+    const unsigned fl = flags[cell];
+    uint64_t w = ((uint64_t)(fl & kTypeMask) << kLinkType) | ((uint64_t)((fl >> kNormalShift) & 7) << kLinkNormal);
+    static_for<Q - 1>([&](auto vc) {
+        constexpr int v = decltype(vc)::value;
+        const int t = flags[nb.at(-L::c(v, 0), -L::c(v, 1), -L::c(v, 2), nx, ny)] & kTypeMask;
+        if (t == kSolid) w |= uint64_t(1) << v;
+        if (t == kVelocity && !regularised) w |= uint64_t(1) << (kLinkVel + v);
+        if (t == kExtrapRight) w |= uint64_t(1) << (kLinkExt + v);
+        if (t == kRefined || t == kTL2C) w |= uint64_t(1) << kLinkOther;
+    });
+    // a refined or transition site's rest population is its own "source"
+    const int t = fl & kTypeMask;
+    if (t == kRefined || t == kTL2C) w |= uint64_t(1) << kLinkOther;
+    link[i] = w;
+}
+
+// gather_in from the link word of a site without refined or transition sources.  HAVE: fin
+// already holds the regular pulls.
+template <int Q, class P, bool ODD, bool HAVE>
+__device__ __forceinline__ void gather_links(const StepArgs &a, uint64_t w, int y, size_t cell, const Nbr &nb, int ty,
+                                             typename P::T *fin) {
+    using L = Lattice<Q>;
+    using S = typename P::S;
+    using T = typename P::T;
+    const S *__restrict__ f = static_cast<const S *>(a.f);
+    const size_t ps = a.ps;
+    const int nx = a.nx, ny = a.ny;
+    // the even layout keeps a bounced population where a regular pull reads it
+    if constexpr (ODD || !HAVE) {
+        static_for<Q>([&](auto vc) {
+            constexpr int v = decltype(vc)::value;
+            constexpr int cx = L::c(v, 0), cy = L::c(v, 1), cz = L::c(v, 2);
+            if constexpr (!ODD) {
+                fin[v] = ld<P>(f + (size_t)v * ps + cell);
+            } else if constexpr (HAVE) {
+                if (v < Q - 1 && ((w >> v) & 1)) fin[v] = ld<P, false>(f + (size_t)v * ps + cell);
+            } else {
+                const size_t reg = (size_t)L::opp(v) * ps + nb.at(-cx, -cy, -cz, nx, ny);
+                const bool solid = v < Q - 1 && ((w >> v) & 1);
+                fin[v] = ld<P, false>(f + (solid ? (size_t)v * ps + cell : reg));
+            }
+        });
+    }
+    if ((w >> kLinkVel) & kLinkMask) {
+        static_for<Q - 1>([&](auto vc) {
+            constexpr int v = decltype(vc)::value;
+            if ((w >> (kLinkVel + v)) & 1) {
+                // as in gather_in: the source row's profile, or with the ramp this row's
+                const int js = a.ramp_on ? y : nb.ys[1 - L::c(v, 1)];
+                const double r = a.ramp_feq;
+                const double us[3] = {a.uin[js] * r, a.uin[ny + js] * r, (L::D == 3) ? a.uin[2 * ny + js] * r : 0.0};
+                fin[v] = feq_store<Q, P>(v, a.rho_in, us, a);
+            }
+        });
+    }
+    // an outlet site is its own rest population's source
+    if (((w >> kLinkExt) & kLinkMask) || ty == kExtrapRight) {
+        static_for<Q>([&](auto vc) {
+            constexpr int v = decltype(vc)::value;
+            if (v < Q - 1 ? (int)((w >> (kLinkExt + v)) & 1) : (ty == kExtrapRight ? 1 : 0))
+                fin[v] = T(mv<typename P::M>(a.xr)[(size_t)v * ny * a.nz + nb.ys[1 - L::c(v, 1)] +
+                                                   (size_t)ny * nb.zs[1 - L::c(v, 2)]]);
+        });
+    }
+}
+
 // Regularised velocity face for a gathered site: rho, u of the BC and the regularised
 // populations in storage convention.
 template <int Q, class P>
@@ -1056,11 +1145,11 @@ __device__ __forceinline__ void velocity_site(const StepArgs &a, unsigned fl, in
 }
 
 // labelled grid: solid (HWBB), velocity (regularised or forced equilibrium), ExtrapolateRight
-// sources, refinement transition layers, body force.  SPEC: issue the regular pulls before the
-// site's flags are known (most sites are plain, and their step then waits on one memory round
-// trip less); sites that turn out otherwise gather again.
+// sources, refinement transition layers, body force.  w: the site's link word.  SPEC: issue the
+// regular pulls before the link word is known (most sites are plain, and their step then waits
+// on one memory round trip less); the pulls from other sources replace theirs.
 template <int Q, class P, bool ODD, bool STORE, bool SPEC = false>
-__device__ __forceinline__ void masked_site(const StepArgs &a, int x, int y, int z) {
+__device__ __forceinline__ void masked_site(const StepArgs &a, int x, int y, int z, const uint64_t *wp) {
     using L = Lattice<Q>;
     using S = typename P::S;
     using T = typename P::T;
@@ -1070,18 +1159,18 @@ __device__ __forceinline__ void masked_site(const StepArgs &a, int x, int y, int
     nb.init(x, y, z, nx, ny, a.nz);
     T fin[Q], fout[Q];
     if constexpr (SPEC) gather_plain<Q, P, ODD>(a, cell, nb, fin);
+    const uint64_t w = *wp;
     const unsigned fl = a.flags[cell];
-    const int ty = fl & kTypeMask;
+    const int ty = (int)(w >> kLinkType) & 15;
     // sites LUMA's sweep 1 skips (:91-95)
     if (ty == kSolid || ty == kRefined || (!a.regularised && ty == kVelocity)) return;
     // edge and corner velocity sites and pressure sites run in k_edge_sites after this kernel
-    if (ty == kPressure || (ty == kVelocity && ((fl >> kNormalShift) & 7) == kNormalEdge)) return;
+    if (ty == kPressure || (ty == kVelocity && ((w >> kLinkNormal) & 7) == kNormalEdge)) return;
     S *__restrict__ f = static_cast<S *>(a.f);
     const size_t ps = a.ps;
 
-    const bool plain = a.plain && ((a.plain[cell >> 5] >> (cell & 31)) & 1u);
-    if (!plain) gather_in<Q, P, ODD>(a, x, y, z, cell, nb, ty, fin);
-    else if constexpr (!SPEC) gather_plain<Q, P, ODD>(a, cell, nb, fin);
+    if ((w >> kLinkOther) & 1) gather_in<Q, P, ODD>(a, x, y, z, cell, nb, ty, fin);
+    else gather_links<Q, P, ODD, SPEC>(a, w, y, cell, nb, ty, fin);
 
     using M = typename P::M;
     const M *F = nullptr;
@@ -1156,7 +1245,8 @@ __device__ __forceinline__ void masked_site(const StepArgs &a, int x, int y, int
         constexpr int cx = L::c(v, 0), cy = L::c(v, 1), cz = L::c(v, 2);
         if constexpr (ODD) {
             const size_t dst = nb.at(cx, cy, cz, nx, ny);
-            if (!plain && (a.flags[dst] & kTypeMask) == kSolid)
+            // x + c_v is the source of the pull along opp v
+            if (v < Q - 1 && ((w >> L::opp(v)) & 1))
                 st<P>(f + (size_t)L::opp(v) * ps + cell, fout[v]);
             else
                 st<P, cx == 0>(f + (size_t)v * ps + dst, fout[v]);
@@ -1168,20 +1258,24 @@ __device__ __forceinline__ void masked_site(const StepArgs &a, int x, int y, int
 
 template <int Q, class P, bool ODD, bool STORE>
 __global__ __launch_bounds__(256) void k_aa_masked(StepArgs a) {
-    const int x = blockIdx.x * blockDim.x + threadIdx.x;
+    const int x = blockIdx.x * blockDim.x + threadIdx.x, y = blockIdx.y, z = blockIdx.z;
     if (x >= a.nx) return;
-    masked_site<Q, P, ODD, STORE, true>(a, x, blockIdx.y, blockIdx.z);
+    masked_site<Q, P, ODD, STORE, true>(a, x, y, z, a.link + cell_of(x, y, z, a.nx, a.ny));
 }
 
-// The same step for a list of sites: on large labelled grids the plain sites run in
-// k_aa_plain and this kernel takes the rest (boundary, transition and bounce-back neighbours).
+// The same step for a list of sites (link words by list entry): on large labelled grids the
+// plain sites run in k_aa_plain and this kernel takes the rest (boundary, transition and
+// bounce-back neighbours).  One wave per block: the list holds a surface of the grid, a few
+// hundred waves whose accesses are long latencies, and blocks of four left half of the CUs
+// without one.  Even / odd, us per step, against flag bytes and blocks of four: inlet and outlet
+// planes of 288 x 96 x 96 FP32 41 / 34 -> 31 / 21, walls of 180 x 131 x 150 FP32 20 / 22 -> 8 / 9.
 template <int Q, class P, bool ODD, bool STORE>
-__global__ __launch_bounds__(256) void k_aa_masked_list(StepArgs a, const int *cells, int n) {
+__global__ __launch_bounds__(64) void k_aa_masked_list(StepArgs a, const int *cells, const uint64_t *links, int n) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    const int cell = cells[i];
-    const int x = cell % a.nx, y = (cell / a.nx) % a.ny, z = cell / (a.nx * a.ny);
-    masked_site<Q, P, ODD, STORE>(a, x, y, z);
+    int x, y, z;
+    cell_coords(a, (uint32_t)cells[i], x, y, z);
+    masked_site<Q, P, ODD, STORE>(a, x, y, z, links + i);
 }
 
 // The step of the plain sites of a labelled grid (k_plain_bits), every other site left to

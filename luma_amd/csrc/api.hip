@@ -242,7 +242,7 @@ int begin_step(lumagpu_grid *g) {
 // The second half: stream, BC, macro (with the IB force), Guo forcing and BGK collision in one
 // pass, the edge/corner and pressure sites around it, then the swap (AA parity) and ++t.
 int end_step(lumagpu_grid *g, int subcycle, hipEvent_t e0, hipEvent_t e1) {
-    LaunchSpec ls{g->Q, g->masked != 0, g->parity == 0, g->store_macro != 0, g->mlist, g->nmlist};
+    LaunchSpec ls{g->Q, g->masked != 0, g->parity == 0, g->store_macro != 0, g->mlist, g->link, g->nmlist};
     ls.forced = g->all_forced || g->ibm || g->host_forced;
     StepArgs a = make_args(g);
     a.subcycle = subcycle;
@@ -398,7 +398,7 @@ std::vector<uint8_t> graph_key(lumagpu_grid *g) {
                             x->d.level, x->d.regularised, x->xr_sel, x->xr_ready, x->xr_fold,
                             x->host_forced, x->ibm != nullptr};
         put(misc, sizeof misc);
-        const void *ptrs[] = {x->mlist, x->edge, x->erho, x->stream, x->force};
+        const void *ptrs[] = {x->mlist, x->link, x->edge, x->erho, x->stream, x->force};
         put(ptrs, sizeof ptrs);
         put(&x->gravity, sizeof x->gravity);
         ibm_graph_key(x, key);
@@ -669,6 +669,33 @@ static int build_mlist(lumagpu_grid *g) {
     return 0;
 }
 
+// link words of the sites k_aa_masked or k_aa_masked_list steps, from the flags on the device
+static int build_links(lumagpu_grid *g) {
+    std::vector<uint8_t> types(g->ncell);
+    for (size_t c = 0; c < g->ncell; ++c) types[c] = g->hflags[c] & ~kForcedBit;
+    if (g->link && types == g->link_types) return 0;   // only force bits changed
+    const size_t n = g->nmlist >= 0 ? (size_t)g->nmlist : g->ncell;
+    (void)hipStreamSynchronize(g->stream);
+    (void)hipFree(g->link);
+    g->link = nullptr;
+    g->link_types.clear();
+    if (n > 0) {
+        if (hipMalloc(&g->link, n * sizeof(uint64_t)) != hipSuccess) {
+            g->link = nullptr;
+            return fail(LUMAGPU_ENOMEM, "link word allocation failed");
+        }
+        const unsigned nb = (unsigned)((n + 255) / 256);
+        const int *cells = g->nmlist >= 0 ? g->mlist : nullptr;
+        if (g->Q == 9)
+            k_links<9><<<nb, 256, 0, g->stream>>>(g->flags, g->d.N, g->d.M, g->d.K, g->d.regularised, cells, n, g->link);
+        else
+            k_links<19><<<nb, 256, 0, g->stream>>>(g->flags, g->d.N, g->d.M, g->d.K, g->d.regularised, cells, n, g->link);
+        HIP_TRY(hipGetLastError());
+    }
+    g->link_types = std::move(types);
+    return 0;
+}
+
 int upload_flags(lumagpu_grid *g) {
     if (g->hflags.size() != g->ncell) return fail(LUMAGPU_ESTATE, "host flag array does not cover the grid");
     if (!g->flags && hipMalloc(&g->flags, g->ncell) != hipSuccess)
@@ -683,6 +710,7 @@ int upload_flags(lumagpu_grid *g) {
     else k_plain_bits<19><<<nb, 256, 0, g->stream>>>(g->flags, g->d.N, g->d.M, g->d.K, g->ncell, g->plain);
     HIP_TRY(hipGetLastError());
     if (int r = build_mlist(g)) return r;
+    if (int r = build_links(g)) return r;
     return build_stale(g);
 }
 hipError_t outlet_prepass(const lumagpu_grid *g) { return launch_extrap(g); }
@@ -771,6 +799,7 @@ int lumagpu_grid_destroy(lumagpu_grid *g) {
     (void)hipFree(g->stale_idx);
     (void)hipFree(g->stale_cells);
     (void)hipFree(g->mlist);
+    (void)hipFree(g->link);
     (void)hipFree(g->force);
     (void)hipFree(g->uin);
     (void)hipFree(g->rho);

@@ -33,6 +33,9 @@ struct lumagpu_grid {
     std::vector<int> stale_list;      // host copy of stale_cells
     // large labelled grids: the sites the plain-site kernel leaves to the labelled one
     int *mlist = nullptr;
+    // link words (k_links): of the listed sites, or of every cell of a grid stepped in one launch
+    uint64_t *link = nullptr;
+    std::vector<uint8_t> link_types;  // the flag bytes (without the force bit) they were built from
     int nmlist = -1;                  // < 0: one labelled launch over the grid
     std::vector<uint8_t> mlist_types; // the site types mlist was built from
     // the captured two-step graph of this hierarchy (root grids), reused while its key holds
@@ -109,6 +112,7 @@ inline StepArgs make_args(const lumagpu_grid *g) {
     a.dy = fast_div_of((uint32_t)g->d.M);
     a.flags = g->flags;
     a.plain = g->plain;
+    a.link = g->nmlist < 0 ? g->link : nullptr;
     a.force = g->force;
     a.uin = g->uin;
     a.rho_out = g->rho;

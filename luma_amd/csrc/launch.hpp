@@ -19,6 +19,7 @@ struct LaunchSpec {
     bool store;     // write rho, u
     // labelled grid stepped as plain sites (k_aa_plain) plus a list of the others
     const int *mlist = nullptr;
+    const uint64_t *mlinks = nullptr;   // their link words
     int nmlist = -1;   // < 0: one k_aa_masked launch over the grid
     bool forced = true;   // some site may carry a body force (IB bodies, gravity, a set force)
 };
@@ -254,7 +255,7 @@ hipError_t launch_step_q(const LaunchSpec &ls, const StepArgs &a, hipStream_t s)
     if (ls.masked && ls.nmlist >= 0) {
         // AA steps touch only a site's own set of slots, so the two disjoint site sets can run
         // one after the other
-        const dim3 lg((unsigned)((ls.nmlist + 255) / 256));
+        const dim3 lg((unsigned)((ls.nmlist + 63) / 64));
         with_bool(ls.odd, [&](auto odd) {
             with_bool(ls.store, [&](auto store) {
                 constexpr bool ODD = decltype(odd)::value, ST = decltype(store)::value;
@@ -265,7 +266,7 @@ hipError_t launch_step_q(const LaunchSpec &ls, const StepArgs &a, hipStream_t s)
                             <<<FL == kRows ? g : fg, FL == kRows ? b : fb, 0, s>>>(a);
                     });
                 });
-                if (ls.nmlist > 0) k_aa_masked_list<Q, P, ODD, ST><<<lg, 256, 0, s>>>(a, ls.mlist, ls.nmlist);
+                if (ls.nmlist > 0) k_aa_masked_list<Q, P, ODD, ST><<<lg, 64, 0, s>>>(a, ls.mlist, ls.mlinks, ls.nmlist);
             });
         });
     } else if (ls.masked) {

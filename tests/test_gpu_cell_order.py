@@ -52,3 +52,25 @@ def test_labelled_channel(shape):
     m = case.lattyp != setups.SOLID
     for a, b in zip(got, want):
         assert np.array_equal(a[m], b[m])
+
+
+# the site list of large labelled grids (2^20 cells and more): walls, a forced-equilibrium inlet and an
+# outlet (their sources and the outlet's own populations), by link words, one wave per block
+def test_listed_sites():
+    case = setups.uniform_inflow_3d(131, 92, 88, 0.03, 0.6)
+    case.lattyp[1:-1, 0, :] = setups.SOLID
+    case.lattyp[40:47, 30:37, 20:31] = setups.SOLID
+    case.forced = False
+    o = OracleGrid(3, 19, case.N, case.M, case.K, omega=case.omega, regularised=False, edges=case.edges)
+    o.set_labels(case.lattyp)
+    o.set_positions(case.xpos, case.ypos, case.zpos)
+    o.set_inlet(case.ux_in, case.uy_in, case.uz_in)
+    o.init_feq(case.rho, case.u)
+    o.run(4, 8)
+    print("[order] listed sites", flush=True)
+    with GpuGrid.from_case(case, "fp64", store_macro=True) as g:
+        g.run(4)
+        got = (g.download_f(),) + g.download_macro()
+    m = (case.lattyp == setups.FLUID) | (case.lattyp == setups.EXTRAP_RIGHT)
+    for a, b in zip(got, (o.get_f(),) + o.get_macro()):
+        assert np.array_equal(a[m], b[m])
