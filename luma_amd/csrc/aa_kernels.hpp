@@ -387,22 +387,55 @@ __device__ __forceinline__ void collide_exact(const T *fin, T rho, const T *u, c
     for (int v = 0; v < Q; ++v) fout[v] = c(v, fin[v]);
 }
 
+// Every population's feq_exact of one site, an opposite pair sharing its two divisions as in
+// CollideExact::pair (the same bits).
+template <int Q, class T>
+__device__ __forceinline__ void feq_all(T rho, const T *u, T cs2, T den2, T *fe) {
+    using L = Lattice<Q>;
+    static_for<(Q - 1) / 2>([&](auto pc) {
+        constexpr int v = 2 * decltype(pc)::value;
+        constexpr int c0 = L::c(v, 0), c1 = L::c(v, 1), c2 = L::c(v, 2);
+        T A, B;
+        if constexpr (L::D == 3) {
+            A = (T(c0) * u[0]) + (T(c1) * u[1]) + (T(c2) * u[2]);
+            B = (T(c0 * c0) - cs2) * (u[0] * u[0]) + (T(c1 * c1) - cs2) * (u[1] * u[1]) +
+                (T(c2 * c2) - cs2) * (u[2] * u[2]) + T(2 * c0 * c1) * u[0] * u[1] +
+                T(2 * c0 * c2) * u[0] * u[2] + T(2 * c1 * c2) * u[1] * u[2];
+        } else {
+            A = (T(c0) * u[0]) + (T(c1) * u[1]);
+            B = (T(c0 * c0) - cs2) * (u[0] * u[0]) + (T(c1 * c1) - cs2) * (u[1] * u[1]) +
+                T(2 * c0 * c1) * u[0] * u[1];
+        }
+        const T a = A / cs2, b = B / den2;
+        fe[v] = rho * T(L::w(v)) * (T(1.0) + a + b);
+        fe[v + 1] = rho * T(L::w(v + 1)) * (T(1.0) + (-a) + b);
+    });
+    fe[Q - 1] = feq_exact<Q, T>(Q - 1, rho, u, cs2, den2);
+}
+
 // The reconstruction shared by the face conditions (:432-508): unknown populations (those
 // entering through the face) by non-equilibrium bounce-back, then every population rebuilt from
-// feq(rho, u) and the non-equilibrium stress of the result.
+// feq(rho, u) and the non-equilibrium stress of the result.  In 2D the equilibria are held from
+// one use to the next; in 3D they would not fit beside the populations.
 template <int Q, class T>
 __device__ __forceinline__ void regularise_face_set(T *fa, int ndir, int nsgn, T rho, const T *u, T cs2, T den2) {
     using L = Lattice<Q>;
     T Sxx = 0, Syy = 0, Sxy = 0, Szz = 0, Sxz = 0, Syz = 0;
+    constexpr bool kHold = Q == 9;
+    T fe[kHold ? Q : 1];
+    if constexpr (kHold) feq_all<Q, T>(rho, u, cs2, den2, fe);
+    auto feq = [&](int v) {
+        if constexpr (kHold) return fe[v];
+        else return feq_exact<Q, T>(v, rho, u, cs2, den2);
+    };
     // Unknown populations first (non-equilibrium bounce-back), in v order as LUMA does:
     // each v's update reads fa[opp v], which for an unknown v is a known population.
 #pragma unroll
     for (int v = 0; v < Q; ++v) {
         const int c0 = L::c(v, 0), c1 = L::c(v, 1), c2 = L::c(v, 2);
         const int o = L::opp(v);
-        if (L::c(v, ndir) == nsgn)
-            fa[v] = feq_exact<Q, T>(v, rho, u, cs2, den2) + (fa[o] - feq_exact<Q, T>(o, rho, u, cs2, den2));
-        const T fneq = fa[v] - feq_exact<Q, T>(v, rho, u, cs2, den2);
+        if (L::c(v, ndir) == nsgn) fa[v] = feq(v) + (fa[o] - feq(o));
+        const T fneq = fa[v] - feq(v);
         Sxx += T(c0 * c0) * fneq;
         Syy += T(c1 * c1) * fneq;
         Sxy += T(c0 * c1) * fneq;
@@ -415,7 +448,7 @@ __device__ __forceinline__ void regularise_face_set(T *fa, int ndir, int nsgn, T
 #pragma unroll
     for (int v = 0; v < Q; ++v) {
         const int c0 = L::c(v, 0), c1 = L::c(v, 1), c2 = L::c(v, 2);
-        fa[v] = feq_exact<Q, T>(v, rho, u, cs2, den2) +
+        fa[v] = feq(v) +
                 (T(L::w(v)) / den2) *
                     (((T(c0 * c0) - cs2) * Sxx) + ((T(c1 * c1) - cs2) * Syy) +
                      ((T(c2 * c2) - cs2) * Szz) + (T(2.0) * T(c0) * T(c1) * Sxy) +
@@ -1037,6 +1070,48 @@ __global__ void k_plain_bits(const uint8_t *flags, int nx, int ny, int nz, size_
     plain[w] = bits;
 }
 
+// Regularised velocity face for a gathered site: rho, u of the BC and the regularised
+// populations in storage convention.
+template <int Q, class P>
+__device__ __forceinline__ void velocity_site(const StepArgs &a, unsigned fl, int y, typename P::T *fin,
+                                              typename P::T &rr, typename P::T *uu) {
+    using L = Lattice<Q>;
+    using T = typename P::T;
+    const int ny = a.ny;
+    const int ncode = (fl >> kNormalShift) & 7;
+    const double r = a.ramp_reg;
+    T vin[3] = {T(a.uin[y] * r), T(a.uin[ny + y] * r), (L::D == 3) ? T(a.uin[2 * ny + y] * r) : T(0)};
+    T fa[Q];
+#pragma unroll
+    for (int v = 0; v < Q; ++v) fa[v] = P::kShift ? fin[v] + T(L::w(v) * a.rho0) : fin[v];
+    regularised_face<Q, T>(fa, ncode, vin, T(a.rho_in), T(a.cs2), T(a.den2), rr, uu);
+#pragma unroll
+    for (int v = 0; v < Q; ++v) fin[v] = P::kShift ? fa[v] - T(L::w(v) * a.rho0) : fa[v];
+}
+
+// A regularised velocity face site from its gathered populations: the BC gives rho, u (no macro
+// on this site, :101-107), then the collision.
+template <int Q, class P>
+__device__ __forceinline__ void velocity_collide(const StepArgs &a, unsigned fl, int y, typename P::T *fin,
+                                                 const typename P::M *F, typename P::T *fout, typename P::M &rho,
+                                                 typename P::M *u) {
+    using T = typename P::T;
+    using M = typename P::M;
+    T rr, uu[3];
+    velocity_site<Q, P>(a, fl, y, fin, rr, uu);
+    if constexpr (!P::kShift) {
+        const CollideExact<Q, T> col{rr, {uu[0], uu[1], uu[2]}, omega_of<T>(a), T(a.cs2), T(a.den2), F};
+        collide_pairs<Q>(col, fin, fout);
+    } else {
+        const CollideShift<Q, T> col(rr - 1.0f, uu, F, shift_k(a));
+        collide_pairs<Q>(col, fin, fout);
+    }
+    rho = M(rr);
+    u[0] = M(uu[0]);
+    u[1] = M(uu[1]);
+    u[2] = M(uu[2]);
+}
+
 // The link word of a site: where each of its pulls comes from, so that a boundary site's step
 // reads one word instead of its neighbours' flag bytes one dependent round trip later.
 //   bits 0..17    the source x - c_v is solid (halfway bounce-back); a push along v ends in a
@@ -1125,25 +1200,6 @@ __device__ __forceinline__ void gather_links(const StepArgs &a, uint64_t w, int 
     }
 }
 
-// Regularised velocity face for a gathered site: rho, u of the BC and the regularised
-// populations in storage convention.
-template <int Q, class P>
-__device__ __forceinline__ void velocity_site(const StepArgs &a, unsigned fl, int y, typename P::T *fin,
-                                              typename P::T &rr, typename P::T *uu) {
-    using L = Lattice<Q>;
-    using T = typename P::T;
-    const int ny = a.ny;
-    const int ncode = (fl >> kNormalShift) & 7;
-    const double r = a.ramp_reg;
-    T vin[3] = {T(a.uin[y] * r), T(a.uin[ny + y] * r), (L::D == 3) ? T(a.uin[2 * ny + y] * r) : T(0)};
-    T fa[Q];
-#pragma unroll
-    for (int v = 0; v < Q; ++v) fa[v] = P::kShift ? fin[v] + T(L::w(v) * a.rho0) : fin[v];
-    regularised_face<Q, T>(fa, ncode, vin, T(a.rho_in), T(a.cs2), T(a.den2), rr, uu);
-#pragma unroll
-    for (int v = 0; v < Q; ++v) fin[v] = P::kShift ? fa[v] - T(L::w(v) * a.rho0) : fa[v];
-}
-
 // labelled grid: solid (HWBB), velocity (regularised or forced equilibrium), ExtrapolateRight
 // sources, refinement transition layers, body force.  w: the site's link word.  SPEC: issue the
 // regular pulls before the link word is known (most sites are plain, and their step then waits
@@ -1182,20 +1238,7 @@ __device__ __forceinline__ void masked_site(const StepArgs &a, int x, int y, int
 
     M rho, u[3];
     if (ty == kVelocity) {
-        // regularised velocity face: the BC gives rho, u; no macro on this site (:101-107)
-        T rr, uu[3];
-        velocity_site<Q, P>(a, fl, y, fin, rr, uu);
-        if constexpr (!P::kShift) {
-            const CollideExact<Q, T> col{rr, {uu[0], uu[1], uu[2]}, omega_of<T>(a), T(a.cs2), T(a.den2), F};
-            collide_pairs<Q>(col, fin, fout);
-        } else {
-            const CollideShift<Q, T> col(rr - 1.0f, uu, F, shift_k(a));
-            collide_pairs<Q>(col, fin, fout);
-        }
-        rho = M(rr);
-        u[0] = M(uu[0]);
-        u[1] = M(uu[1]);
-        u[2] = M(uu[2]);
+        velocity_collide<Q, P>(a, fl, y, fin, F, fout, rho, u);
     } else if (ty == kExtrapRight) {
         // outlet site: streamed (sources right of it are the x = 0 column, through the periodic
         // wrap; sources on the outlet itself give the value two cells left, :246-251) and

@@ -364,6 +364,41 @@ int run_fused_graph(lumagpu_grid *g, int reps) {
     return 0;
 }
 
+// Small 2D grids take several steps per launch (k_multi2d): one level, no bodies, nothing that
+// changes from step to step, and site types whose sources the window holds.  2^18 cells: above,
+// a step fills the chip by itself, and the window's repeated cells cost more than launches.
+bool multi_ok(const lumagpu_grid *g) {
+    return g->Q == 9 && (g->d.precision == LUMAGPU_FP64 || g->d.precision == LUMAGPU_FP32S) && !g->parent &&
+           g->kids.empty() && ibm_marker_count(g) == 0 && !g->gravity_on && !(g->ramp_time > 0.0) &&
+           !(g->re_ramp > 0.0) && g->nedge == 0 && g->simple_types && g->ncell <= (size_t(1) << 18) && g->has_state;
+}
+
+// up to n steps from the post-local layout, as many as whole launches take; *done: steps run
+int run_multi(lumagpu_grid *g, int n, int *done) {
+    *done = 0;
+    if (!g->f2) {
+        if (hipMalloc(&g->f2, g->ps * g->Q * g->elem) != hipSuccess) {
+            // one step per launch needs no second array
+            (void)hipGetLastError();
+            g->f2 = nullptr;
+            return 0;
+        }
+    }
+    // begin_step's state for a grid without bodies
+    g->all_forced = g->sweep1_zero = 0;
+    while (n - *done >= 2) {
+        const int H = plan_multi2d(g->d.N, g->d.M, n - *done, g->d.precision == LUMAGPU_FP64);
+        const StepArgs a = make_args(g);
+        const hipError_t e = g->d.precision == LUMAGPU_FP64 ? launch_multi2d_f64(a, g->f2, H, g->store_macro, g->stream)
+                                                            : launch_multi2d_f32s(a, g->f2, H, g->store_macro, g->stream);
+        if (e != hipSuccess) return fail(LUMAGPU_EHIP, std::string("multi-step launch: ") + hipGetErrorString(e));
+        std::swap(g->f, g->f2);
+        g->t += H;
+        *done += H;
+    }
+    return 0;
+}
+
 // no host work inside a step anywhere in the hierarchy (flexible bodies download forces and
 // run the FEM on the host every step)
 bool graph_ok(const lumagpu_grid *g) {
@@ -704,6 +739,10 @@ int upload_flags(lumagpu_grid *g) {
     if (!g->plain && hipMalloc(&g->plain, nw * sizeof(uint32_t)) != hipSuccess)
         return fail(LUMAGPU_ENOMEM, "plain-site bitmap allocation failed");
     HIP_TRY(hipMemcpyAsync(g->flags, g->hflags.data(), g->ncell, hipMemcpyHostToDevice, g->stream));
+    g->simple_types = std::all_of(g->hflags.begin(), g->hflags.end(), [](uint8_t f) {
+        const int t = f & kTypeMask;
+        return t == kSolid || t == kFluid || t == kVelocity;
+    });
     g->host_forced = std::any_of(g->hflags.begin(), g->hflags.end(), [](uint8_t f) { return (f & kForcedBit) != 0; });
     const unsigned nb = (unsigned)((nw + 255) / 256);
     if (g->Q == 9) k_plain_bits<9><<<nb, 256, 0, g->stream>>>(g->flags, g->d.N, g->d.M, g->d.K, g->ncell, g->plain);
@@ -1409,6 +1448,15 @@ int lumagpu_run(lumagpu_grid *g, int nsteps) {
             if (int r = fused_pair(g, nullptr, nullptr)) return r;
             s += 2;
         }
+    }
+    if (nsteps - s >= 2 && multi_ok(g)) {
+        if (g->parity != 0) {
+            if (int r = apply_step(g, 0, nullptr, nullptr)) return r;
+            ++s;
+        }
+        int done = 0;
+        if (int r = run_multi(g, nsteps - s, &done)) return r;
+        s += done;
     }
     // Long runs of a hierarchy without host work per step replay a captured pair of steps: the
     // step alternates between the two AA kernels, so two steps are the period (the child's

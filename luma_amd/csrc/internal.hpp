@@ -21,7 +21,7 @@ struct lumagpu_grid {
     size_t ncell = 0, ps = 0, elem = 0;
     size_t melem = 8;                 // bytes per element of the macro, force and side arrays
     void *f = nullptr;
-    void *f2 = nullptr;               // second population array of the two-step (temporal-blocking) kernel
+    void *f2 = nullptr;               // second population array of the kernels that take several steps per launch
     int fuse_shape = -1, fuse_zc = 0; // its tile shape (FusedShape, -1: off) and z planes per block
     uint8_t *flags = nullptr;
     uint32_t *plain = nullptr;        // plain-site bitmap, rebuilt with every flag upload
@@ -76,6 +76,7 @@ struct lumagpu_grid {
     double pressure_drho = 0.0;       // GridUnits::pd2dlbm(L_PRESSURE_DELTA)
     double re = 0.0, re_ramp = 0.0;   // L_RE and L_REYNOLDS_RAMP in dimensionless time (0: off)
     int masked = 0;
+    int simple_types = 1;             // solid, fluid and velocity sites only
     int zslab = 0;                    // planes 0 and K-1 are halo planes of a z-sharded box
     int has_state = 0;
     int half = 0;                     // between lumagpu_stream_bc_macro and lumagpu_force_collide_swap

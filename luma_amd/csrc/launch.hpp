@@ -9,6 +9,7 @@
 #include "aa_kernels.hpp"
 #include "fused_kernels.hpp"
 #include "ibm_kernels.hpp"
+#include "multi2d_kernels.hpp"
 
 namespace lumagpu {
 
@@ -35,6 +36,10 @@ hipError_t launch_step_dual32(const LaunchSpec &ls, const StepArgs &a, hipStream
 hipError_t launch_fused2_f64(int shape, const StepArgs &a, void *dst, int zc, bool store, hipStream_t s);
 hipError_t launch_fused2_f32s(int shape, const StepArgs &a, void *dst, int zc, bool store, hipStream_t s);
 hipError_t launch_fused2_f16s(int shape, const StepArgs &a, void *dst, int zc, bool store, hipStream_t s);
+
+// H steps (even) of a small D2Q9 grid in one launch, a.f -> dst (multi2d_kernels.hpp)
+hipError_t launch_multi2d_f64(const StepArgs &a, void *dst, int H, int store, hipStream_t s);
+hipError_t launch_multi2d_f32s(const StepArgs &a, void *dst, int H, int store, hipStream_t s);
 
 hipError_t launch_aux_f64(int op, int Q, const StepArgs &a, const double *p0, const double *p1,
                           double *out, int parity, int masked, hipStream_t s);

@@ -11,6 +11,9 @@ hipError_t launch_fused2_f64(int shape, const StepArgs &a, void *dst, int zc, bo
     return launch_fused2_p<P64>(shape, a, dst, zc, store, s);
 }
 
+hipError_t launch_multi2d_f64(const StepArgs &a, void *dst, int H, int store, hipStream_t s) {
+    return launch_multi2d_p<P64>(a, dst, H, store, s);
+}
 hipError_t launch_aux_f64(int op, int Q, const StepArgs &a, const double *p0, const double *p1,
                           double *out, int parity, int masked, hipStream_t s) {
     return launch_aux_p<P64>(op, Q, a, p0, p1, out, parity, masked, s);
