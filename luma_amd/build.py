@@ -38,6 +38,7 @@ UNITS = [
     ("lbm_dual.hip", ["-ffp-contract=off"]),
     ("lbm_dual32.hip", ["-ffp-contract=off"]),
     ("api.hip", ["-ffp-contract=off"]),
+    ("host_copy.hip", []),
     ("ibm.hip", ["-ffp-contract=off", "-fno-builtin-sin", "-fno-builtin-cos"]),
     ("adjoint.hip", ["-ffp-contract=off"]),
     ("io.hip", ["-ffp-contract=off"]),

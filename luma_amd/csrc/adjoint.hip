@@ -487,7 +487,7 @@ int adj_run(lumagpu_grid *g, int nsteps, int every, const double dir[3], int bac
             k_adj_to_luma<19, T><<<nb, 256, 0, g->stream>>>(static_cast<const T *>(lam.p), nc, g->d.N, g->d.M,
                                                           g->d.K, static_cast<double *>(lout.p));
         HIP_TRY(hipGetLastError());
-        HIP_TRY(hipMemcpyAsync(lambda0, lout.p, (size_t)g->Q * nc * sizeof(double), hipMemcpyDeviceToHost, g->stream));
+        if (int r = copy_to_host(g, lambda0, lout.p, (size_t)g->Q * nc * sizeof(double))) return r;
         HIP_TRY(hipStreamSynchronize(g->stream));
     }
     std::vector<double> hx, he, hd;

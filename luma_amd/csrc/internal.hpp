@@ -53,6 +53,9 @@ struct lumagpu_grid {
     hipStream_t stream = nullptr;     // the stream this grid's work goes to: the root's, in a hierarchy
     hipStream_t own_stream = nullptr; // created with the grid
     int device = 0;                   // the GPU the grid was created on
+    int counted = 0;                  // host_copy_grid_added was called for it
+    void *pin = nullptr;              // pinned, device-visible staging of small downloads
+    size_t pin_bytes = 0;
     hipEvent_t ev_done = nullptr;     // recorded on this grid's stream after its sub-steps
     hipEvent_t ev_ready = nullptr;    // recorded before a child reads this grid's populations
     lumagpu_grid *parent = nullptr;   // GridObj::parentGrid (non-owning)
@@ -93,6 +96,12 @@ namespace lumagpu {
 
 // thread-local message behind lumagpu_last_error()
 int fail(int code, const std::string &msg);
+
+// device memory to the caller's, on g's stream (host_copy.hip); the pinned slots it uses live
+// while any grid does
+int copy_to_host(const lumagpu_grid *g, void *dst, const void *src, size_t bytes);
+void host_copy_grid_added();
+void host_copy_grid_gone();
 
 #define HIP_TRY(expr)                                                                        \
     do {                                                                                     \
