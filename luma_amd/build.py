@@ -39,6 +39,7 @@ UNITS = [
     ("lbm_dual32.hip", ["-ffp-contract=off"]),
     ("api.hip", ["-ffp-contract=off"]),
     ("host_copy.hip", []),
+    ("lu_device.hip", ["-ffp-contract=off"]),
     ("ibm.hip", ["-ffp-contract=off", "-fno-builtin-sin", "-fno-builtin-cos"]),
     ("adjoint.hip", ["-ffp-contract=off"]),
     ("io.hip", ["-ffp-contract=off"]),

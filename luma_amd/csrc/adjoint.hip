@@ -20,6 +20,7 @@
 #include "adjoint_kernels.hpp"
 #include "ibm_system.hpp"
 #include "launch.hpp"
+#include "lu_device.hpp"
 
 namespace lumagpu {
 namespace {
@@ -152,13 +153,17 @@ int epsilon_chain(const lumagpu_grid *g, const std::vector<const Marker *> &ms, 
 void ds_chain(const lumagpu_grid *g, const Body &b, const double *dsbar, double *xg) {
     const int n = (int)b.m.size(), D = g->D;
     const double dh = g->d.dh;
+    // positions side by side (a marker record spans 1.6 KB)
+    std::vector<double> p(3 * (size_t)n);
+    for (int m = 0; m < n; ++m)
+        for (int a = 0; a < 3; ++a) p[3 * (size_t)m + a] = b.m[m].pos[a];
     for (int m = 0; m < n; ++m) {
         double best = 10.0;
         int arg = -1;
         for (int q = 0; q < n; ++q) {
             if (q == m) continue;
             double acc = 0.0;
-            for (int a = 0; a < 3; ++a) acc += std::pow(b.m[m].pos[a] - b.m[q].pos[a], 2);
+            for (int a = 0; a < 3; ++a) acc += std::pow(p[3 * (size_t)m + a] - p[3 * (size_t)q + a], 2);
             const double dist = std::sqrt(acc) / dh;
             if (dist < best) {
                 best = dist;
@@ -174,21 +179,81 @@ void ds_chain(const lumagpu_grid *g, const Body &b, const double *dsbar, double 
     }
 }
 
+// epsilon_chain on the device for a system of kLuDeviceMin markers and more: assembly, LU and the sums
+// over near pairs are O(n^2) and O(n^3) work that one host thread took 94 ms for at 804 markers
+// (here 6.5 ms); the O(n^2) substitutions stay on the host.  first: the system's first marker
+// in the grid's marker arrays; sdd: the gradients of the delta weights.
+int epsilon_chain_device(const lumagpu_grid *g, const std::vector<const Marker *> &ms, int first, const double *sdd,
+                         const double *epsbar, double *dsbar, double *xg) {
+    const IbmSystem *s = g->ibm;
+    const size_t n = ms.size(), S = (size_t)s->S;
+    std::vector<double> h(5 * n + 3 * n * S, 0.0);
+    for (size_t i = 0; i < n; ++i) {
+        for (int a = 0; a < 3; ++a) h[3 * i + a] = ms[i]->pos[a];
+        h[3 * n + i] = ms[i]->dilation;
+        h[4 * n + i] = ms[i]->area;
+        for (int k = 0; k < ms[i]->ns; ++k)
+            for (int a = 0; a < 3; ++a) h[5 * n + 3 * (i * S + k) + a] = ms[i]->sxyz[k][a];
+    }
+    // markers; then mu, xg and dsbar; the matrix; pivots and info
+    DevBuf geo, vec, mat, piv;
+    if (int r = geo.alloc(h.size() * sizeof(double))) return r;
+    if (int r = vec.alloc(5 * n * sizeof(double))) return r;
+    if (int r = mat.alloc(n * n * sizeof(double))) return r;
+    if (int r = piv.alloc((n + 1) * sizeof(int))) return r;
+    double *gd = static_cast<double *>(geo.p), *vd = static_cast<double *>(vec.p), *a = static_cast<double *>(mat.p);
+    int *pd = static_cast<int *>(piv.p);
+    HIP_TRY(hipMemcpyAsync(gd, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice, g->stream));
+    const EpsSystem e{(int)n,       s->S,           g->D,          g->d.dh,
+                      gd,           gd + 3 * n,     gd + 4 * n,    gd + 5 * n,
+                      s->d_ns + first, s->d_sdelta + (size_t)first * S, sdd + (size_t)first * S * 3, s->d_eps + first,
+                      s->d_ds + first};
+    k_eps_matrix<<<dim3((unsigned)((n + 255) / 256), (unsigned)n), 256, 0, g->stream>>>(e, a);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(lu_factor_device((int)n, a, pd, pd + n, g->stream));
+    std::vector<double> lu(n * n);
+    std::vector<int> hp(n + 1);
+    HIP_TRY(hipMemcpyAsync(hp.data(), pd, hp.size() * sizeof(int), hipMemcpyDeviceToHost, g->stream));
+    if (int r = copy_to_host(g, lu.data(), a, lu.size() * sizeof(double))) return r;
+    HIP_TRY(hipStreamSynchronize(g->stream));
+    if (hp[n]) return fail(LUMAGPU_EPHYS, "singular IB epsilon system");
+    std::vector<double> v(5 * n);
+    std::copy(epsbar, epsbar + n, v.begin());
+    lu_substitute((int)n, lu.data(), hp.data(), v.data());
+    std::copy(xg, xg + 3 * n, v.begin() + n);
+    std::copy(dsbar, dsbar + n, v.begin() + 4 * n);
+    HIP_TRY(hipMemcpyAsync(vd, v.data(), v.size() * sizeof(double), hipMemcpyHostToDevice, g->stream));
+    k_eps_chain<<<(unsigned)((n + 3) / 4), 256, 0, g->stream>>>(e, vd, vd + n, vd + 4 * n);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipMemcpyAsync(v.data(), vd, v.size() * sizeof(double), hipMemcpyDeviceToHost, g->stream));
+    HIP_TRY(hipStreamSynchronize(g->stream));
+    std::copy(v.begin() + n, v.begin() + 4 * n, xg);
+    std::copy(v.begin() + 4 * n, v.end(), dsbar);
+    return 0;
+}
+
 // dJ/dx of every marker through epsilon and ds, per body or through the universal system
-int position_chains(const lumagpu_grid *g, const double *epsbar, const double *dsbar_dev, double *xg) {
+int position_chains(const lumagpu_grid *g, const double *sdd, const double *epsbar, const double *dsbar_dev,
+                    double *xg) {
     const IbmSystem *s = g->ibm;
     std::vector<double> dsbar(dsbar_dev, dsbar_dev + s->nm);
+    auto chain = [&](const std::vector<const Marker *> &ms, int first) {
+        const double *eb = epsbar + first;
+        double *db = dsbar.data() + first, *xb = xg + 3 * (size_t)first;
+        const int n = (int)ms.size();
+        if (n >= kLuDeviceMin && n <= kLuDeviceMax) return epsilon_chain_device(g, ms, first, sdd, eb, db, xb);
+        return epsilon_chain(g, ms, eb, db, xb);
+    };
     if (s->universal) {
         std::vector<const Marker *> ms;
         for (const auto &b : s->bodies)
             for (const auto &m : b.m) ms.push_back(&m);
-        if (int r = epsilon_chain(g, ms, epsbar, dsbar.data(), xg)) return r;
+        if (int r = chain(ms, 0)) return r;
     } else {
         for (const auto &b : s->bodies) {
             std::vector<const Marker *> ms;
             for (const auto &m : b.m) ms.push_back(&m);
-            if (int r = epsilon_chain(g, ms, epsbar + b.first, dsbar.data() + b.first, xg + 3 * (size_t)b.first))
-                return r;
+            if (int r = chain(ms, b.first)) return r;
         }
     }
     for (const auto &b : s->bodies) ds_chain(g, b, dsbar.data() + b.first, xg + 3 * (size_t)b.first);
@@ -503,7 +568,7 @@ int adj_run(lumagpu_grid *g, int nsteps, int every, const double dir[3], int bac
     if (res) *res = lumagpu_adj_result{hacc[0], hacc[1] + hacc[3] + hacc[5], hacc[2] + hacc[4] + hacc[6]};
     if (ib && dpos) {
         for (size_t i = 0; i < hx.size(); ++i) dpos[i] = hx[i];
-        if (int r = position_chains(g, he.data(), hd.data(), dpos)) return r;
+        if (int r = position_chains(g, static_cast<const double *>(sdd.p), he.data(), hd.data(), dpos)) return r;
     }
     return 0;
 }

@@ -491,6 +491,105 @@ __global__ void k_adj_ibm_site(IbmArgs ib, const double *mbar, const uint8_t *fl
             T(rb + L::c(v, 0) * jb[0] + L::c(v, 1) * jb[1] + L::c(v, 2) * jb[2]);
 }
 
+// ---- positions through epsilon and ds -------------------------------------------------------
+// One system's markers (a body's, or with the universal system every marker's), index 0 .. n-1.
+struct EpsSystem {
+    int n, S, D;
+    double dh;
+    const double *pos, *dil, *area;   // [3n], [n], [n]
+    const double *sxyz;               // [n][S][3] support positions
+    const int *ns;                    // [n]
+    const double *sdelta, *sddelta;   // [n][S] delta weights, [n][S][3] their gradients in the position
+    const double *eps, *ds;           // [n]
+};
+
+// delta_kernel (ObjectManager_ops_ibm.cpp:255-272) and its derivative, as the host evaluates them
+__device__ __forceinline__ double dev_delta(double radius, double dil) {
+    const double m = ::fabs(radius) / dil;
+    if (m > 1.5) return 0.0;
+    if (m > 0.5) return (5.0 - (3.0 * m) - ::sqrt(-3.0 * ((1.0 - m) * (1.0 - m)) + 1.0)) / 6.0;
+    return (1.0 + ::sqrt(1.0 - 3.0 * (m * m))) / 3.0;
+}
+__device__ __forceinline__ double dev_delta_deriv(double radius, double dil) {
+    const double m = ::fabs(radius) / dil, sgn = radius < 0.0 ? -1.0 : 1.0;
+    if (m > 1.5) return 0.0;
+    double d;
+    if (m > 0.5) {
+        const double q = 1.0 - m;
+        d = (-3.0 - 3.0 * q / ::sqrt(1.0 - 3.0 * q * q)) / 6.0;
+    } else {
+        d = -m / ::sqrt(1.0 - 3.0 * m * m);
+    }
+    return sgn * d / dil;
+}
+// far_apart: no support of one carries a delta weight of the other
+__device__ __forceinline__ bool eps_far(const EpsSystem &e, int I, int J) {
+    const double lim = (1.5 * e.dil[I] + 1.5 * e.dil[J] + 0.01) * e.dh;
+    for (int a = 0; a < e.D; ++a)
+        if (::fabs(e.pos[3 * J + a] - e.pos[3 * I + a]) > lim) return true;
+    return false;
+}
+__device__ __forceinline__ double eps_delta_at(const EpsSystem &e, int J, const double *s) {
+    double v = 1.0;
+    for (int a = 0; a < e.D; ++a) v *= dev_delta((e.pos[3 * J + a] - s[a]) / e.dh, e.dil[J]);
+    return v;
+}
+
+// A_IJ = ds_J sum_k delta_I(s_k) delta(x_J; s_k) area_I into a[J * n + I]; one thread per pair
+static __global__ __launch_bounds__(256) void k_eps_matrix(EpsSystem e, double *a) {
+    const int I = blockIdx.x * blockDim.x + threadIdx.x, J = blockIdx.y;
+    if (I >= e.n) return;
+    double acc = 0.0;
+    if (!eps_far(e, I, J))
+        for (int k = 0; k < e.ns[I]; ++k)
+            acc += e.sdelta[(size_t)I * e.S + k] * eps_delta_at(e, J, e.sxyz + ((size_t)I * e.S + k) * 3) * e.area[I];
+    a[(size_t)J * e.n + I] = acc * e.ds[J];
+}
+
+// With A^T mu = epsbar: dJ/dA_IJ = -mu_I eps_J, and A's entries depend on both markers' positions and
+// on ds_J.  One wave per marker m, its lanes the other markers: m as the row (its own weights'
+// gradients) and as the column (its delta at the other's supports, and ds_m).
+static __global__ __launch_bounds__(256) void k_eps_chain(EpsSystem e, const double *mu, double *xg, double *dsbar) {
+    const int m = blockIdx.x * 4 + (int)(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (m >= e.n) return;   // the whole wave
+    double x[3] = {0.0, 0.0, 0.0}, dsb = 0.0;
+    for (int q = lane; q < e.n; q += 64) {
+        if (eps_far(e, m, q)) continue;
+        const double row = -mu[m] * e.eps[q], col = -mu[q] * e.eps[m];
+        if (row != 0.0)
+            for (int k = 0; k < e.ns[m]; ++k) {
+                const size_t mk = (size_t)m * e.S + k;
+                const double t = row * e.ds[q] * eps_delta_at(e, q, e.sxyz + 3 * mk) * e.area[m];
+                for (int a = 0; a < e.D; ++a) x[a] += t * e.sddelta[3 * mk + a];
+            }
+        if (col != 0.0) {
+            double acc = 0.0;
+            for (int k = 0; k < e.ns[q]; ++k) {
+                const size_t qk = (size_t)q * e.S + k;
+                double ph[3] = {1.0, 1.0, 1.0}, dph[3] = {0.0, 0.0, 0.0};
+                for (int a = 0; a < e.D; ++a) {
+                    const double r = (e.pos[3 * m + a] - e.sxyz[3 * qk + a]) / e.dh;
+                    ph[a] = dev_delta(r, e.dil[m]);
+                    dph[a] = dev_delta_deriv(r, e.dil[m]) / e.dh;
+                }
+                const double w = e.sdelta[qk] * e.area[q];
+                acc += w * (ph[0] * ph[1] * ph[2]);
+                const double t = col * e.ds[m] * w;
+                x[0] += t * dph[0] * ph[1] * ph[2];
+                x[1] += t * ph[0] * dph[1] * ph[2];
+                x[2] += t * ph[0] * ph[1] * dph[2];
+            }
+            dsb += col * acc;
+        }
+    }
+    for (int a = 0; a < 3; ++a) x[a] = wave_sum_bcast(x[a]);
+    dsb = wave_sum_bcast(dsb);
+    if (lane == 0) {
+        for (int a = 0; a < 3; ++a) xg[3 * m + a] += x[a];
+        dsbar[m] += dsb;
+    }
+}
+
 // (1/T) dir . sum_m F_m eps_m ds_m vd_m added to acc[0]; one 64-lane wave, fixed order
 static __global__ void k_adj_objective(IbmArgs ib, double dx, double dy, double dz, double invT, double *acc) {
     const int lane = threadIdx.x;

@@ -17,6 +17,7 @@
 #include <memory>
 
 #include "ibm_system.hpp"
+#include "lu_device.hpp"
 
 namespace lumagpu {
 
@@ -409,6 +410,27 @@ int lu_solve_band(int n, int kl, int ku, std::vector<Dual> &a, std::vector<Dual>
 
 namespace {
 
+// lu_solve with the factorisation on the device (see lu_device.hip: the same factors)
+int lu_solve_device(const lumagpu_grid *g, int n, std::vector<double> &a, std::vector<double> &x) {
+    struct Buf {
+        void *p = nullptr;
+        ~Buf() { (void)hipFree(p); }
+    } da, dp;
+    std::vector<int> piv((size_t)n + 1);
+    if (hipMalloc(&da.p, a.size() * sizeof(double)) != hipSuccess || hipMalloc(&dp.p, piv.size() * sizeof(int)) != hipSuccess)
+        return fail(LUMAGPU_ENOMEM, "IB epsilon system allocation failed");
+    double *ad = static_cast<double *>(da.p);
+    int *pd = static_cast<int *>(dp.p);
+    HIP_TRY(hipMemcpyAsync(ad, a.data(), a.size() * sizeof(double), hipMemcpyHostToDevice, g->stream));
+    HIP_TRY(lu_factor_device(n, ad, pd, pd + n, g->stream));
+    HIP_TRY(hipMemcpyAsync(piv.data(), pd, piv.size() * sizeof(int), hipMemcpyDeviceToHost, g->stream));
+    if (int r = copy_to_host(g, a.data(), ad, a.size() * sizeof(double))) return r;
+    HIP_TRY(hipStreamSynchronize(g->stream));
+    if (piv[n]) return fail(LUMAGPU_EPHYS, "singular IB epsilon system");
+    lu_substitute(n, a.data(), piv.data(), x.data());
+    return 0;
+}
+
 // ibm_findEpsilon, :773-920: A_IJ = ds_J * sum_s delta_I(s) delta(x_J - x_s) A_I, A eps = 1.
 // On a tangent-form grid also d eps from A d(eps) = -dA eps, with dA from the marker, delta
 // and ds tangents.
@@ -487,7 +509,11 @@ int find_epsilon(const lumagpu_grid *g, Body &b) {
     // a chain of markers (a filament) gives a matrix banded in marker order: the banded solver,
     // which skips only the exact zeros outside the band, otherwise the dense one
     const bool band = 4 * (kl + ku) < n;
-    if (int r = band ? lu_solve_band_t(n, kl, ku, A, rhs, "singular IB epsilon system") : lu_solve(n, A, rhs)) return r;
+    int r = 0;
+    if (band) r = lu_solve_band_t(n, kl, ku, A, rhs, "singular IB epsilon system");
+    else if (n >= kLuDeviceMin && n <= kLuDeviceMax) r = lu_solve_device(g, n, A, rhs);
+    else r = lu_solve(n, A, rhs);
+    if (r) return r;
     for (int i = 0; i < n; ++i) b.m[i].eps = rhs[i];
     if (tan) {
         std::vector<double> drhs(n, 0.0);

@@ -1,0 +1,78 @@
+"""Epsilon systems solved on the device in the position gradient (bodies of 192 markers and more): the
+gradient against central differences of the forward, as in the other gradient tests, for body
+sizes around the device's lower limit, multiples of the factorisation's 16-column panels and its
+1024 rows per block; and a singular system's refusal."""
+import numpy as np
+import pytest
+
+from luma_amd import setups
+from luma_amd.grid import GpuGrid
+from oracle.oracle import OracleGrid, OracleIBM
+
+pytestmark = pytest.mark.gpu
+
+
+def _grid(pos, shape):
+    case = setups.uniform_inflow_3d(*shape, 0.03, 0.6)
+    g = GpuGrid.from_case(case, "fp64")
+    g.ibm_add_body(pos)
+    g.ibm_initialise()
+    return g
+
+
+# 191 is solved on the host; 192 = 12 panels, 193 leaves one column; 1040 takes two rows per thread
+@pytest.mark.parametrize("n", [191, 192, 193, 300, 1040])
+def test_position_gradient_against_differences(n):
+    radius = float(np.sqrt(n / (4.0 * np.pi)))      # one marker per unit area
+    shape = (int(2 * radius) + 16,) + (int(2 * radius) + 10,) * 2
+    centre = tuple(0.5 * s + 0.13 for s in shape)
+    pos = setups.sphere_markers(centre, radius, 1.0, n=n) + np.random.default_rng(n).normal(0.0, 0.03, (n, 3))
+    print(f"[eps] {n}", flush=True)
+    with _grid(pos, shape) as g:
+        out = g.adj_run(6, 3, initial=False)
+    grad = out["dJ_dpos"]
+    # a random direction over all markers.  Among n spacings some lie within the moves of a kink (the
+    # nearest marker changes, a support enters), which enters J by O(h) of those markers' share:
+    # h = 1e-5 keeps that at 1e-8 here, and the rounding of J over h at 1e-11 (h = 1e-4 is 5e-3
+    # off at 192 markers for a host-solved gradient too)
+    d = np.random.default_rng(n + 1).standard_normal((n, 3))
+    h, J = 1e-5, []
+    for s in (1.0, -1.0):
+        with _grid(pos + s * h * d, shape) as g:
+            J.append(g.adj_run(6, 3, backward=False)["J"])
+    fd = (J[0] - J[1]) / (2.0 * h)
+    assert abs((grad * d).sum() - fd) <= 1e-4 * abs(fd) + 1e-9
+
+
+# the systems of ibm_initialise go the same way: epsilon bit for bit the oracle's LU
+@pytest.mark.parametrize("n", [192, 207, 500, 1100])
+def test_epsilon_bitwise(n):
+    radius = float(np.sqrt(n / (4.0 * np.pi)))
+    shape = (int(2 * radius) + 10,) * 3
+    pos = setups.sphere_markers(tuple(0.5 * s + 0.13 for s in shape), radius, 1.0, n=n) + \
+        np.random.default_rng(n).normal(0.0, 0.03, (n, 3))
+    case = setups.uniform_inflow_3d(*shape, 0.03, 0.6)
+    print(f"[eps] bitwise {n}", flush=True)
+    o = OracleGrid(3, 19, case.N, case.M, case.K, omega=case.omega, regularised=False, forced=True, edges=case.edges)
+    o.set_labels(case.lattyp)
+    o.set_positions(case.xpos, case.ypos, case.zpos)
+    ib = OracleIBM(o, 1.0)
+    ib.add_body(pos)
+    ib.initialise()
+    with _grid(pos, shape) as g:
+        m = g.ibm_markers(0)
+    want = ib.markers(0)
+    assert np.array_equal(m["ds"], want["ds"]) and np.array_equal(m["eps"], want["eps"])
+
+
+def test_singular_system_is_refused():
+    # two markers at one place give two equal rows
+    pos = setups.sphere_markers((12.0, 11.0, 11.0), 4.0, 1.0, n=200)
+    pos[150] = pos[20]
+    case = setups.uniform_inflow_3d(26, 22, 22, 0.03, 0.6)
+    with GpuGrid.from_case(case, "fp64") as g:
+        g.ibm_add_body(pos)
+        with pytest.raises(Exception, match="singular|epsilon"):
+            g.ibm_initialise()
+            g.adj_run(2, 2, initial=False)
+            raise RuntimeError("epsilon system accepted")
