@@ -101,6 +101,7 @@ __device__ __forceinline__ uint32_t fast_div(uint32_t n, const FastDiv &f) {
 
 struct StepArgs {
     void *f;                      // population array
+    void *fo;                     // where listed and edge sites write: f, or the array a pair of steps goes to
     size_t ps;                    // population stride in elements
     int nx, ny, nz;               // x = LUMA i (N_lim), y = j (M_lim), z = k (K_lim)
     FastDiv dx, dy;               // division by nx, ny (kernels that take cells in linear order)
@@ -1222,7 +1223,7 @@ __device__ __forceinline__ void masked_site(const StepArgs &a, int x, int y, int
     if (ty == kSolid || ty == kRefined || (!a.regularised && ty == kVelocity)) return;
     // edge and corner velocity sites and pressure sites run in k_edge_sites after this kernel
     if (ty == kPressure || (ty == kVelocity && ((w >> kLinkNormal) & 7) == kNormalEdge)) return;
-    S *__restrict__ f = static_cast<S *>(a.f);
+    S *f = static_cast<S *>(a.fo);
     const size_t ps = a.ps;
 
     if ((w >> kLinkOther) & 1) gather_in<Q, P, ODD>(a, x, y, z, cell, nb, ty, fin);
@@ -1517,7 +1518,7 @@ __global__ __launch_bounds__(256) void k_edge_sites(StepArgs a, EdgeArgs e, int 
     const unsigned fl = a.flags[cell];
     const int pk = e.nrm[i];
     const int n[3] = {(pk & 3) - 1, ((pk >> 2) & 3) - 1, ((pk >> 4) & 3) - 1};
-    S *__restrict__ f = static_cast<S *>(a.f);
+    S *f = static_cast<S *>(a.fo);
     const size_t ps = a.ps;
     Nbr nb;
     nb.init(x, y, z, nx, ny, a.nz);

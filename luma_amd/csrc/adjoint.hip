@@ -34,7 +34,7 @@ struct DevBuf {
         if (p) (void)hipFree(p);
     }
     int alloc(size_t bytes) {
-        if (hipMalloc(&p, bytes) != hipSuccess) {
+        if (dev_malloc(&p, bytes) != hipSuccess) {
             p = nullptr;
             return fail(LUMAGPU_ENOMEM, "adjoint buffer allocation failed (" + std::to_string(bytes) + " bytes)");
         }

@@ -51,6 +51,54 @@ hipError_t launch_aux(const lumagpu_grid *g, int op, const double *p0, const dou
     }
 }
 
+// ---- the second population array ----------------------------------------------------------------
+// A run allocates it where its kernels take several steps per launch, if that leaves at least half of the
+// free memory free, and keeps it with the grid.  When an allocation of this library fails, the arrays of
+// grids that are not stepping at that moment are given back (g_f2_grids) and it is tried again, so
+// a program's grids fit as they would without them.
+std::mutex g_f2_grids_mu;
+std::vector<lumagpu_grid *> g_f2_grids;
+
+// the arrays of grids that no run holds, back to the device
+void f2_give_back() {
+    std::lock_guard<std::mutex> lock(g_f2_grids_mu);
+    for (size_t k = 0; k < g_f2_grids.size();) {
+        lumagpu_grid *o = g_f2_grids[k];
+        if (!o->f2_mu.try_lock()) {
+            ++k;
+            continue;
+        }
+        if (o->stream) (void)hipStreamSynchronize(o->stream);
+        (void)hipFree(o->f2);
+        o->f2 = nullptr;
+        o->f2_auto = o->pair_synced = 0;
+        o->f2_mu.unlock();
+        g_f2_grids.erase(g_f2_grids.begin() + k);
+    }
+}
+
+void f2_forget(lumagpu_grid *g) {
+    std::lock_guard<std::mutex> lock(g_f2_grids_mu);
+    g_f2_grids.erase(std::remove(g_f2_grids.begin(), g_f2_grids.end(), g), g_f2_grids.end());
+}
+
+// with g->f2_mu held: true when g->f2 is there
+bool f2_ensure(lumagpu_grid *g) {
+    if (g->f2) return true;
+    const size_t bytes = g->ps * g->Q * g->elem;
+    size_t avail = 0, total = 0;
+    if (hipMemGetInfo(&avail, &total) != hipSuccess || bytes > avail / 2 || hipMalloc(&g->f2, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        g->f2 = nullptr;
+        return false;
+    }
+    g->f2_auto = 1;
+    g->pair_synced = 0;
+    std::lock_guard<std::mutex> lock(g_f2_grids_mu);
+    g_f2_grids.push_back(g);
+    return true;
+}
+
 int ensure_stage(lumagpu_grid *g, size_t bytes) {
     if (g->stage_bytes >= bytes) return 0;
     if (g->stage) {
@@ -59,7 +107,7 @@ int ensure_stage(lumagpu_grid *g, size_t bytes) {
         g->stage = nullptr;
         g->stage_bytes = 0;
     }
-    if (hipMalloc(&g->stage, bytes) != hipSuccess) return fail(LUMAGPU_ENOMEM, "staging allocation failed");
+    if (dev_malloc((void **)&g->stage, bytes) != hipSuccess) return fail(LUMAGPU_ENOMEM, "staging allocation failed");
     g->stage_bytes = bytes;
     return 0;
 }
@@ -121,6 +169,16 @@ hipError_t launch_zslab(const lumagpu_grid *g, const StepArgs &a, int phase) {
 }  // namespace
 
 namespace lumagpu {
+hipError_t dev_malloc(void **p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e != hipErrorOutOfMemory) return e;
+    (void)hipGetLastError();
+    f2_give_back();
+    e = hipMalloc(p, bytes);
+    if (e != hipSuccess) *p = nullptr;
+    return e;
+}
+
 hipError_t launch_edges(const lumagpu_grid *g, const StepArgs &a, int phase) {
     EdgeArgs e{};
     e.n = g->nedge;
@@ -258,6 +316,16 @@ int begin_step(lumagpu_grid *g) {
     return 0;
 }
 
+// after a step's kernels: the next step's outlet sources are in the other buffer if they wrote them
+void outlet_written(lumagpu_grid *g, const StepArgs &a) {
+    if (a.xr_next) {
+        g->xr_sel ^= 1;
+        g->xr_ready = 1;
+    } else {
+        g->xr_ready = 0;
+    }
+}
+
 // The second half: stream, BC, macro (with the IB force), Guo forcing and BGK collision in one
 // pass, the edge/corner and pressure sites around it, then the swap (AA parity) and ++t.
 int end_step(lumagpu_grid *g, int subcycle, hipEvent_t e0, hipEvent_t e1) {
@@ -280,12 +348,7 @@ int end_step(lumagpu_grid *g, int subcycle, hipEvent_t e0, hipEvent_t e1) {
     hipError_t e = launch_step(g, ls, a);
     if (e != hipSuccess) return fail(LUMAGPU_EHIP, std::string("step launch: ") + hipGetErrorString(e));
     if (e1) HIP_TRY(hipEventRecord(e1, g->stream));
-    if (a.xr_next) {
-        g->xr_sel ^= 1;
-        g->xr_ready = 1;
-    } else {
-        g->xr_ready = 0;
-    }
+    outlet_written(g, a);
     if (halo) {
         e = launch_zslab(g, a, 1);
         if (e != hipSuccess) return fail(LUMAGPU_EHIP, std::string("halo launch: ") + hipGetErrorString(e));
@@ -387,7 +450,7 @@ int run_fused_graph(lumagpu_grid *g, int reps) {
 // changes from step to step, and site types whose sources the window holds.  2^18 cells: above,
 // a step fills the chip by itself, and the window's repeated cells cost more than launches.
 bool multi_ok(const lumagpu_grid *g) {
-    return g->Q == 9 && (g->d.precision == LUMAGPU_FP64 || g->d.precision == LUMAGPU_FP32S) && !g->parent &&
+    return !g->fuse_off && g->Q == 9 && (g->d.precision == LUMAGPU_FP64 || g->d.precision == LUMAGPU_FP32S) && !g->parent &&
            g->kids.empty() && ibm_marker_count(g) == 0 && !g->gravity_on && !(g->ramp_time > 0.0) &&
            !(g->re_ramp > 0.0) && g->nedge == 0 && g->simple_types && g->ncell <= (size_t(1) << 18) && g->has_state;
 }
@@ -395,14 +458,7 @@ bool multi_ok(const lumagpu_grid *g) {
 // up to n steps from the post-local layout, as many as whole launches take; *done: steps run
 int run_multi(lumagpu_grid *g, int n, int *done) {
     *done = 0;
-    if (!g->f2) {
-        if (hipMalloc(&g->f2, g->ps * g->Q * g->elem) != hipSuccess) {
-            // one step per launch needs no second array
-            (void)hipGetLastError();
-            g->f2 = nullptr;
-            return 0;
-        }
-    }
+    if (!f2_ensure(g)) return 0;   // one step per launch needs no second array
     // begin_step's state for a grid without bodies
     g->all_forced = g->sweep1_zero = 0;
     while (n - *done >= 2) {
@@ -414,6 +470,124 @@ int run_multi(lumagpu_grid *g, int n, int *done) {
         std::swap(g->f, g->f2);
         g->t += H;
         *done += H;
+    }
+    return 0;
+}
+
+// Two steps per launch on large D3Q19 grids in FP32-shifted storage (fused_kernels.hpp): one level, a
+// step that is the same kernels every time (no gravity reset, no Reynolds ramp), site types of the
+// list kernels, bodies rigid and settled (their supports flagged), outlet sources written by the
+// step.  us per step, single -> pairs: periodic boxes 32^3 10.7 -> 3.4, 64^3 9.4 -> 6.5, 128^3 53 -> 37,
+// 160^3 108 -> 77; walls with a set force 48^3 11.3 -> 13.1, 64^3 14.2 -> 14.9, 65^3 22.5 -> 20.2,
+// 96^3 42 -> 29, 160^3 129 -> 106: labelled grids, with three launches a pair, from 2^18 cells.
+constexpr size_t kPairMin = size_t(1) << 15, kPairMinLabelled = (size_t(1) << 18) + 1;
+bool pair_ok(const lumagpu_grid *g) {
+    if (g->fuse_off || g->Q != 19 || g->d.precision != LUMAGPU_FP32S || g->parent || !g->kids.empty() || g->zslab ||
+        g->gravity_on || g->re_ramp > 0.0 || !g->has_state || g->ncell < (g->masked ? kPairMinLabelled : kPairMin) ||
+        g->ps * g->elem >= (size_t(1) << 32))
+        return false;
+    if (g->has_outlet && !g->xr_fold) return false;
+    if (g->masked && !g->pair_types) return false;
+    return !ibm_has_flexible(g) && !(g->host_forced && ibm_marker_count(g) > 0);
+}
+
+// the deep cells and the lists around them, from the flags on the device
+int pair_sets(lumagpu_grid *g) {
+    if (!g->masked || g->pair_version == g->flags_version) return 0;
+    const size_t nw = (g->ncell + 31) / 32 + 1;   // a whole pair of words at the end
+    struct Buf {
+        uint32_t *p = nullptr;
+        ~Buf() { (void)hipFree(p); }
+    } rest, near;
+    if ((!g->pair_deep && hipMalloc(&g->pair_deep, nw * 4) != hipSuccess) || hipMalloc(&rest.p, nw * 4) != hipSuccess ||
+        hipMalloc(&near.p, nw * 4) != hipSuccess)
+        return fail(LUMAGPU_ENOMEM, "site set allocation failed");
+    const StepArgs a = make_args(g);
+    const unsigned nb = (unsigned)((g->ncell + 255) / 256);
+    k_deep_bits<19><<<nb, 256, 0, g->stream>>>(a, ibm_marker_count(g) > 0, g->pair_deep, rest.p);
+    k_near_bits<19><<<nb, 256, 0, g->stream>>>(a, g->pair_deep, rest.p, near.p);
+    HIP_TRY(hipGetLastError());
+    const size_t words = (g->ncell + 31) / 32;
+    std::vector<uint32_t> hr(words), hn(words);
+    HIP_TRY(hipMemcpyAsync(hr.data(), rest.p, words * 4, hipMemcpyDeviceToHost, g->stream));
+    HIP_TRY(hipMemcpyAsync(hn.data(), near.p, words * 4, hipMemcpyDeviceToHost, g->stream));
+    HIP_TRY(hipStreamSynchronize(g->stream));
+    std::vector<int> cells;
+    auto take = [&](const std::vector<uint32_t> &m) {
+        const size_t before = cells.size();
+        for (size_t w = 0; w < words; ++w)
+            for (uint32_t b = m[w]; b; b &= b - 1) cells.push_back((int)(32 * w + __builtin_ctz(b)));
+        return (int)(cells.size() - before);
+    };
+    g->n_near = take(hn);
+    g->n_rest = take(hr);
+    (void)hipFree(g->pair_cells);
+    (void)hipFree(g->pair_links);
+    g->pair_cells = nullptr;
+    g->pair_links = nullptr;
+    if (!cells.empty()) {
+        if (hipMalloc(&g->pair_cells, cells.size() * sizeof(int)) != hipSuccess ||
+            hipMalloc(&g->pair_links, cells.size() * sizeof(uint64_t)) != hipSuccess)
+            return fail(LUMAGPU_ENOMEM, "site list allocation failed");
+        HIP_TRY(hipMemcpyAsync(g->pair_cells, cells.data(), cells.size() * sizeof(int), hipMemcpyHostToDevice, g->stream));
+        k_links<19><<<(unsigned)((cells.size() + 255) / 256), 256, 0, g->stream>>>(
+            g->flags, g->d.N, g->d.M, g->d.K, g->d.regularised, g->pair_cells, cells.size(), g->pair_links);
+        HIP_TRY(hipGetLastError());
+        HIP_TRY(hipStreamSynchronize(g->stream));
+    }
+    g->pair_version = g->flags_version;
+    return 0;
+}
+
+// One half of a pair for the listed sites: what apply_step does around its step kernel, the even half from
+// f into f2 and before the deep cells, the odd half in place after them.
+int pair_half(lumagpu_grid *g, bool odd, PairPlan plan) {
+    if (int r = begin_step(g)) return r;
+    if (g->ibm)
+        if (int r = ibm_apply(g, true)) return r;
+    StepArgs a = make_args(g);
+    if (g->ib_fold) ibm_fold_args(g, a);
+    g->ib_fold = 0;
+    if (!odd) a.fo = g->f2;
+    const bool store = g->store_macro != 0;
+    auto check = [](hipError_t e) {
+        return e == hipSuccess ? 0 : fail(LUMAGPU_EHIP, std::string("two-step launch: ") + hipGetErrorString(e));
+    };
+    if (g->nedge)
+        if (int r = check(launch_edges(g, a, 0))) return r;
+    if (g->masked) {
+        const int *cells = odd ? g->pair_cells + g->n_near : g->pair_cells;
+        const uint64_t *links = odd ? g->pair_links + g->n_near : g->pair_links;
+        if (int r = check(launch_list_f32s(a, odd, odd && store, cells, links, odd ? g->n_rest : g->n_near, g->stream)))
+            return r;
+    }
+    if (g->nedge)
+        if (int r = check(launch_edges(g, a, 1))) return r;
+    outlet_written(g, a);
+    if (!odd) {
+        if (int r = check(launch_pair_f32s(a, g->f2, plan, g->masked ? g->pair_deep : nullptr, g->host_forced != 0, store,
+                                           g->stream)))
+            return r;
+        std::swap(g->f, g->f2);
+    }
+    g->parity ^= 1;
+    g->t += 1;
+    return 0;
+}
+
+// up to n steps from the post-neighbour layout, two at a time; *done: steps run
+int run_pairs(lumagpu_grid *g, int n, int *done) {
+    *done = 0;
+    if (!f2_ensure(g)) return 0;
+    if (int r = pair_sets(g)) return r;
+    if (g->masked && !g->pair_synced)
+        HIP_TRY(hipMemcpyAsync(g->f2, g->f, g->ps * g->Q * g->elem, hipMemcpyDeviceToDevice, g->stream));
+    g->pair_synced = 1;
+    const PairPlan plan = plan_pair(g->d.N, g->d.M, g->d.K);
+    while (n - *done >= 2) {
+        for (bool odd : {false, true})
+            if (int r = pair_half(g, odd, plan)) return r;
+        *done += 2;
     }
     return 0;
 }
@@ -751,6 +925,8 @@ static int build_links(lumagpu_grid *g) {
 }
 
 int upload_flags(lumagpu_grid *g) {
+    ++g->flags_version;
+    g->pair_synced = 0;
     if (g->hflags.size() != g->ncell) return fail(LUMAGPU_ESTATE, "host flag array does not cover the grid");
     if (!g->flags && hipMalloc(&g->flags, g->ncell) != hipSuccess)
         return fail(LUMAGPU_ENOMEM, "flag array allocation failed");
@@ -761,6 +937,10 @@ int upload_flags(lumagpu_grid *g) {
     g->simple_types = std::all_of(g->hflags.begin(), g->hflags.end(), [](uint8_t f) {
         const int t = f & kTypeMask;
         return t == kSolid || t == kFluid || t == kVelocity;
+    });
+    g->pair_types = std::all_of(g->hflags.begin(), g->hflags.end(), [](uint8_t f) {
+        const int t = f & kTypeMask;
+        return t == kSolid || t == kFluid || t == kVelocity || t == kPressure || t == kExtrapRight;
     });
     g->host_forced = std::any_of(g->hflags.begin(), g->hflags.end(), [](uint8_t f) { return (f & kForcedBit) != 0; });
     const unsigned nb = (unsigned)((nw + 255) / 256);
@@ -822,10 +1002,10 @@ int lumagpu_grid_create(const lumagpu_grid_desc *desc, lumagpu_grid **out) {
     if (hipEventCreateWithFlags(&g->ev_done, hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&g->ev_ready, hipEventDisableTiming) != hipSuccess)
         return cleanup(LUMAGPU_EHIP, "hipEventCreate failed");
-    if (hipMalloc(&g->f, g->ps * g->Q * g->elem) != hipSuccess)
+    if (dev_malloc(&g->f, g->ps * g->Q * g->elem) != hipSuccess)
         return cleanup(LUMAGPU_ENOMEM, "population array allocation failed");
-    if (hipMalloc(&g->rho, g->ncell * g->melem) != hipSuccess ||
-        hipMalloc(&g->u, g->ncell * g->D * g->melem) != hipSuccess)
+    if (dev_malloc((void **)&g->rho, g->ncell * g->melem) != hipSuccess ||
+        dev_malloc((void **)&g->u, g->ncell * g->D * g->melem) != hipSuccess)
         return cleanup(LUMAGPU_ENOMEM, "macro array allocation failed");
     if (hipMalloc(&g->uin, 3 * (size_t)d.M * sizeof(double)) != hipSuccess)
         return cleanup(LUMAGPU_ENOMEM, "inlet array allocation failed");
@@ -837,7 +1017,7 @@ int lumagpu_grid_create(const lumagpu_grid_desc *desc, lumagpu_grid **out) {
         hipMalloc(&g->moments_out, kMomentCount * sizeof(double)) != hipSuccess)
         return cleanup(LUMAGPU_ENOMEM, "reduction buffers allocation failed");
     if (d.forced) {
-        if (hipMalloc(&g->force, g->ncell * g->D * g->melem) != hipSuccess)
+        if (dev_malloc((void **)&g->force, g->ncell * g->D * g->melem) != hipSuccess)
             return cleanup(LUMAGPU_ENOMEM, "force array allocation failed");
         if (hipMemsetAsync(g->force, 0, g->ncell * g->D * g->melem, g->stream) != hipSuccess)
             return cleanup(LUMAGPU_EHIP, "force array clear failed");
@@ -854,7 +1034,11 @@ int lumagpu_grid_destroy(lumagpu_grid *g) {
     if (g->counted) host_copy_grid_gone();
     (void)hipHostFree(g->pin);
     (void)hipFree(g->f);
+    f2_forget(g);
     (void)hipFree(g->f2);
+    (void)hipFree(g->pair_deep);
+    (void)hipFree(g->pair_cells);
+    (void)hipFree(g->pair_links);
     (void)hipFree(g->flags);
     (void)hipFree(g->plain);
     (void)hipFree(g->stale);
@@ -1091,8 +1275,9 @@ int lumagpu_checkpoint_save(lumagpu_grid *g, lumagpu_checkpoint **out) {
     auto *ck = new lumagpu_checkpoint();
     ck->owner = g;
     ck->fbytes = g->ps * g->Q * g->elem;
-    if (hipMalloc(&ck->f, ck->fbytes) != hipSuccess || hipMalloc(&ck->rho, g->ncell * g->melem) != hipSuccess ||
-        hipMalloc(&ck->u, g->ncell * g->D * g->melem) != hipSuccess) {
+    if (dev_malloc(&ck->f, ck->fbytes) != hipSuccess ||
+        dev_malloc((void **)&ck->rho, g->ncell * g->melem) != hipSuccess ||
+        dev_malloc((void **)&ck->u, g->ncell * g->D * g->melem) != hipSuccess) {
         lumagpu_checkpoint_free(ck);
         return fail(LUMAGPU_ENOMEM, "checkpoint allocation failed");
     }
@@ -1118,6 +1303,7 @@ int lumagpu_checkpoint_restore(lumagpu_grid *g, const lumagpu_checkpoint *ck) {
     HIP_TRY(copy3(Copy3{{ck->f, ck->rho, ck->u}, {g->f, g->rho, g->u}, {ck->fbytes / 8, nm, nm * g->D}}, g->stream));
     g->xr_ready = 0;
     g->parity = ck->parity;
+    g->pair_synced = 0;
     g->t = ck->t;
     g->has_state = ck->has_state;
     return 0;
@@ -1215,6 +1401,7 @@ int lumagpu_init_equilibrium(lumagpu_grid *g, const double *rho, const double *u
     HIP_TRY(macro_from_luma(g, drho, du));
     g->parity = 0;
     g->has_state = 1;
+    g->pair_synced = 0;
     g->xr_ready = 0;
     if (int r = capture_stale(g)) return r;
     HIP_TRY(hipStreamSynchronize(g->stream));
@@ -1230,6 +1417,7 @@ int lumagpu_upload_f(lumagpu_grid *g, const double *f) {
     HIP_TRY(launch_aux(g, kAuxUpload, g->stage, nullptr, nullptr));
     g->parity = 0;
     g->has_state = 1;
+    g->pair_synced = 0;
     g->xr_ready = 0;
     if (int r = capture_stale(g)) return r;
     HIP_TRY(hipStreamSynchronize(g->stream));
@@ -1352,7 +1540,11 @@ int lumagpu_set_velocity_ramp(lumagpu_grid *g, double ramp_time) {
 
 int lumagpu_set_temporal_blocking(lumagpu_grid *g, int shape, int zchunk) {
     if (int r = check_grid(g)) return r;
+    std::lock_guard<std::mutex> lock(g->f2_mu);
     if (shape < 0) {
+        f2_forget(g);
+        g->f2_auto = 0;
+        g->fuse_off = 1;
         if (g->f2) {
             HIP_TRY(hipStreamSynchronize(g->stream));
             HIP_TRY(hipFree(g->f2));
@@ -1372,10 +1564,15 @@ int lumagpu_set_temporal_blocking(lumagpu_grid *g, int shape, int zchunk) {
     if (!fused_shape_fits(shape, g->d.N, g->d.M))
         return fail(LUMAGPU_EINVAL, "N and M must be whole numbers of the tile's x and y extents");
     if (zchunk < 1 || g->d.K < 3) return fail(LUMAGPU_EINVAL, "z chunk must be >= 1 and K >= 3");
-    if (!g->f2 && hipMalloc(&g->f2, g->ps * g->Q * g->elem) != hipSuccess) {
+    if (!g->f2 && dev_malloc(&g->f2, g->ps * g->Q * g->elem) != hipSuccess) {
         g->f2 = nullptr;
         return fail(LUMAGPU_ENOMEM, "second population array");
     }
+    // asked for: no longer one to give back
+    f2_forget(g);
+    g->f2_auto = 0;
+    g->pair_synced = 0;
+    g->fuse_off = 0;
     g->fuse_shape = shape;
     g->fuse_zc = zchunk;
     return 0;
@@ -1483,12 +1680,14 @@ int lumagpu_reset_forces(lumagpu_grid *g) {
         k_force_clear<Dual><<<nb, 256, 0, g->stream>>>(a, g->force, g->flags, g->D);
     HIP_TRY(hipGetLastError());
     for (auto &f : g->hflags) f &= (uint8_t)~kForcedBit;
+    ++g->flags_version;
     ibm_forget_flags(g);
     return 0;
 }
 
 int lumagpu_run(lumagpu_grid *g, int nsteps) {
     if (int r = check_grid(g)) return r;
+    std::lock_guard<std::mutex> lock(g->f2_mu);
     if (nsteps < 0) return fail(LUMAGPU_EINVAL, "negative step count");
     if (g->half) return fail(LUMAGPU_ESTATE, "a split step is open on this grid: finish it with lumagpu_force_collide_swap");
     int s = 0;
@@ -1509,6 +1708,15 @@ int lumagpu_run(lumagpu_grid *g, int nsteps) {
             if (int r = fused_pair(g, nullptr, nullptr)) return r;
             s += 2;
         }
+    }
+    if (nsteps - s >= 5 && pair_ok(g)) {
+        // single steps until the bodies' supports are flagged and the layout is the one pairs start from
+        for (int k = 0; k < 2 && (g->parity == 0 || !ibm_settled(g)); ++k, ++s)
+            if (int r = apply_step(g, 0, nullptr, nullptr)) return r;
+        int done = 0;
+        if (g->parity != 0 && ibm_settled(g) && pair_ok(g))
+            if (int r = run_pairs(g, nsteps - s, &done)) return r;
+        s += done;
     }
     if (nsteps - s >= 2 && multi_ok(g)) {
         if (g->parity != 0) {

@@ -42,8 +42,8 @@ struct FuseTile {
 // round-robin dispatch) take consecutive tiles: neighbouring tiles, whose ring rows overlap,
 // then run on the same XCD and share its L2.
 __device__ __forceinline__ int fused_tile_of(int b, int nblocks) {
-    if (nblocks % 8) return b;
-    return (b % 8) * (nblocks / 8) + b / 8;
+    const int q = nblocks / 8, r = nblocks % 8, x = b % 8;   // the first r XCDs take one more
+    return x * q + (x < r ? x : r) + b / 8;
 }
 
 // The 16 populations with a component in x or y, which the odd step takes from other columns
@@ -64,8 +64,15 @@ constexpr int lateral_index() {
 // (the value cell x + c_v of the tile pulls, stored at that cell's index): 16 * TX * TY values
 // instead of 19 * (TX + 2)(TY + 2), so two copies of a 32 x 16 tile take 64 KiB and two blocks
 // fit a CU; the odd step's LDS reads are then contiguous across the wave.
-template <class P, int TX, int TY, bool STORE, bool DB, bool O32 = false, bool PF = false, bool WIN = false>
-__global__ __launch_bounds__((TX + 2) * (TY + 2)) void k_aa_fused2(StepArgs a, void *dst_v, int zc) {
+// MASK: any extents (tiles at the far x and y sides are cut) and a bitmap of the cells the odd step
+// takes (deep, see k_deep_bits; null: all).  The even step runs on every cell of tile and ring; what
+// it makes of a cell that is not a plain one is read by no deep cell.
+// FORCED: a set force field (force_xyz at every cell, zero where the field is): the even step of
+// a cell loads it, the odd step takes it from registers.
+template <class P, int TX, int TY, bool STORE, bool DB, bool O32 = false, bool PF = false, bool WIN = false,
+          bool MASK = false, bool FORCED = false>
+__global__ __launch_bounds__((TX + 2) * (TY + 2)) void k_aa_fused2(StepArgs a, void *dst_v, int zc,
+                                                                   const uint32_t *deep) {
     using L = Lattice<19>;
     using S = typename P::S;
     using T = typename P::T;
@@ -78,7 +85,8 @@ __global__ __launch_bounds__((TX + 2) * (TY + 2)) void k_aa_fused2(StepArgs a, v
     __shared__ S shm[WIN ? 2 * 16 * TT : (DB ? 2 : 1) * Q * C];
 
     const int nx = a.nx, ny = a.ny, nz = a.nz;
-    const int ntx = nx / TX, nty = ny / TY, ntz = (nz + zc - 1) / zc;
+    const int ntx = MASK ? (nx + TX - 1) / TX : nx / TX, nty = MASK ? (ny + TY - 1) / TY : ny / TY;
+    const int ntz = (nz + zc - 1) / zc;
     const int tile = fused_tile_of(blockIdx.x, ntx * nty * ntz);
     const int tx = tile % ntx, ty = (tile / ntx) % nty, tz = tile / (ntx * nty);
     const int t = threadIdx.x;
@@ -101,9 +109,10 @@ __global__ __launch_bounds__((TX + 2) * (TY + 2)) void k_aa_fused2(StepArgs a, v
     }
     const int lc = ly * WX + lx;   // the cell's slot in the LDS copy
     int gx = tx * TX - 1 + lx, gy = ty * TY - 1 + ly;
-    gx = gx < 0 ? gx + nx : (gx >= nx ? gx - nx : gx);
-    gy = gy < 0 ? gy + ny : (gy >= ny ? gy - ny : gy);
-    const bool inner = t < TX * TY;
+    // a cut tile ends at the grid's last cell; the cell past it is ring, what lies beyond idles at 0
+    const bool inner = t < TX * TY && (!MASK || (gx < nx && gy < ny));
+    gx = gx < 0 ? gx + nx : (gx >= nx ? (MASK ? 0 : gx - nx) : gx);
+    gy = gy < 0 ? gy + ny : (gy >= ny ? (MASK ? 0 : gy - ny) : gy);
     const int z0 = tz * zc, z1 = min(z0 + zc, nz);
 
     const S *__restrict__ src = static_cast<const S *>(a.f);
@@ -126,14 +135,38 @@ __global__ __launch_bounds__((TX + 2) * (TY + 2)) void k_aa_fused2(StepArgs a, v
     };
     // even step of a column cell from its loaded populations: post-collision populations in
     // storage precision
-    auto even_from = [&](const S *raw, S *e) {
+    using FM = typename P::M;
+    struct Force {
+        FM v[3];
+    };
+    auto load_force = [&](int z) {
+        Force F{};
+        if constexpr (FORCED) {
+            const FM *fx = mv<FM>(a.force);
+            const size_t cell = col + plane * (size_t)z;
+            F.v[0] = fx[cell];
+            F.v[1] = fx[a.ncell + cell];
+            F.v[2] = fx[2 * a.ncell + cell];
+        }
+        return F;
+    };
+    auto deep_word = [&](int z) -> uint32_t {
+        if constexpr (MASK) {
+            if (deep) {
+                const size_t cell = col + plane * (size_t)z;
+                return deep[cell >> 5] >> (cell & 31);
+            }
+        }
+        return 1u;
+    };
+    auto even_from = [&](const S *raw, const Force &F, S *e) {
         T fin[Q];
         static_for<Q>([&](auto vc) {
             constexpr int v = decltype(vc)::value;
             fin[v] = static_cast<T>(raw[v]);
         });
         typename P::M rho, u[3];
-        const auto c = make_collider<Q, P>(fin, nullptr, a, rho, u);
+        const auto c = make_collider<Q, P>(fin, FORCED ? F.v : nullptr, a, rho, u);
         static_for<(Q - 1) / 2>([&](auto pc) {
             constexpr int v = 2 * decltype(pc)::value;
             T ov, oo;
@@ -143,24 +176,27 @@ __global__ __launch_bounds__((TX + 2) * (TY + 2)) void k_aa_fused2(StepArgs a, v
         });
         e[Q - 1] = static_cast<S>(c(Q - 1, fin[Q - 1]));
     };
-    auto even = [&](int z, S *e) {
+    auto even = [&](int z, S *e, Force &F) {
         S raw[Q];
         load(z, raw);
-        even_from(raw, e);
+        F = load_force(z);
+        even_from(raw, F, e);
     };
     auto wrapz = [&](int z) { return z < 0 ? z + nz : (z >= nz ? z - nz : z); };
 
     // own column's populations awaiting publication: c_z = 0 of plane p, c_z = +1 of planes p
     // and p - 1 (indexed by population; only the entries of the matching group are used)
     S rmid[Q], rup[Q], rup_prev[Q];
+    Force fcur, fnext{};       // the force at planes p and p + 1
+    uint32_t dcur = deep_word(z0);
     {
         S e[Q];
-        even(wrapz(z0 - 1), e);
+        even(wrapz(z0 - 1), e, fcur);
         static_for<Q>([&](auto vc) {
             constexpr int v = decltype(vc)::value;
             if constexpr (L::c(v, 2) == 1) rup_prev[v] = e[v];
         });
-        even(z0, e);
+        even(z0, e, fcur);
         static_for<Q>([&](auto vc) {
             constexpr int v = decltype(vc)::value;
             if constexpr (L::c(v, 2) == 1) rup[v] = e[v];
@@ -171,18 +207,22 @@ __global__ __launch_bounds__((TX + 2) * (TY + 2)) void k_aa_fused2(StepArgs a, v
     // one plane: the even step of plane p + 1 (its populations loaded into `cur`, or loaded
     // here), publication, the odd step of plane p.  With PF the loads of plane p + 2 go into
     // `nxt` first; the caller alternates two buffers, so no copy ties the loads to the loop end.
-    auto plane_step = [&](int p, const S *cur, S *nxt) {
+    // fe / fl: with PF, the force of plane p + 1 (loaded with `cur`) and where that of plane p + 2 goes
+    auto plane_step = [&](int p, const S *cur, S *nxt, const Force &fe, Force &fl) {
         S e[Q];
+        const uint32_t dnext = deep_word(wrapz(p + 1));
         if constexpr (PF) {
             // unconditionally (the last plane's load is spare): a branch here would make the
             // wait for `cur` also wait for these loads
             load(wrapz(p + 2), nxt);
+            fl = load_force(wrapz(p + 2));
             // keep the loads ahead of the plane's work (the scheduler would otherwise sink them
             // towards their use in the next plane)
             __builtin_amdgcn_sched_barrier(0);
-            even_from(cur, e);
+            fnext = fe;
+            even_from(cur, fe, e);
         } else {
-            even(wrapz(p + 1), e);
+            even(wrapz(p + 1), e, fnext);
         }
         S *sh = WIN ? shm + (p & 1) * (16 * TT) : (DB ? shm + (p & 1) * (Q * C) : shm);
         if constexpr (!DB) __syncthreads();   // the previous plane's odd step has read the LDS copy
@@ -217,7 +257,7 @@ __global__ __launch_bounds__((TX + 2) * (TY + 2)) void k_aa_fused2(StepArgs a, v
             }
         });
         __syncthreads();
-        if (inner) {
+        if (inner && (dcur & 1u)) {
             T fin[Q];
             static_for<Q>([&](auto vc) {
                 constexpr int v = decltype(vc)::value;
@@ -231,7 +271,7 @@ __global__ __launch_bounds__((TX + 2) * (TY + 2)) void k_aa_fused2(StepArgs a, v
                 }
             });
             typename P::M rho, u[3];
-            const auto c = make_collider<Q, P>(fin, nullptr, a, rho, u);
+            const auto c = make_collider<Q, P>(fin, FORCED ? fcur.v : nullptr, a, rho, u);
             if constexpr (STORE) store_macro<3>(a, col + plane * (size_t)p, rho, u);
             const int xm = gx == 0 ? nx - 1 : gx - 1, xp = gx == nx - 1 ? 0 : gx + 1;
             const int ym = gy == 0 ? ny - 1 : gy - 1, yp = gy == ny - 1 ? 0 : gy + 1;
@@ -257,21 +297,25 @@ __global__ __launch_bounds__((TX + 2) * (TY + 2)) void k_aa_fused2(StepArgs a, v
             });
             put(std::integral_constant<int, Q - 1>{}, c(Q - 1, fin[Q - 1]));
         }
+        if constexpr (FORCED) fcur = fnext;
+        dcur = dnext;
     };
     if constexpr (PF) {
         S bufA[Q], bufB[Q];
         load(wrapz(z0 + 1), bufA);
+        Force fA = load_force(wrapz(z0 + 1)), fB{};
         // pairs of planes with no branch inside the loop body (a conditional second plane merges
         // a path with bufB's loads still in flight into the loop header, whose wait would then
         // cover every outstanding load and store), then an odd last plane
         const int zp = z0 + ((z1 - z0) & ~1);
         for (int p = z0; p < zp; p += 2) {
-            plane_step(p, bufA, bufB);
-            plane_step(p + 1, bufB, bufA);
+            plane_step(p, bufA, bufB, fA, fB);
+            plane_step(p + 1, bufB, bufA, fB, fA);
         }
-        if (zp < z1) plane_step(zp, bufA, bufB);
+        if (zp < z1) plane_step(zp, bufA, bufB, fA, fB);
     } else {
-        for (int p = z0; p < z1; ++p) plane_step(p, nullptr, nullptr);
+        Force none{};
+        for (int p = z0; p < z1; ++p) plane_step(p, nullptr, nullptr, none, none);
     }
 }
 
@@ -304,12 +348,12 @@ hipError_t launch_fused2_t(const StepArgs &a, void *dst, int zc, bool store, hip
     // (measured at 256^3 FP32, 64x8: 302 us per step against 318 with 64-bit addresses)
     const bool o32 = a.ps * sizeof(typename P::S) < (size_t(1) << 32);
     if (o32) {
-        if (store) k_aa_fused2<P, TX, TY, true, DB, true, PF, WIN><<<g, b, 0, s>>>(a, dst, zc);
-        else k_aa_fused2<P, TX, TY, false, DB, true, PF, WIN><<<g, b, 0, s>>>(a, dst, zc);
+        if (store) k_aa_fused2<P, TX, TY, true, DB, true, PF, WIN><<<g, b, 0, s>>>(a, dst, zc, nullptr);
+        else k_aa_fused2<P, TX, TY, false, DB, true, PF, WIN><<<g, b, 0, s>>>(a, dst, zc, nullptr);
         return hipGetLastError();
     }
-    if (store) k_aa_fused2<P, TX, TY, true, DB, false, PF, WIN><<<g, b, 0, s>>>(a, dst, zc);
-    else k_aa_fused2<P, TX, TY, false, DB, false, PF, WIN><<<g, b, 0, s>>>(a, dst, zc);
+    if (store) k_aa_fused2<P, TX, TY, true, DB, false, PF, WIN><<<g, b, 0, s>>>(a, dst, zc, nullptr);
+    else k_aa_fused2<P, TX, TY, false, DB, false, PF, WIN><<<g, b, 0, s>>>(a, dst, zc, nullptr);
     return hipGetLastError();
 }
 
@@ -335,6 +379,125 @@ hipError_t launch_fused2_p(int shape, const StepArgs &a, void *dst, int zc, bool
         if (shape == 56 + kFuse32x16) return launch_fused2_t<P, 32, 16, true, true, true>(a, dst, zc, store, s);
     }
     return hipErrorInvalidValue;
+}
+
+// ---- two steps per launch on any D3Q19 grid --------------------------------------------------
+// Where the neighbourhood of a cell holds nothing but plain cells (fluid, no boundary source, no
+// body force of its own), its two steps need no flag: these deep cells take k_aa_fused2, and the rest,
+// a surface, takes two list launches around it, out of the populations `src` into `dst`:
+//   1. the even step of the list S1 = S + its neighbours, src -> dst (S: stepped, not deep)
+//   2. k_aa_fused2 on the deep cells, src -> dst
+//   3. the odd step of S, in place in dst
+// A slot belongs, in each of the two layouts, to one cell, which alone reads and writes it.  Step 1
+// leaves the even results of S1 in their cells' slots; step 2 writes the slots that deep cells own
+// in the odd layout, so it comes after 1 and spares every slot that step 3 reads, since those are
+// owned by S.  A slot of neither kind belongs to a solid, forced-equilibrium or other site that
+// never steps: it holds what it held (pair_sync copies those after a change of state or labels),
+// or what S pushes there.
+
+// deep: plain, and every neighbour plain; with bodies, none of them a support (forced)
+// rest: the cells k_aa_masked_list steps that are not deep
+template <int Q>
+__global__ __launch_bounds__(256) void k_deep_bits(StepArgs a, int bodies, uint32_t *deep, uint32_t *rest) {
+    using L = Lattice<Q>;
+    const size_t c = (size_t)blockIdx.x * 256 + threadIdx.x;
+    bool is_deep = false, is_rest = false;
+    if (c < a.ncell) {
+        auto plain = [&](size_t k) {
+            return ((a.plain[k >> 5] >> (k & 31)) & 1u) && !(bodies && (a.flags[k] & kForcedBit));
+        };
+        is_deep = plain(c);
+        int x, y, z;
+        cell_coords(a, (uint32_t)c, x, y, z);
+        Nbr nb;
+        nb.init(x, y, z, a.nx, a.ny, a.nz);
+        for (int v = 0; v < Q - 1 && is_deep; ++v)
+            is_deep = plain(nb.at(L::c(v, 0), L::c(v, 1), L::c(v, 2), a.nx, a.ny));
+        const unsigned fl = a.flags[c];
+        const int t = fl & kTypeMask;
+        const bool stepped = t == kFluid || t == kExtrapRight ||
+                             (t == kVelocity && a.regularised && ((fl >> kNormalShift) & 7) != kNormalEdge);
+        is_rest = stepped && !is_deep;
+    }
+    const uint64_t d = __ballot(is_deep), r = __ballot(is_rest);
+    if ((threadIdx.x & 31) == 0 && c < a.ncell) {
+        deep[c >> 5] = (uint32_t)(d >> (threadIdx.x & 32));
+        rest[c >> 5] = (uint32_t)(r >> (threadIdx.x & 32));
+    }
+}
+// near: rest and the stepped neighbours of rest (a neighbour of a listed or edge site that steps
+// and is not in rest is deep)
+template <int Q>
+__global__ __launch_bounds__(256) void k_near_bits(StepArgs a, const uint32_t *deep, const uint32_t *rest, uint32_t *near) {
+    using L = Lattice<Q>;
+    const size_t c = (size_t)blockIdx.x * 256 + threadIdx.x;
+    bool in = false;
+    if (c < a.ncell) {
+        auto bit = [](const uint32_t *m, size_t k) { return ((m[k >> 5] >> (k & 31)) & 1u) != 0; };
+        in = bit(rest, c);
+        if (!in && bit(deep, c)) {
+            int x, y, z;
+            cell_coords(a, (uint32_t)c, x, y, z);
+            Nbr nb;
+            nb.init(x, y, z, a.nx, a.ny, a.nz);
+            for (int v = 0; v < Q - 1 && !in; ++v) in = bit(rest, nb.at(L::c(v, 0), L::c(v, 1), L::c(v, 2), a.nx, a.ny));
+        }
+    }
+    const uint64_t m = __ballot(in);
+    if ((threadIdx.x & 31) == 0 && c < a.ncell) near[c >> 5] = (uint32_t)(m >> (threadIdx.x & 32));
+}
+
+// Tile and z chunk for a grid: one block fits a CU, so the cost is the rounds of 256 blocks times
+// the planes each takes, its two of start-up included (an even step without an odd one: counted as
+// one), times the tile's cells; 64 x 8 unless its cut tiles cost more than 32 x 16's.
+struct PairPlan {
+    int shape, zc;
+};
+inline PairPlan plan_pair(int nx, int ny, int nz) {
+    PairPlan best{kFuse64x8, nz};
+    double cost = 0.0;
+    for (int shape : {kFuse64x8, kFuse32x16}) {
+        int tx, ty;
+        fused_tile(shape, tx, ty);
+        const long tiles = (long)((nx + tx - 1) / tx) * ((ny + ty - 1) / ty);
+        for (int n = 1; n <= nz; ++n) {
+            const int zc = (nz + n - 1) / n;
+            const double rounds = (double)((tiles * ((nz + zc - 1) / zc) + 255) / 256);
+            // 32 x 16 moves its rows in halves of the 64 x 8 tile's lines: 1.08 per cell
+            const double c = rounds * (zc + 1) * (shape == kFuse64x8 ? 1.0 : 1.08);
+            if (cost == 0.0 || c < cost) {
+                cost = c;
+                best = PairPlan{shape, zc};
+            }
+        }
+    }
+    return best;
+}
+
+template <class P, int TX, int TY, bool MASK, bool FORCED>
+hipError_t launch_pair_t(const StepArgs &a, void *dst, int zc, const uint32_t *deep, bool store, hipStream_t s) {
+    const unsigned nb = (unsigned)(((a.nx + TX - 1) / TX) * ((a.ny + TY - 1) / TY) * ((a.nz + zc - 1) / zc));
+    const dim3 b(FuseTile<TX, TY>::C);
+    const bool o32 = a.ps * sizeof(typename P::S) < (size_t(1) << 32);
+    if (!o32) return hipErrorInvalidValue;   // pair_ok keeps such grids on single steps
+    if (store) k_aa_fused2<P, TX, TY, true, true, true, true, false, MASK, FORCED><<<nb, b, 0, s>>>(a, dst, zc, deep);
+    else k_aa_fused2<P, TX, TY, false, true, true, true, false, MASK, FORCED><<<nb, b, 0, s>>>(a, dst, zc, deep);
+    return hipGetLastError();
+}
+
+// the deep cells of any grid (deep null: every cell), with or without a set force field
+template <class P>
+hipError_t launch_pair_p(const StepArgs &a, void *dst, PairPlan pl, const uint32_t *deep, bool forced, bool store,
+                         hipStream_t s) {
+    const bool whole = !deep && !forced && fused_shape_fits(pl.shape, a.nx, a.ny);
+    if (pl.shape == kFuse64x8) {
+        if (whole) return launch_pair_t<P, 64, 8, false, false>(a, dst, pl.zc, deep, store, s);
+        if (forced) return launch_pair_t<P, 64, 8, true, true>(a, dst, pl.zc, deep, store, s);
+        return launch_pair_t<P, 64, 8, true, false>(a, dst, pl.zc, deep, store, s);
+    }
+    if (whole) return launch_pair_t<P, 32, 16, false, false>(a, dst, pl.zc, deep, store, s);
+    if (forced) return launch_pair_t<P, 32, 16, true, true>(a, dst, pl.zc, deep, store, s);
+    return launch_pair_t<P, 32, 16, true, false>(a, dst, pl.zc, deep, store, s);
 }
 
 }  // namespace lumagpu

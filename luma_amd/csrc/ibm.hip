@@ -725,6 +725,12 @@ int ibm_marker_count(const lumagpu_grid *g) {
     return n;
 }
 
+bool ibm_settled(const lumagpu_grid *g) {
+    const IbmSystem *s = g->ibm;
+    if (!s || ibm_marker_count(g) == 0) return true;
+    return s->initialised && !ibm_has_flexible(g) && !s->sites_dirty && s->site_map_ok;
+}
+
 bool ibm_has_flexible(const lumagpu_grid *g) {
     if (!g->ibm) return false;
     for (const auto &b : g->ibm->bodies)
@@ -777,6 +783,7 @@ int clear_gone(lumagpu_grid *g) {
             // ordered before it, which the stream gives
             HIP_TRY(hipStreamSynchronize(g->stream));
             for (int c : gone) g->hflags[c] &= (uint8_t)~kForcedBit;
+            ++g->flags_version;
         }
     }
     return 0;
@@ -826,6 +833,7 @@ int spread(lumagpu_grid *g) {
         for (int c : s->sites) g->hflags[c] |= kForcedBit;
         s->flagged = s->sites;
         s->sites_dirty = 0;
+        ++g->flags_version;
         if (!ibm_has_flexible(g))
             if (int r = build_site_map(g)) return r;
     }

@@ -5,6 +5,7 @@
 
 #include <cmath>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -22,6 +23,17 @@ struct lumagpu_grid {
     size_t melem = 8;                 // bytes per element of the macro, force and side arrays
     void *f = nullptr;
     void *f2 = nullptr;               // second population array of the kernels that take several steps per launch
+    int f2_auto = 0;                  // it was allocated by a run, not asked for: given back when memory is short
+    std::mutex f2_mu;                 // held by whoever uses or frees f2
+    int fuse_off = 0;                 // lumagpu_set_temporal_blocking turned several steps per launch off
+    // two steps per launch on a large 3D grid (fused_kernels.hpp): the deep cells, the cells around the
+    // others (S1) and the others (S) with their link words
+    uint32_t *pair_deep = nullptr;
+    int *pair_cells = nullptr;
+    uint64_t *pair_links = nullptr;
+    int n_near = 0, n_rest = 0;
+    uint64_t flags_version = 1, pair_version = 0;   // of the flag bytes; those the sets were built from
+    int pair_synced = 0;              // slots that no step writes are the same in f and f2
     int fuse_shape = -1, fuse_zc = 0; // its tile shape (FusedShape, -1: off) and z planes per block
     uint8_t *flags = nullptr;
     uint32_t *plain = nullptr;        // plain-site bitmap, rebuilt with every flag upload
@@ -80,6 +92,7 @@ struct lumagpu_grid {
     double re = 0.0, re_ramp = 0.0;   // L_RE and L_REYNOLDS_RAMP in dimensionless time (0: off)
     int masked = 0;
     int simple_types = 1;             // solid, fluid and velocity sites only
+    int pair_types = 1;               // those, pressure and ExtrapolateRight sites only
     int zslab = 0;                    // planes 0 and K-1 are halo planes of a z-sharded box
     int has_state = 0;
     int half = 0;                     // between lumagpu_stream_bc_macro and lumagpu_force_collide_swap
@@ -96,6 +109,9 @@ namespace lumagpu {
 
 // thread-local message behind lumagpu_last_error()
 int fail(int code, const std::string &msg);
+
+// hipMalloc that, short of memory, first takes back what runs allocated for themselves (api.hip)
+hipError_t dev_malloc(void **p, size_t bytes);
 
 // device memory to the caller's, on g's stream (host_copy.hip); the pinned slots it uses live
 // while any grid does
@@ -114,6 +130,7 @@ inline StepArgs make_args(const lumagpu_grid *g) {
     StepArgs a;
     std::memset(&a, 0, sizeof a);   // padding included: the bytes key the cached step graph
     a.f = g->f;
+    a.fo = g->f;
     a.ps = g->ps;
     a.nx = g->d.N;
     a.ny = g->d.M;
@@ -209,6 +226,8 @@ int upload_kids(lumagpu_grid *g);
 void ibm_forget_flags(lumagpu_grid *g);
 // the grid carries a flexible (FEM) body, whose step runs host work
 bool ibm_has_flexible(const lumagpu_grid *g);
+// no bodies, or initialised rigid ones whose supports are flagged
+bool ibm_settled(const lumagpu_grid *g);
 // markers of all IB bodies on the grid
 int ibm_marker_count(const lumagpu_grid *g);
 // one LBM_multi_opt of the grid (children first), as lumagpu_step; defined in api.hip

@@ -37,6 +37,13 @@ hipError_t launch_fused2_f64(int shape, const StepArgs &a, void *dst, int zc, bo
 hipError_t launch_fused2_f32s(int shape, const StepArgs &a, void *dst, int zc, bool store, hipStream_t s);
 hipError_t launch_fused2_f16s(int shape, const StepArgs &a, void *dst, int zc, bool store, hipStream_t s);
 
+// two steps of the deep cells of a D3Q19 grid (every cell with deep null), a.f -> dst, and one step of a
+// list of sites, a.f -> a.fo (fused_kernels.hpp)
+hipError_t launch_pair_f32s(const StepArgs &a, void *dst, PairPlan pl, const uint32_t *deep, bool forced, bool store,
+                            hipStream_t s);
+hipError_t launch_list_f32s(const StepArgs &a, bool odd, bool store, const int *cells, const uint64_t *links, int n,
+                            hipStream_t s);
+
 // H steps (even) of a small D2Q9 grid in one launch, a.f -> dst (multi2d_kernels.hpp)
 hipError_t launch_multi2d_f64(const StepArgs &a, void *dst, int H, int store, hipStream_t s);
 hipError_t launch_multi2d_f32s(const StepArgs &a, void *dst, int H, int store, hipStream_t s);
@@ -252,6 +259,19 @@ void with_bool(bool b, F &&f) {
 }
 
 template <int Q, class P>
+hipError_t launch_list_p(const StepArgs &a, bool odd, bool store, const int *cells, const uint64_t *links, int n,
+                         hipStream_t s) {
+    if (n <= 0) return hipSuccess;
+    const dim3 g((unsigned)((n + 63) / 64));
+    with_bool(odd, [&](auto o) {
+        with_bool(store, [&](auto st) {
+            k_aa_masked_list<Q, P, decltype(o)::value, decltype(st)::value><<<g, 64, 0, s>>>(a, cells, links, n);
+        });
+    });
+    return hipGetLastError();
+}
+
+template <int Q, class P>
 hipError_t launch_step_q(const LaunchSpec &ls, const StepArgs &a, hipStream_t s) {
     const dim3 b = cell_block(a.nx), g = cell_grid(a.nx, a.ny, a.nz - 2 * a.zoff);
     const CellOrder order = cell_order<P>(a);
@@ -260,7 +280,6 @@ hipError_t launch_step_q(const LaunchSpec &ls, const StepArgs &a, hipStream_t s)
     if (ls.masked && ls.nmlist >= 0) {
         // AA steps touch only a site's own set of slots, so the two disjoint site sets can run
         // one after the other
-        const dim3 lg((unsigned)((ls.nmlist + 63) / 64));
         with_bool(ls.odd, [&](auto odd) {
             with_bool(ls.store, [&](auto store) {
                 constexpr bool ODD = decltype(odd)::value, ST = decltype(store)::value;
@@ -271,9 +290,9 @@ hipError_t launch_step_q(const LaunchSpec &ls, const StepArgs &a, hipStream_t s)
                             <<<FL == kRows ? g : fg, FL == kRows ? b : fb, 0, s>>>(a);
                     });
                 });
-                if (ls.nmlist > 0) k_aa_masked_list<Q, P, ODD, ST><<<lg, 64, 0, s>>>(a, ls.mlist, ls.mlinks, ls.nmlist);
             });
         });
+        return launch_list_p<Q, P>(a, ls.odd, ls.store, ls.mlist, ls.mlinks, ls.nmlist, s);
     } else if (ls.masked) {
         with_bool(ls.odd, [&](auto odd) {
             with_bool(ls.store, [&](auto store) {

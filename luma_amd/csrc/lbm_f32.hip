@@ -12,6 +12,14 @@ hipError_t launch_step_f16s(const LaunchSpec &ls, const StepArgs &a, hipStream_t
 hipError_t launch_fused2_f32s(int shape, const StepArgs &a, void *dst, int zc, bool store, hipStream_t s) {
     return launch_fused2_p<P32S>(shape, a, dst, zc, store, s);
 }
+hipError_t launch_pair_f32s(const StepArgs &a, void *dst, PairPlan pl, const uint32_t *deep, bool forced, bool store,
+                            hipStream_t s) {
+    return launch_pair_p<P32S>(a, dst, pl, deep, forced, store, s);
+}
+hipError_t launch_list_f32s(const StepArgs &a, bool odd, bool store, const int *cells, const uint64_t *links, int n,
+                            hipStream_t s) {
+    return launch_list_p<19, P32S>(a, odd, store, cells, links, n, s);
+}
 hipError_t launch_fused2_f16s(int shape, const StepArgs &a, void *dst, int zc, bool store, hipStream_t s) {
     return launch_fused2_p<P16S>(shape, a, dst, zc, store, s);
 }
