@@ -101,7 +101,7 @@ __device__ __forceinline__ uint32_t fast_div(uint32_t n, const FastDiv &f) {
 
 struct StepArgs {
     void *f;                      // population array
-    void *fo;                     // where listed and edge sites write: f, or the array a pair of steps goes to
+    void *fo;                     // where labelled steps write: f, or the array a pair of steps or a tape takes
     size_t ps;                    // population stride in elements
     int nx, ny, nz;               // x = LUMA i (N_lim), y = j (M_lim), z = k (K_lim)
     FastDiv dx, dy;               // division by nx, ny (kernels that take cells in linear order)
@@ -1349,7 +1349,7 @@ __global__ __launch_bounds__(256) void k_aa_plain(StepArgs a) {
         if (!((a.plain[cell >> 5] >> (cell & 31)) & 1u)) return;
     }
     constexpr bool kNT = FLAT != kFlatOdd;
-    S *__restrict__ f = static_cast<S *>(a.f);
+    S *f = static_cast<S *>(a.fo);
     const size_t ps = a.ps;
     Nbr nb;
     nb.init(x, y, z, nx, ny, a.nz);

@@ -25,42 +25,84 @@
 namespace lumagpu {
 namespace {
 
+// A device buffer of a run, from the blocks the grid keeps between runs: allocating and freeing some
+// thirty arrays of the grid's size took 12 ms of a 100-step gradient on 1.2 M cells.  Everything on them
+// is ordered by the grid's stream.  Contents are what the last user left.
 struct DevBuf {
+    lumagpu_grid *g = nullptr;
     void *p = nullptr;
     DevBuf() = default;
     DevBuf(const DevBuf &) = delete;
     DevBuf &operator=(const DevBuf &) = delete;
     ~DevBuf() {
-        if (p) (void)hipFree(p);
+        if (!p) return;
+        for (auto &b : g->blocks)
+            if (b.p == p) b.used = 0;
     }
-    int alloc(size_t bytes) {
+    int alloc(lumagpu_grid *grid, size_t bytes) {
+        g = grid;
+        for (auto &b : g->blocks)
+            if (!b.used && b.bytes >= bytes && b.bytes - bytes <= bytes / 8 + 4096) {
+                b.used = 1;
+                p = b.p;
+                return 0;
+            }
         if (dev_malloc(&p, bytes) != hipSuccess) {
             p = nullptr;
             return fail(LUMAGPU_ENOMEM, "adjoint buffer allocation failed (" + std::to_string(bytes) + " bytes)");
         }
+        g->blocks.push_back({p, bytes, 1});
         return 0;
     }
 };
 
-template <class P>
-hipError_t launch_adj_collide(const lumagpu_grid *g, const StepArgs &a, const AdjArgs<typename P::T> &b) {
-    const dim3 bl = cell_block(a.nx), gr((a.nx + bl.x - 1) / bl.x, a.ny, a.nz);
-    const bool odd = g->parity == 0;
-    if (g->Q == 9) {
-        if (odd) k_adj_collide<9, P, true><<<gr, bl, 0, g->stream>>>(a, b);
-        else k_adj_collide<9, P, false><<<gr, bl, 0, g->stream>>>(a, b);
-    } else {
-        if (odd) k_adj_collide<19, P, true><<<gr, bl, 0, g->stream>>>(a, b);
-        else k_adj_collide<19, P, false><<<gr, bl, 0, g->stream>>>(a, b);
+// The grid keeps its blocks while they are at most a sixteenth of the device's memory.
+void trim_blocks(lumagpu_grid *g) {
+    size_t held = 0, avail = 0, total = 0;
+    for (const auto &b : g->blocks) held += b.bytes;
+    if (hipMemGetInfo(&avail, &total) == hipSuccess && held <= total / 16) {
+        if (held > 0) scratch_listed(g);
+        return;
     }
+    for (auto &b : g->blocks) (void)hipFree(b.p);
+    g->blocks.clear();
+}
+
+// nlist < 0: every site in one launch; else the plain sites and a list of the others (see AdjMode)
+constexpr int kAdjListBlock = 64;
+// cells from which the reversed step splits its sites: below, one launch more costs as much as the waves
+// that take both paths
+constexpr size_t kAdjSplitMin = size_t(1) << 17;
+template <int Q, class P>
+void launch_adj_collide_q(const lumagpu_grid *g, const StepArgs &a, const AdjArgs<typename P::T> &b, const int *cells,
+                          int nlist) {
+    const dim3 bl = cell_block(a.nx), gr((a.nx + bl.x - 1) / bl.x, a.ny, a.nz);
+    with_bool(g->parity == 0, [&](auto o) {
+        constexpr bool ODD = decltype(o)::value;
+        if (nlist < 0) {
+            k_adj_collide<Q, P, ODD, kAdjAll><<<gr, bl, 0, g->stream>>>(a, b, nullptr, 0);
+            return;
+        }
+        k_adj_collide<Q, P, ODD, kAdjPlain><<<gr, bl, 0, g->stream>>>(a, b, nullptr, 0);
+        if (nlist > 0)
+            k_adj_collide<Q, P, ODD, kAdjList>
+                <<<(nlist + kAdjListBlock - 1) / kAdjListBlock, kAdjListBlock, 0, g->stream>>>(a, b, cells, nlist);
+    });
+}
+template <class P>
+hipError_t launch_adj_collide(const lumagpu_grid *g, const StepArgs &a, const AdjArgs<typename P::T> &b,
+                              const int *cells, int nlist) {
+    if (g->Q == 9) launch_adj_collide_q<9, P>(g, a, b, cells, nlist);
+    else launch_adj_collide_q<19, P>(g, a, b, cells, nlist);
     return hipGetLastError();
 }
 
 template <class P>
-hipError_t launch_adj_stream(const lumagpu_grid *g, const StepArgs &a, const AdjArgs<typename P::T> &b) {
+hipError_t launch_adj_stream(const lumagpu_grid *g, const StepArgs &a, const AdjArgs<typename P::T> &b,
+                             typename P::T *out) {
     const dim3 bl = cell_block(a.nx), gr((a.nx + bl.x - 1) / bl.x, a.ny, a.nz);
-    if (g->Q == 9) k_adj_stream<9, P><<<gr, bl, 0, g->stream>>>(a, b);
-    else k_adj_stream<19, P><<<gr, bl, 0, g->stream>>>(a, b);
+    if (g->Q == 9) k_adj_stream<9, P><<<gr, bl, 0, g->stream>>>(a, b, out);
+    else k_adj_stream<19, P><<<gr, bl, 0, g->stream>>>(a, b, out);
     return hipGetLastError();
 }
 
@@ -183,7 +225,7 @@ void ds_chain(const lumagpu_grid *g, const Body &b, const double *dsbar, double 
 // over near pairs are O(n^2) and O(n^3) work that one host thread took 94 ms for at 804 markers
 // (here 6.5 ms); the O(n^2) substitutions stay on the host.  first: the system's first marker
 // in the grid's marker arrays; sdd: the gradients of the delta weights.
-int epsilon_chain_device(const lumagpu_grid *g, const std::vector<const Marker *> &ms, int first, const double *sdd,
+int epsilon_chain_device(lumagpu_grid *g, const std::vector<const Marker *> &ms, int first, const double *sdd,
                          const double *epsbar, double *dsbar, double *xg) {
     const IbmSystem *s = g->ibm;
     const size_t n = ms.size(), S = (size_t)s->S;
@@ -197,10 +239,10 @@ int epsilon_chain_device(const lumagpu_grid *g, const std::vector<const Marker *
     }
     // markers; then mu, xg and dsbar; the matrix; pivots and info
     DevBuf geo, vec, mat, piv;
-    if (int r = geo.alloc(h.size() * sizeof(double))) return r;
-    if (int r = vec.alloc(5 * n * sizeof(double))) return r;
-    if (int r = mat.alloc(n * n * sizeof(double))) return r;
-    if (int r = piv.alloc((n + 1) * sizeof(int))) return r;
+    if (int r = geo.alloc(g, h.size() * sizeof(double))) return r;
+    if (int r = vec.alloc(g, 5 * n * sizeof(double))) return r;
+    if (int r = mat.alloc(g, n * n * sizeof(double))) return r;
+    if (int r = piv.alloc(g, (n + 1) * sizeof(int))) return r;
     double *gd = static_cast<double *>(geo.p), *vd = static_cast<double *>(vec.p), *a = static_cast<double *>(mat.p);
     int *pd = static_cast<int *>(piv.p);
     HIP_TRY(hipMemcpyAsync(gd, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice, g->stream));
@@ -233,7 +275,7 @@ int epsilon_chain_device(const lumagpu_grid *g, const std::vector<const Marker *
 }
 
 // dJ/dx of every marker through epsilon and ds, per body or through the universal system
-int position_chains(const lumagpu_grid *g, const double *sdd, const double *epsbar, const double *dsbar_dev,
+int position_chains(lumagpu_grid *g, const double *sdd, const double *epsbar, const double *dsbar_dev,
                     double *xg) {
     const IbmSystem *s = g->ibm;
     std::vector<double> dsbar(dsbar_dev, dsbar_dev + s->nm);
@@ -260,10 +302,26 @@ int position_chains(const lumagpu_grid *g, const double *sdd, const double *epsb
     return 0;
 }
 
+// While a segment runs along the tape or is reversed, the grid's pointers stand on the tape; they go
+// back to the grid's own arrays on every way out.
+struct OnTape {
+    lumagpu_grid *g;
+    void *own;
+    int store;
+    ~OnTape() {
+        g->store_macro = store;
+        g->f = own;
+        g->f_to = nullptr;
+        g->xr_tape = nullptr;
+        g->xr_ready = 0;
+    }
+};
+
 template <class P>
 int adj_run(lumagpu_grid *g, int nsteps, int every, const double dir[3], int backward, lumagpu_adj_result *res,
             double *dpos, double *lambda0) {
     g->xr_ready = 0;   // the populations change outside the step kernels
+    g->pair_synced = 0;
     using T = typename P::T;
     IbmSystem *s = g->ibm;
     const bool ib = s && s->nm > 0;
@@ -271,32 +329,93 @@ int adj_run(lumagpu_grid *g, int nsteps, int every, const double dir[3], int bac
     const double invT = 1.0 / nsteps;
     const int nck = (nsteps + every - 1) / every;
     const int t_start = g->t;   // step t of the run runs at grid time t_start + t (velocity ramp)
+    // A labelled step can write its successor state elsewhere, so a segment runs from its checkpoint
+    // along the tape without a copy per step, the last segment already in the forward run; outlet
+    // sources are taped beside the states.  Every slot a step reads was written by the step before,
+    // except where an outlet row's source is a site that never steps (xr_fold): such grids, and unlabelled
+    // ones, step in place and copy.
+    const bool along = backward && g->masked && (!g->has_outlet || g->xr_fold);
+    const size_t xr_size = (size_t)g->Q * g->d.M * g->d.K;
 
-    std::vector<DevBuf> ck(nck);
-    std::vector<int> ckpar(nck);
+    OnTape guard{g, g->f, g->store_macro};
+    std::vector<DevBuf> ck(nck), tape(every);
+    std::vector<int> ckpar(nck), tpar(every);
     for (auto &b : ck)
-        if (int r = b.alloc(fbytes)) return r;
-    DevBuf fin, accJ;
-    if (int r = fin.alloc(fbytes)) return r;
+        if (int r = b.alloc(g, fbytes)) return r;
+    DevBuf fin, accJ, xrt;
+    if (!along && backward)
+        if (int r = fin.alloc(g, fbytes)) return r;
+    if (backward)
+        for (int i = along ? 1 : 0; i < std::min(every, nsteps); ++i)
+            if (int r = tape[i].alloc(g, fbytes)) return r;
+    if (along && g->has_outlet)
+        if (int r = xrt.alloc(g, (size_t)(std::min(every, nsteps) + 1) * xr_size * sizeof(double))) return r;
     // J; omega (fluid sites) and inlet scale (sources); omega and inlet scale (edge, corner and
     // pressure sites); omega and inlet scale (regularised faces)
-    if (int r = accJ.alloc(7 * sizeof(double))) return r;
+    if (int r = accJ.alloc(g, 7 * sizeof(double))) return r;
     HIP_TRY(hipMemsetAsync(accJ.p, 0, 7 * sizeof(double), g->stream));
+
+    auto objective = [&]() {
+        if (!ib) return 0;
+        k_adj_objective<<<1, 64, 0, g->stream>>>(ibm_args(g), dir[0], dir[1], dir[2], invT,
+                                                 static_cast<double *>(accJ.p));
+        HIP_TRY(hipGetLastError());
+        return 0;
+    };
+    // state i of segment seg on the tape
+    auto state = [&](int seg, int i) { return along && i == 0 ? ck[seg].p : tape[i].p; };
+    // along the tape: the steps of a segment from its checkpoint, n of them, the last one into `end`
+    auto run_along = [&](int seg, int n, void *end, bool forward) {
+        g->parity = ckpar[seg];
+        g->t = t_start + seg * every;
+        g->xr_ready = 0;
+        const int len = std::min(nsteps, (seg + 1) * every) - seg * every;
+        for (int i = 0; i < len; ++i) {
+            tpar[i] = g->parity;
+            g->f = state(seg, i);
+            if (g->has_outlet) g->xr_tape = static_cast<double *>(xrt.p) + i * xr_size;
+            if (i >= n) {
+                // the segment's last state: its outlet sources came with the step before
+                if (g->has_outlet && !g->xr_ready) HIP_TRY(outlet_prepass(g));
+                break;
+            }
+            g->f_to = i + 1 < len ? state(seg, i + 1) : end;
+            if (int r = step_grid(g, 0)) return r;
+            g->xr_ready = 1;
+            if (forward)
+                if (int r = objective()) return r;
+        }
+        g->f = guard.own;
+        g->f_to = nullptr;
+        g->xr_tape = nullptr;
+        g->xr_ready = 0;
+        // the end state's sites that never step, when its last step (even) pushed nothing to them
+        if (forward && !g->d.regularised && len >= 2 && tpar[len - 1] != 0) {
+            using S = typename P::S;
+            const S *from = static_cast<const S *>(state(seg, len - 1));
+            const unsigned nb = (unsigned)((g->ncell + 255) / 256);
+            const StepArgs a = make_args(g);
+            if (g->Q == 9) k_adj_carry<9, S><<<nb, 256, 0, g->stream>>>(a, from, static_cast<S *>(end));
+            else k_adj_carry<19, S><<<nb, 256, 0, g->stream>>>(a, from, static_cast<S *>(end));
+            HIP_TRY(hipGetLastError());
+        }
+        return 0;
+    };
 
     // forward with checkpoints
     for (int t = 0; t < nsteps; ++t) {
         if (t % every == 0) {
             HIP_TRY(hipMemcpyAsync(ck[t / every].p, g->f, fbytes, hipMemcpyDeviceToDevice, g->stream));
             ckpar[t / every] = g->parity;
+            if (along && t / every == nck - 1) {
+                if (int r = run_along(nck - 1, nsteps - t, g->f, true)) return r;
+                break;
+            }
         }
         if (int r = step_grid(g, 0)) return r;
-        if (ib) {
-            k_adj_objective<<<1, 64, 0, g->stream>>>(ibm_args(g), dir[0], dir[1], dir[2], invT,
-                                                     static_cast<double *>(accJ.p));
-            HIP_TRY(hipGetLastError());
-        }
+        if (int r = objective()) return r;
     }
-    HIP_TRY(hipMemcpyAsync(fin.p, g->f, fbytes, hipMemcpyDeviceToDevice, g->stream));
+    if (fin.p) HIP_TRY(hipMemcpyAsync(fin.p, g->f, fbytes, hipMemcpyDeviceToDevice, g->stream));
     const int fin_par = g->parity, fin_t = g->t;
     const double fin_omega = g->d.omega;
     double hacc[7] = {0, 0, 0, 0, 0, 0, 0};
@@ -309,31 +428,77 @@ int adj_run(lumagpu_grid *g, int nsteps, int every, const double dir[3], int bac
 
     // backward buffers
     const size_t nc = g->ncell;
+    // the macro arrays as the forward run left them: the reversed steps rewrite them at the supports
+    DevBuf mrho, mu;
+    const size_t mbytes = nc * g->melem;
+    if (ib) {
+        if (int r = mrho.alloc(g, mbytes)) return r;
+        if (int r = mu.alloc(g, mbytes * g->D)) return r;
+        HIP_TRY(hipMemcpyAsync(mrho.p, g->rho, mbytes, hipMemcpyDeviceToDevice, g->stream));
+        HIP_TRY(hipMemcpyAsync(mu.p, g->u, mbytes * g->D, hipMemcpyDeviceToDevice, g->stream));
+    }
+    guard.store = g->store_macro;   // the recomputed steps' fields are nobody's
+    g->store_macro = 0;
     // blocks of the collide and stream launches (cell_block rows)
     const int nblk = (int)((g->d.N + cell_block(g->d.N).x - 1) / cell_block(g->d.N).x) * g->d.M * g->d.K;
-    std::vector<DevBuf> tape(every);
-    std::vector<int> tpar(every);
-    for (auto &b : tape)
-        if (int r = b.alloc(fbytes)) return r;
-    DevBuf lam, gbar, fbar, part;
-    if (int r = lam.alloc((size_t)g->Q * nc * sizeof(T))) return r;
-    if (int r = gbar.alloc((size_t)g->Q * nc * sizeof(T))) return r;
-    if (int r = fbar.alloc(3 * nc * sizeof(double))) return r;
+    // the adjoint of the streamed populations, this step's and the later one's (zero after the last
+    // step), with the populations' plane stride: planes of a power of two times the element apart
+    // fall on the same memory channels
+    const size_t gbytes = (size_t)g->Q * g->ps * sizeof(T);
+    DevBuf gb[2], fbar, part;
+    if (int r = gb[0].alloc(g, gbytes)) return r;
+    if (int r = gb[1].alloc(g, gbytes)) return r;
+    if (int r = fbar.alloc(g, 3 * nc * sizeof(double))) return r;
+    // large grids: the fluid sites that are not plain, and those that feed an outlet
+    DevBuf list_cells;
+    int nlist = -1;
+    if (nc >= kAdjSplitMin && g->plain) {
+        const size_t words = (nc + 31) / 32;
+        std::vector<uint32_t> plain(words);
+        HIP_TRY(hipMemcpyAsync(plain.data(), g->plain, words * sizeof(uint32_t), hipMemcpyDeviceToHost, g->stream));
+        HIP_TRY(hipStreamSynchronize(g->stream));
+        std::vector<int> lc;
+        for (size_t w = 0; w < words; ++w)
+            for (uint32_t m = ~plain[w]; m; m &= m - 1) {
+                const size_t c = 32 * w + __builtin_ctz(m);
+                if (c < nc && (g->hflags[c] & kTypeMask) == kFluid) lc.push_back((int)c);
+            }
+        if (g->has_outlet)
+            for (size_t row = 0; row < nc; row += g->d.N) {
+                const size_t c = row + g->d.N - 3;
+                if ((plain[c >> 5] >> (c & 31)) & 1u) lc.push_back((int)c);
+            }
+        std::sort(lc.begin(), lc.end());
+        nlist = (int)lc.size();
+        if (nlist > 0) {
+            if (int r = list_cells.alloc(g, lc.size() * sizeof(int))) return r;
+            HIP_TRY(hipMemcpy(list_cells.p, lc.data(), lc.size() * sizeof(int), hipMemcpyHostToDevice));
+        }
+    }
+    const int nblk_all = nblk + (nlist > 0 ? (nlist + kAdjListBlock - 1) / kAdjListBlock : 0);
     // omega (collision), inlet scale (streaming from forced-equilibrium sources)
-    if (int r = part.alloc(2 * (size_t)nblk * sizeof(double))) return r;
-    HIP_TRY(hipMemsetAsync(lam.p, 0, (size_t)g->Q * nc * sizeof(T), g->stream));
+    if (int r = part.alloc(g, 2 * (size_t)nblk_all * sizeof(double))) return r;
+    HIP_TRY(hipMemsetAsync(gb[0].p, 0, gbytes, g->stream));
     HIP_TRY(hipMemsetAsync(fbar.p, 0, 3 * nc * sizeof(double), g->stream));
-    AdjArgs<T> ab{static_cast<T *>(lam.p), static_cast<T *>(gbar.p), static_cast<double *>(fbar.p),
-                  static_cast<double *>(part.p), nblk};
+    AdjArgs<T> ab{};
+    ab.gin = static_cast<const T *>(gb[0].p);
+    ab.gbar = static_cast<T *>(gb[1].p);
+    ab.ps = g->ps;
+    ab.fbar = static_cast<double *>(fbar.p);
+    ab.part = static_cast<double *>(part.p);
+    ab.nblk = nblk;
+    ab.nblk_all = nblk_all;
+    ab.outlet = g->has_outlet;
+    ab.ramp_feq = 1.0;
     DevBuf mbar, xbar, epsbar, dsbar, sdd;
     AdjIbm aj{};
     if (ib) {
         const size_t nm = (size_t)s->nm;
-        if (int r = mbar.alloc(4 * nm * sizeof(double))) return r;
-        if (int r = xbar.alloc(3 * nm * sizeof(double))) return r;
-        if (int r = epsbar.alloc(nm * sizeof(double))) return r;
-        if (int r = dsbar.alloc(nm * sizeof(double))) return r;
-        if (int r = sdd.alloc(nm * s->S * 3 * sizeof(double))) return r;
+        if (int r = mbar.alloc(g, 4 * nm * sizeof(double))) return r;
+        if (int r = xbar.alloc(g, 3 * nm * sizeof(double))) return r;
+        if (int r = epsbar.alloc(g, nm * sizeof(double))) return r;
+        if (int r = dsbar.alloc(g, nm * sizeof(double))) return r;
+        if (int r = sdd.alloc(g, nm * s->S * 3 * sizeof(double))) return r;
         HIP_TRY(hipMemsetAsync(xbar.p, 0, 3 * nm * sizeof(double), g->stream));
         HIP_TRY(hipMemsetAsync(epsbar.p, 0, nm * sizeof(double), g->stream));
         HIP_TRY(hipMemsetAsync(dsbar.p, 0, nm * sizeof(double), g->stream));
@@ -390,12 +555,12 @@ int adj_run(lumagpu_grid *g, int nsteps, int every, const double dir[3], int bac
         }
         ptr.push_back((int)ent.size());
         n_enb = (int)cells.size();
-        if (int r = dbar.alloc(ne * sizeof(double))) return r;
-        if (int r = tbar.alloc(3 * (size_t)ne * sizeof(double))) return r;
-        if (int r = epart.alloc(2 * (size_t)ne * sizeof(double))) return r;
-        if (int r = enb_cell.alloc(cells.size() * sizeof(int))) return r;
-        if (int r = enb_ptr.alloc(ptr.size() * sizeof(int))) return r;
-        if (int r = enb_ent.alloc(ent.size() * sizeof(int))) return r;
+        if (int r = dbar.alloc(g, ne * sizeof(double))) return r;
+        if (int r = tbar.alloc(g, 3 * (size_t)ne * sizeof(double))) return r;
+        if (int r = epart.alloc(g, 2 * (size_t)ne * sizeof(double))) return r;
+        if (int r = enb_cell.alloc(g, cells.size() * sizeof(int))) return r;
+        if (int r = enb_ptr.alloc(g, ptr.size() * sizeof(int))) return r;
+        if (int r = enb_ent.alloc(g, ent.size() * sizeof(int))) return r;
         HIP_TRY(hipMemcpy(enb_cell.p, cells.data(), cells.size() * sizeof(int), hipMemcpyHostToDevice));
         HIP_TRY(hipMemcpy(enb_ptr.p, ptr.data(), ptr.size() * sizeof(int), hipMemcpyHostToDevice));
         HIP_TRY(hipMemcpy(enb_ent.p, ent.data(), ent.size() * sizeof(int), hipMemcpyHostToDevice));
@@ -405,7 +570,7 @@ int adj_run(lumagpu_grid *g, int nsteps, int every, const double dir[3], int bac
     // the IB set-up made (no bitmap) gets one with no plain site
     DevBuf nobits;
     if (!g->plain) {
-        if (int r = nobits.alloc((nc + 31) / 32 * sizeof(uint32_t))) return r;
+        if (int r = nobits.alloc(g, (nc + 31) / 32 * sizeof(uint32_t))) return r;
         HIP_TRY(hipMemsetAsync(nobits.p, 0, (nc + 31) / 32 * sizeof(uint32_t), g->stream));
     }
 
@@ -420,31 +585,38 @@ int adj_run(lumagpu_grid *g, int nsteps, int every, const double dir[3], int bac
         }
         nface = (int)fc.size();
         if (nface > 0) {
-            if (int r = face_cells.alloc(fc.size() * sizeof(int))) return r;
-            if (int r = fpart.alloc(2 * fc.size() * sizeof(double))) return r;
+            if (int r = face_cells.alloc(g, fc.size() * sizeof(int))) return r;
+            if (int r = fpart.alloc(g, 2 * fc.size() * sizeof(double))) return r;
             HIP_TRY(hipMemcpy(face_cells.p, fc.data(), fc.size() * sizeof(int), hipMemcpyHostToDevice));
         }
     }
 
-    void *const f_own = g->f;
     int rc = 0;
+    StepArgs a_first;   // the arguments of the step reversed last
     for (int seg = nck - 1; seg >= 0 && !rc; --seg) {
         const int t0 = seg * every, t1 = std::min(nsteps, t0 + every);
-        HIP_TRY(hipMemcpyAsync(g->f, ck[seg].p, fbytes, hipMemcpyDeviceToDevice, g->stream));
-        g->parity = ckpar[seg];
-        g->t = t_start + t0;
-        g->xr_ready = 0;
-        for (int t = t0; t < t1 && !rc; ++t) {
-            HIP_TRY(hipMemcpyAsync(tape[t - t0].p, g->f, fbytes, hipMemcpyDeviceToDevice, g->stream));
-            tpar[t - t0] = g->parity;
-            if (t + 1 < t1) rc = step_grid(g, 0);
+        if (along) {
+            // the states of the last segment are on the tape from the forward run
+            if (seg < nck - 1) rc = run_along(seg, t1 - t0 - 1, nullptr, false);
+        } else {
+            HIP_TRY(hipMemcpyAsync(g->f, ck[seg].p, fbytes, hipMemcpyDeviceToDevice, g->stream));
+            g->parity = ckpar[seg];
+            g->t = t_start + t0;
+            g->xr_ready = 0;
+            for (int t = t0; t < t1 && !rc; ++t) {
+                HIP_TRY(hipMemcpyAsync(tape[t - t0].p, g->f, fbytes, hipMemcpyDeviceToDevice, g->stream));
+                tpar[t - t0] = g->parity;
+                if (t + 1 < t1) rc = step_grid(g, 0);
+            }
         }
         for (int t = t1 - 1; t >= t0 && !rc; --t) {
             // the step's input state stands in for the grid's populations while it is reversed
-            g->f = tape[t - t0].p;
+            g->f = state(seg, t - t0);
             g->t = t_start + t;
             g->parity = tpar[t - t0];
-            if (g->has_outlet) {
+            if (along && g->has_outlet) {
+                g->xr_tape = static_cast<double *>(xrt.p) + (t - t0) * xr_size;
+            } else if (g->has_outlet) {
                 hipError_t e = outlet_prepass(g);
                 if (e != hipSuccess) rc = fail(LUMAGPU_EHIP, std::string("adjoint outlet: ") + hipGetErrorString(e));
             }
@@ -459,9 +631,16 @@ int adj_run(lumagpu_grid *g, int nsteps, int every, const double dir[3], int bac
             StepArgs a = make_args(g);
             if (!a.plain) a.plain = static_cast<const uint32_t *>(nobits.p);
             if (!rc) {
+                AdjSums sums{};
+                int nsum = 0;
+                auto add_sum = [&](const double *part, int n, double *to) {
+                    sums.part[nsum] = part;
+                    sums.n[nsum] = n;
+                    sums.acc[nsum++] = to;
+                };
                 // the edge sites' extrapolation densities of this step
                 hipError_t e = g->nedge ? launch_edges(g, a, 0) : hipSuccess;
-                if (e == hipSuccess) e = launch_adj_collide<P>(g, a, ab);
+                if (e == hipSuccess) e = launch_adj_collide<P>(g, a, ab, static_cast<const int *>(list_cells.p), nlist);
                 if (e == hipSuccess && nface) {
                     const dim3 fb(64), fg((unsigned)((nface + 63) / 64), (unsigned)(g->Q + 2));
                     const int *fcp = static_cast<const int *>(face_cells.p);
@@ -475,10 +654,7 @@ int adj_run(lumagpu_grid *g, int nsteps, int every, const double dir[3], int bac
                         else k_adj_faces<19, P, false><<<fg, fb, 0, g->stream>>>(a, ab, fcp, nface, fp);
                     }
                     e = hipGetLastError();
-                    if (e == hipSuccess) {
-                        k_adj_sum_partials<<<1, 1024, 0, g->stream>>>(fp, nface, 2, w_om, acc + 5);
-                        e = hipGetLastError();
-                    }
+                    add_sum(fp, nface, acc + 5);
                 }
                 if (e == hipSuccess && g->nedge) {
                     const dim3 eb(64), eg((unsigned)((g->nedge + 63) / 64), (unsigned)(g->Q + 4));
@@ -492,21 +668,18 @@ int adj_run(lumagpu_grid *g, int nsteps, int every, const double dir[3], int bac
                         else k_adj_edges<9, P, false><<<eg, eb, 0, g->stream>>>(a, ea, ab, db, tb, ep);
                         e = hipGetLastError();
                         if (e == hipSuccess)
-                            k_adj_edge_nbrs<9, T><<<nbg, nbb, 0, g->stream>>>(n_enb, nc_p, np_p, ne_p, db, tb, g->erho, nc,
-                                                                             ab.gbar);
+                            k_adj_edge_nbrs<9, T><<<nbg, nbb, 0, g->stream>>>(n_enb, nc_p, np_p, ne_p, db, tb, g->erho,
+                                                                             ab.ps, ab.gbar);
                     } else {
                         if (g->parity == 0) k_adj_edges<19, P, true><<<eg, eb, 0, g->stream>>>(a, ea, ab, db, tb, ep);
                         else k_adj_edges<19, P, false><<<eg, eb, 0, g->stream>>>(a, ea, ab, db, tb, ep);
                         e = hipGetLastError();
                         if (e == hipSuccess)
                             k_adj_edge_nbrs<19, T><<<nbg, nbb, 0, g->stream>>>(n_enb, nc_p, np_p, ne_p, db, tb, g->erho,
-                                                                              nc, ab.gbar);
+                                                                              ab.ps, ab.gbar);
                     }
                     if (e == hipSuccess) e = hipGetLastError();
-                    if (e == hipSuccess) {
-                        k_adj_sum_partials<<<1, 1024, 0, g->stream>>>(ep, g->nedge, 2, w_om, acc + 3);
-                        e = hipGetLastError();
-                    }
+                    add_sum(ep, g->nedge, acc + 3);
                 }
                 if (e == hipSuccess && ib) {
                     IbmArgs ia = ibm_args(g);
@@ -515,25 +688,52 @@ int adj_run(lumagpu_grid *g, int nsteps, int every, const double dir[3], int bac
                     if (e == hipSuccess) {
                         if (g->Q == 9)
                             k_adj_ibm_site<9, T><<<(s->nsites + 127) / 128, 128, 0, g->stream>>>(
-                                ia, aj.mbar, g->flags, ab.gbar);
+                                ia, aj.mbar, g->flags, ab.ps, ab.gbar);
                         else
                             k_adj_ibm_site<19, T><<<(s->nsites + 127) / 128, 128, 0, g->stream>>>(
-                                ia, aj.mbar, g->flags, ab.gbar);
+                                ia, aj.mbar, g->flags, ab.ps, ab.gbar);
                         e = hipGetLastError();
                     }
                 }
-                if (e == hipSuccess) e = launch_adj_stream<P>(g, a, ab);
                 if (e == hipSuccess) {
-                    k_adj_sum_partials<<<1, 1024, 0, g->stream>>>(ab.part, nblk, 2, w_om, acc + 1);
+                    add_sum(ab.part, nblk_all, acc + 1);
+                    k_adj_sum_partials<<<nsum, 1024, 0, g->stream>>>(sums, w_om);
                     e = hipGetLastError();
                 }
                 if (e != hipSuccess) rc = fail(LUMAGPU_EHIP, std::string("adjoint launch: ") + hipGetErrorString(e));
             }
-            g->f = f_own;
+            // what this step streamed is the later step's adjoint for the one before it
+            T *next = const_cast<T *>(ab.gin);
+            ab.gin = ab.gbar;
+            ab.gbar = next;
+            ab.ramp_feq = a.ramp_feq;
+            ab.ramp_on = a.ramp_on;
+            a_first = a;
+            g->f = guard.own;
+            g->xr_tape = nullptr;
         }
     }
+    if (!rc) {
+        // the first step's streaming: the initial populations' adjoint (into the free array) and its
+        // share of the inlet scale, from the blocks over the grid alone
+        ab.nblk_all = nblk;
+        hipError_t e = launch_adj_stream<P>(g, a_first, ab, lambda0 ? ab.gbar : nullptr);
+        if (e == hipSuccess) {
+            AdjSums sums{};
+            sums.part[0] = ab.part;
+            sums.n[0] = nblk;
+            sums.acc[0] = acc + 1;
+            k_adj_sum_partials<<<1, 1024, 0, g->stream>>>(sums, 1.0);
+            e = hipGetLastError();
+        }
+        if (e != hipSuccess) rc = fail(LUMAGPU_EHIP, std::string("adjoint launch: ") + hipGetErrorString(e));
+    }
     // the grid returns to the end of the forward run
-    HIP_TRY(hipMemcpyAsync(g->f, fin.p, fbytes, hipMemcpyDeviceToDevice, g->stream));
+    if (ib) {
+        HIP_TRY(hipMemcpyAsync(g->rho, mrho.p, mbytes, hipMemcpyDeviceToDevice, g->stream));
+        HIP_TRY(hipMemcpyAsync(g->u, mu.p, mbytes * g->D, hipMemcpyDeviceToDevice, g->stream));
+    }
+    if (fin.p) HIP_TRY(hipMemcpyAsync(g->f, fin.p, fbytes, hipMemcpyDeviceToDevice, g->stream));
     g->parity = fin_par;
     g->t = fin_t;
     g->d.omega = fin_omega;
@@ -543,13 +743,13 @@ int adj_run(lumagpu_grid *g, int nsteps, int every, const double dir[3], int bac
     if (lambda0) {
         // LUMA's layout on the device, then one copy
         DevBuf lout;
-        if (int r = lout.alloc((size_t)g->Q * nc * sizeof(double))) return r;
+        if (int r = lout.alloc(g, (size_t)g->Q * nc * sizeof(double))) return r;
         const unsigned nb = (unsigned)((nc + 255) / 256);
         if (g->Q == 9)
-            k_adj_to_luma<9, T><<<nb, 256, 0, g->stream>>>(static_cast<const T *>(lam.p), nc, g->d.N, g->d.M, g->d.K,
+            k_adj_to_luma<9, T><<<nb, 256, 0, g->stream>>>(ab.gbar, g->ps, nc, g->d.N, g->d.M, g->d.K,
                                                          static_cast<double *>(lout.p));
         else
-            k_adj_to_luma<19, T><<<nb, 256, 0, g->stream>>>(static_cast<const T *>(lam.p), nc, g->d.N, g->d.M,
+            k_adj_to_luma<19, T><<<nb, 256, 0, g->stream>>>(ab.gbar, g->ps, nc, g->d.N, g->d.M,
                                                           g->d.K, static_cast<double *>(lout.p));
         HIP_TRY(hipGetLastError());
         if (int r = copy_to_host(g, lambda0, lout.p, (size_t)g->Q * nc * sizeof(double))) return r;
@@ -591,7 +791,10 @@ extern "C" int lumagpu_adj_run(lumagpu_grid *g, int nsteps, int checkpoint_every
         if (int r = ensure_flags(g)) return r;
         if (int r = upload_flags(g)) return r;
     }
-    if (g->d.precision == LUMAGPU_FP64)
-        return adj_run<P64>(g, nsteps, checkpoint_every, dir, backward, res, dJ_dpos, lambda0);
-    return adj_run<P32S>(g, nsteps, checkpoint_every, dir, backward, res, dJ_dpos, lambda0);
+    std::lock_guard<std::recursive_mutex> lock(g->f2_mu);
+    const int r = g->d.precision == LUMAGPU_FP64
+                      ? adj_run<P64>(g, nsteps, checkpoint_every, dir, backward, res, dJ_dpos, lambda0)
+                      : adj_run<P32S>(g, nsteps, checkpoint_every, dir, backward, res, dJ_dpos, lambda0);
+    trim_blocks(g);
+    return r;
 }

@@ -11,12 +11,15 @@
 // Objective: J = (1/T) sum_t dir . sum_m F_m eps_m ds_m vd_m (the body force LUMA writes to
 // Body_<id>_LD, ObjectManager_ops_io.cpp:98-121, averaged over the T steps).
 //
-// The adjoint runs the step backwards: the collision's transposed Jacobian per site
-// (k_adj_collide; regularised faces in k_adj_faces, edges and corners in k_adj_edges), then spread and interpolation swapped (the spread's adjoint gathers the
+// The adjoint runs the step backwards: reverse streaming of the later step (adj_lam: every
+// population adjoint is gathered from the site that pulled it) and the collision's transposed
+// Jacobian per site in one kernel (k_adj_collide; regularised faces in k_adj_faces, edges and
+// corners in k_adj_edges), then spread and interpolation swapped (the spread's adjoint gathers the
 // site force adjoint to the markers, k_adj_ibm_marker; the interpolation's adjoint spreads the
-// marker adjoint to the sites through the same per-site gather lists, k_adj_ibm_site), then
-// reverse streaming (k_adj_stream: every population adjoint is gathered from the site that
-// pulled it).  Adjoint arrays are plain [v][cell] (no AA layout): lam = dJ/df, gbar = dJ/dg.
+// marker adjoint to the sites through the same per-site gather lists, k_adj_ibm_site).  Only
+// gbar = dJ/dg goes through memory, in two arrays that trade places; lam = dJ/df is written once,
+// after the first step (k_adj_stream).  Adjoint arrays are plain [v][cell] (no AA layout), their
+// planes padded like the populations'.
 #pragma once
 
 #include "aa_kernels.hpp"
@@ -26,11 +29,17 @@ namespace lumagpu {
 
 template <class T>
 struct AdjArgs {
-    T *lam;          // [Q][ncell] adjoint of the post-collision populations
-    T *gbar;         // [Q][ncell] adjoint of the streamed populations
+    const T *gin;    // [Q][ps] adjoint of the populations the later step streamed
+    T *gbar;         // [Q][ps] adjoint of the streamed populations
+    size_t ps;       // plane stride of both
+    double ramp_feq; // StepArgs::ramp_feq of the later step (its velocity sources)
+    int ramp_on;
     double *fbar;    // [3][ncell] adjoint of the body-force field (flagged sites)
-    double *part;    // per-block partial sums: omega [0, nblk), inlet scale [nblk, 2 nblk)
-    int nblk;
+    // per-block partial sums: omega [0, nblk_all), the later step's inlet scale [nblk_all, 2 nblk_all);
+    // nblk blocks over the grid, then those of the site list
+    double *part;
+    int nblk, nblk_all;
+    int outlet;      // the grid has ExtrapolateRight sites
 };
 
 __device__ __forceinline__ int block_linear() {
@@ -61,6 +70,85 @@ __device__ __forceinline__ bool regularised_boundary_site(const StepArgs &a, uns
     return a.regularised && (ty == kVelocity || ty == kPressure);
 }
 
+// Reverse streaming at a fluid or regularised boundary site: lam_w(x) gathers the adjoint of
+// every streamed population that read f_w(x) -- the pull by x + c_w (a fluid or regularised
+// boundary site), the bounce-back at x itself when x + c_w is solid, and the pull through an
+// ExtrapolateRight source two cells to the right.  pl: a plain site (every neighbour fluid) is
+// pulled by its neighbours alone, no neighbour flag is read.  fx: the flag byte two cells to the
+// right (of the site itself at the grid's last two columns).
+template <int Q, class T>
+__device__ __forceinline__ void adj_lam(const StepArgs &a, const AdjArgs<T> &b, int x, int y, int z, size_t cell,
+                                        const Nbr &nb, bool pl, unsigned fx, T *acc) {
+    using L = Lattice<Q>;
+    const int nx = a.nx, ny = a.ny;
+    if (pl) {
+        static_for<Q>([&](auto wc) {
+            constexpr int w = decltype(wc)::value;
+            acc[w] = b.gin[(size_t)w * b.ps + nb.at(L::c(w, 0), L::c(w, 1), L::c(w, 2), nx, ny)];
+        });
+    } else {
+#pragma unroll
+        for (int w = 0; w < Q; ++w) {
+            const size_t yn = nb.at(L::c(w, 0), L::c(w, 1), L::c(w, 2), nx, ny);
+            const unsigned fn = a.flags[yn];
+            const int tn = fn & kTypeMask;
+            const bool pulled = tn == kFluid || regularised_boundary_site(a, fn);
+            // one load at a selected address: a load in each branch took the kernel from 138 to 256 registers
+            const T t = b.gin[tn == kSolid ? (size_t)L::opp(w) * b.ps + cell : (size_t)w * b.ps + yn];
+            acc[w] = (pulled || tn == kSolid) ? t : T(0);
+        }
+    }
+    if (x + 2 < nx && (fx & kTypeMask) == kExtrapRight) {
+        Nbr ns;
+        ns.init(x + 2, y, z, nx, ny, a.nz);
+#pragma unroll
+        for (int w = 0; w < Q; ++w) {
+            const size_t yp = ns.at(L::c(w, 0), L::c(w, 1), L::c(w, 2), nx, ny);
+            if ((a.flags[yp] & kTypeMask) == kFluid) acc[w] += b.gin[(size_t)w * b.ps + yp];
+        }
+    }
+}
+// the same at a listed boundary site
+template <int Q, class T>
+__device__ __forceinline__ void adj_lam_site(const StepArgs &a, const AdjArgs<T> &b, int x, int y, int z, size_t cell,
+                                             const Nbr &nb, double *lam) {
+    T acc[Q];
+    adj_lam<Q, T>(a, b, x, y, z, cell, nb, false, a.flags[x + 2 < a.nx ? cell + 2 : cell], acc);
+#pragma unroll
+    for (int v = 0; v < Q; ++v) lam[v] = double(acc[v]);
+}
+
+// The later step's derivative with respect to a scale s of the inlet profile (u_in -> s u_in) at a
+// site that pulls from forced-equilibrium velocity sources: gbar_v d feq_v(rho_in, s u_in) / ds at
+// s = 1.  A rolled loop over v (uniform, so its velocities come from scalar loads): few sites need it,
+// and unrolled its FP64 terms would hold registers that the whole kernel pays for.
+template <int Q, class T>
+__device__ __forceinline__ double adj_inlet(const StepArgs &a, const AdjArgs<T> &b, int x, int y, int z, size_t cell) {
+    using L = Lattice<Q>;
+    const int nx = a.nx, ny = a.ny;
+    double in_site = 0.0;
+#pragma unroll 1
+    for (int v = 0; v < Q; ++v) {
+        const int c0 = L::c(v, 0), c1 = L::c(v, 1), c2 = L::c(v, 2);
+        int sx = x - c0, sy = y - c1, sz = z - c2;
+        sx = sx < 0 ? nx - 1 : (sx >= nx ? 0 : sx);
+        sy = sy < 0 ? ny - 1 : (sy >= ny ? 0 : sy);
+        sz = sz < 0 ? a.nz - 1 : (sz >= a.nz ? 0 : sz);
+        if ((a.flags[cell_of(sx, sy, sz, nx, ny)] & kTypeMask) != kVelocity) continue;
+        // the source's velocity as the step's gather_in takes it (with a velocity ramp, the ramped
+        // profile of the pulling site's row)
+        const int js = b.ramp_on ? y : sy;
+        const double rf = b.ramp_feq;
+        const double us[3] = {a.uin[js] * rf, a.uin[ny + js] * rf, (L::D == 3) ? a.uin[2 * ny + js] * rf : 0.0};
+        const double cu = c0 * us[0] + c1 * us[1] + c2 * us[2];
+        // d feq_v / du . u_in = w rho_in (3 c.u + 9 (c.u)^2 - 3 u.u)
+        const double usq = us[0] * us[0] + us[1] * us[1] + us[2] * us[2];
+        const double d = L::w(v) * a.rho_in * (3.0 * cu + 9.0 * cu * cu - 3.0 * usq);
+        in_site += double(b.gin[(size_t)v * b.ps + cell]) * d;
+    }
+    return in_site;
+}
+
 // One forward-mode (Dual) pass of the transposed Jacobian of a regularised velocity face site's
 // update (regularised_face, :313-510, then BGK, :765-790) at its streamed populations g
 // (absolute): lam . d f' / d p for seed s, p = population s for s < Q, omega for s = Q and the
@@ -88,112 +176,150 @@ __device__ double adj_regularised_face(const StepArgs &a, unsigned fl, int y, co
     return acc;
 }
 
-// Transposed collision Jacobian at every fluid site: gbar = (d f'/d g)^T lam, fbar =
-// (d f'/d F)^T lam at forced sites, and the omega derivative sum_v lam_v d f'_v / d omega
-// (part[block]).  Regularised velocity faces run in k_adj_faces: their forward-mode passes
-// take several times this path's registers, and one kernel holding both ran at one wave per
-// SIMD with spills.
-// FP64 D3Q19: at most 256 VGPRs, two waves per SIMD (it needs 286 for one: 1.83 ms against
-// 1.21 ms with 28 B of spills on 6.3 M cells)
-template <int Q, class P, bool ODD>
-__global__ __launch_bounds__(256, (sizeof(typename P::T) == 8 && Q == 19) ? 2 : 1) void k_adj_collide(
-    StepArgs a, AdjArgs<typename P::T> b) {
+// Which sites a launch of k_adj_collide takes.  Small grids: all, in one launch.  Large ones as the
+// forward step: the plain sites by bitmap, without a flag, and a list of the others; rows whose
+// first and last sites are not plain otherwise send most waves through both paths one after the
+// other.  The column that feeds an outlet (x = nx - 3) is listed too: its populations are pulled
+// twice.
+enum AdjMode : int { kAdjAll = 0, kAdjPlain = 1, kAdjList = 2 };
+
+// One fluid site: reverse streaming of the later step (adj_lam) and the transposed collision Jacobian:
+// gbar = (d f'/d g)^T lam, fbar = (d f'/d F)^T lam at a forced site; returns the omega derivative
+// sum_v lam_v d f'_v / d omega.
+template <int Q, class P, bool ODD, int MODE>
+__device__ __forceinline__ double adj_site(const StepArgs &a, const AdjArgs<typename P::T> &b, int x, int y, int z,
+                                           size_t cell, bool pl, unsigned fx, unsigned fl, double &in_site) {
     using L = Lattice<Q>;
     using T = typename P::T;
-    const int x = blockIdx.x * blockDim.x + threadIdx.x;
-    const int y = blockIdx.y, z = blockIdx.z;
-    double om_site = 0.0;
-    if (x < a.nx) {
-        const size_t cell = cell_of(x, y, z, a.nx, a.ny);
-        // the flag byte and the plain-site bit in one round trip (plain sites are fluid sites
-        // whose pulls read no neighbour flag)
-        const bool pl = (a.plain[cell >> 5] >> (cell & 31)) & 1u;   // never null in the adjoint
-        const unsigned fl = a.flags[cell];
-        if (pl || (fl & kTypeMask) == kFluid) {   // a plain site is a fluid site
-            // the site's adjoint first: its loads need no flag, so they are in flight with the pulls
-            T lam[Q];
+    Nbr nb;
+    nb.init(x, y, z, a.nx, a.ny, a.nz);
+    T lam[Q];
+    adj_lam<Q, T>(a, b, x, y, z, cell, nb, pl, fx, lam);
+    if constexpr (MODE != kAdjPlain)
+        if (!a.regularised && !pl) in_site = adj_inlet<Q, T>(a, b, x, y, z, cell);
+    T fin[Q];
+    if (pl) gather_plain<Q, P, ODD>(a, cell, nb, fin);
+    else if constexpr (MODE != kAdjPlain) gather_in<Q, P, ODD>(a, x, y, z, cell, nb, kFluid, fin);
+    T g[Q];
 #pragma unroll
-            for (int v = 0; v < Q; ++v) lam[v] = b.lam[(size_t)v * a.ncell + cell];
-            Nbr nb;
-            nb.init(x, y, z, a.nx, a.ny, a.nz);
-            T fin[Q];
-            if (pl) gather_plain<Q, P, ODD>(a, cell, nb, fin);
-            else gather_in<Q, P, ODD>(a, x, y, z, cell, nb, kFluid, fin);
-            T g[Q];
+    for (int v = 0; v < Q; ++v) g[v] = P::kShift ? fin[v] + T(L::w(v) * a.rho0) : fin[v];
+    const bool forced = (fl & kForcedBit) != 0;
+    T F[3] = {T(0), T(0), T(0)};
+    if (forced) {
+        F[0] = T(a.force[cell]);
+        F[1] = T(a.force[a.ncell + cell]);
+        if constexpr (L::D == 3) F[2] = T(a.force[2 * a.ncell + cell]);
+    }
+    T rho = T(0), j[3] = {T(0), T(0), T(0)};
 #pragma unroll
-            for (int v = 0; v < Q; ++v) g[v] = P::kShift ? fin[v] + T(L::w(v) * a.rho0) : fin[v];
-            const bool forced = (fl & kForcedBit) != 0;
-            T F[3] = {T(0), T(0), T(0)};
-            if (forced) {
-                F[0] = T(a.force[cell]);
-                F[1] = T(a.force[a.ncell + cell]);
-                if constexpr (L::D == 3) F[2] = T(a.force[2 * a.ncell + cell]);
-            }
-            T rho = T(0), j[3] = {T(0), T(0), T(0)};
+    for (int v = 0; v < Q; ++v) {
+        rho += g[v];
+        j[0] += T(L::c(v, 0)) * g[v];
+        j[1] += T(L::c(v, 1)) * g[v];
+        j[2] += T(L::c(v, 2)) * g[v];
+    }
+    j[0] += T(0.5) * F[0];
+    j[1] += T(0.5) * F[1];
+    if constexpr (L::D == 3) {
+        if (a.fz_compat) j[0] += T(0.5) * F[2];
+        else j[2] += T(0.5) * F[2];
+    }
+    const T u[3] = {j[0] / rho, j[1] / rho, j[2] / rho};
+    const T usq = u[0] * u[0] + u[1] * u[1] + u[2] * u[2];
+    const T uF = u[0] * F[0] + u[1] * F[1] + u[2] * F[2];
+    const T om = T(a.omega), guo = T(1) - T(0.5) * om;
+    T S0 = T(0), Ua[3] = {T(0), T(0), T(0)}, Ga[3] = {T(0), T(0), T(0)}, Fb[3] = {T(0), T(0), T(0)};
+    T omb = T(0);
 #pragma unroll
-            for (int v = 0; v < Q; ++v) {
-                rho += g[v];
-                j[0] += T(L::c(v, 0)) * g[v];
-                j[1] += T(L::c(v, 1)) * g[v];
-                j[2] += T(L::c(v, 2)) * g[v];
-            }
-            j[0] += T(0.5) * F[0];
-            j[1] += T(0.5) * F[1];
-            if constexpr (L::D == 3) {
-                if (a.fz_compat) j[0] += T(0.5) * F[2];
-                else j[2] += T(0.5) * F[2];
-            }
-            const T u[3] = {j[0] / rho, j[1] / rho, j[2] / rho};
-            const T usq = u[0] * u[0] + u[1] * u[1] + u[2] * u[2];
-            const T uF = u[0] * F[0] + u[1] * F[1] + u[2] * F[2];
-            const T om = T(a.omega), guo = T(1) - T(0.5) * om;
-            T S0 = T(0), Ua[3] = {T(0), T(0), T(0)}, Ga[3] = {T(0), T(0), T(0)}, Fb[3] = {T(0), T(0), T(0)};
-            T omb = T(0);
+    for (int v = 0; v < Q; ++v) {
+        const T cx = T(L::c(v, 0)), cy = T(L::c(v, 1)), cz = T(L::c(v, 2)), w = T(L::w(v));
+        const T cu = cx * u[0] + cy * u[1] + cz * u[2];
+        const T cF = cx * F[0] + cy * F[1] + cz * F[2];
+        const T e = T(1) + T(3) * cu + T(4.5) * cu * cu - T(1.5) * usq;
+        const T lw = lam[v] * w;
+        S0 += lw * e;
+        Ua[0] += lw * (T(3) * cx + T(9) * cu * cx - T(3) * u[0]);
+        Ua[1] += lw * (T(3) * cy + T(9) * cu * cy - T(3) * u[1]);
+        Ua[2] += lw * (T(3) * cz + T(9) * cu * cz - T(3) * u[2]);
+        T dom = w * rho * e - g[v];
+        if (forced) {
+            Ga[0] += lw * (T(-3) * F[0] + T(9) * cx * cF);
+            Ga[1] += lw * (T(-3) * F[1] + T(9) * cy * cF);
+            Ga[2] += lw * (T(-3) * F[2] + T(9) * cz * cF);
+            Fb[0] += lw * (T(3) * (cx - u[0]) + T(9) * cu * cx);
+            Fb[1] += lw * (T(3) * (cy - u[1]) + T(9) * cu * cy);
+            Fb[2] += lw * (T(3) * (cz - u[2]) + T(9) * cu * cz);
+            dom -= T(0.5) * w * (T(3) * (cF - uF) + T(9) * cu * cF);
+        }
+        omb += lam[v] * dom;
+    }
+    T ub[3], jb[3];
+    for (int d = 0; d < 3; ++d) {
+        ub[d] = om * rho * Ua[d] + guo * Ga[d];
+        jb[d] = ub[d] / rho;
+    }
+    if constexpr (L::D == 2) jb[2] = T(0);
+    const T rb = om * S0 - (ub[0] * u[0] + ub[1] * u[1] + ub[2] * u[2]) / rho;
 #pragma unroll
-            for (int v = 0; v < Q; ++v) {
-                const T cx = T(L::c(v, 0)), cy = T(L::c(v, 1)), cz = T(L::c(v, 2)), w = T(L::w(v));
-                const T cu = cx * u[0] + cy * u[1] + cz * u[2];
-                const T cF = cx * F[0] + cy * F[1] + cz * F[2];
-                const T e = T(1) + T(3) * cu + T(4.5) * cu * cu - T(1.5) * usq;
-                const T lw = lam[v] * w;
-                S0 += lw * e;
-                Ua[0] += lw * (T(3) * cx + T(9) * cu * cx - T(3) * u[0]);
-                Ua[1] += lw * (T(3) * cy + T(9) * cu * cy - T(3) * u[1]);
-                Ua[2] += lw * (T(3) * cz + T(9) * cu * cz - T(3) * u[2]);
-                T dom = w * rho * e - g[v];
-                if (forced) {
-                    Ga[0] += lw * (T(-3) * F[0] + T(9) * cx * cF);
-                    Ga[1] += lw * (T(-3) * F[1] + T(9) * cy * cF);
-                    Ga[2] += lw * (T(-3) * F[2] + T(9) * cz * cF);
-                    Fb[0] += lw * (T(3) * (cx - u[0]) + T(9) * cu * cx);
-                    Fb[1] += lw * (T(3) * (cy - u[1]) + T(9) * cu * cy);
-                    Fb[2] += lw * (T(3) * (cz - u[2]) + T(9) * cu * cz);
-                    dom -= T(0.5) * w * (T(3) * (cF - uF) + T(9) * cu * cF);
-                }
-                omb += lam[v] * dom;
+    for (int v = 0; v < Q; ++v)
+        b.gbar[(size_t)v * b.ps + cell] = (T(1) - om) * lam[v] + rb + T(L::c(v, 0)) * jb[0] +
+                                            T(L::c(v, 1)) * jb[1] + T(L::c(v, 2)) * jb[2];
+    if (forced) {
+        double Fbar[3] = {double(guo * Fb[0] + T(0.5) * jb[0]), double(guo * Fb[1] + T(0.5) * jb[1]),
+                          double(guo * Fb[2])};
+        if constexpr (L::D == 3) Fbar[2] += double(T(0.5) * (a.fz_compat ? jb[0] : jb[2]));
+        for (int d = 0; d < L::D; ++d) b.fbar[(size_t)d * a.ncell + cell] = Fbar[d];
+    }
+    return double(omb);
+}
+
+// Every fluid site (see AdjMode), one pass: f and gin read, gbar written, 3 Q values per cell; with
+// the streaming in a kernel of its own it was 5 Q, lam written and read again.  192 x 80 x 80 FP32
+// per reversed step: 133 + 59 us in two kernels over all sites, 52 + 45 us (plain sites, list) here.  Regularised
+// velocity faces run in k_adj_faces: their forward-mode passes take several times this path's
+// registers, and one kernel holding both ran at one wave per SIMD with spills.
+// FP64 D3Q19: at most 256 VGPRs, two waves per SIMD (it needs 286 for one: 1.83 ms against
+// 1.21 ms with 28 B of spills on 6.3 M cells)
+template <int Q, class P, bool ODD, int MODE>
+__global__ __launch_bounds__(256, (sizeof(typename P::T) == 8 && Q == 19) ? 2 : 1) void k_adj_collide(
+    StepArgs a, AdjArgs<typename P::T> b, const int *cells, int n) {
+    double om_site = 0.0, in_site = 0.0;
+    if constexpr (MODE == kAdjList) {
+        const int i = blockIdx.x * blockDim.x + threadIdx.x;
+        if (i < n) {
+            const size_t cell = (size_t)cells[i];
+            int x, y, z;
+            cell_coords(a, (uint32_t)cell, x, y, z);
+            const bool pl = (a.plain[cell >> 5] >> (cell & 31)) & 1u;
+            const unsigned fx = a.flags[x + 2 < a.nx ? cell + 2 : cell];
+            om_site = adj_site<Q, P, ODD, MODE>(a, b, x, y, z, cell, pl, fx, a.flags[cell], in_site);
+        }
+    } else {
+        const int x = blockIdx.x * blockDim.x + threadIdx.x;
+        const int y = blockIdx.y, z = blockIdx.z;
+        if (x < a.nx) {
+            const size_t cell = cell_of(x, y, z, a.nx, a.ny);
+            // the flag bytes and the plain-site bit in one round trip (plain sites are fluid sites
+            // whose pulls read no neighbour flag)
+            const bool pl = (a.plain[cell >> 5] >> (cell & 31)) & 1u;   // never null in the adjoint
+            const unsigned fl = a.flags[cell];
+            if constexpr (MODE == kAdjPlain) {
+                // the flag byte of the cell itself is no outlet's
+                if (pl && !(b.outlet && x == a.nx - 3))
+                    om_site = adj_site<Q, P, ODD, MODE>(a, b, x, y, z, cell, true, kFluid, fl, in_site);
+            } else {
+                const unsigned fx = a.flags[x + 2 < a.nx ? cell + 2 : cell];
+                if (pl || (fl & kTypeMask) == kFluid)   // a plain site is a fluid site
+                    om_site = adj_site<Q, P, ODD, MODE>(a, b, x, y, z, cell, pl, fx, fl, in_site);
             }
-            T ub[3], jb[3];
-            for (int d = 0; d < 3; ++d) {
-                ub[d] = om * rho * Ua[d] + guo * Ga[d];
-                jb[d] = ub[d] / rho;
-            }
-            if constexpr (L::D == 2) jb[2] = T(0);
-            const T rb = om * S0 - (ub[0] * u[0] + ub[1] * u[1] + ub[2] * u[2]) / rho;
-#pragma unroll
-            for (int v = 0; v < Q; ++v)
-                b.gbar[(size_t)v * a.ncell + cell] = (T(1) - om) * lam[v] + rb + T(L::c(v, 0)) * jb[0] +
-                                                    T(L::c(v, 1)) * jb[1] + T(L::c(v, 2)) * jb[2];
-            if (forced) {
-                double Fbar[3] = {double(guo * Fb[0] + T(0.5) * jb[0]), double(guo * Fb[1] + T(0.5) * jb[1]),
-                                  double(guo * Fb[2])};
-                if constexpr (L::D == 3) Fbar[2] += double(T(0.5) * (a.fz_compat ? jb[0] : jb[2]));
-                for (int d = 0; d < L::D; ++d) b.fbar[(size_t)d * a.ncell + cell] = Fbar[d];
-            }
-            om_site = double(omb);
         }
     }
-    const double s = block_sum(om_site);
-    if (threadIdx.x == 0) b.part[block_linear()] = s;
+    const double s = block_sum(om_site), si = MODE == kAdjPlain ? 0.0 : block_sum(in_site);
+    if (threadIdx.x == 0) {
+        const int blk = block_linear() + (MODE == kAdjList ? b.nblk : 0);
+        b.part[blk] = s;
+        b.part[b.nblk_all + blk] = si;
+    }
 }
 
 // Regularised velocity face sites (cells[i]): gbar from adj_regularised_face at the site's
@@ -216,13 +342,11 @@ __global__ __launch_bounds__(64) void k_adj_faces(StepArgs a, AdjArgs<typename P
     T fin[Q];
     gather_in<Q, P, ODD>(a, x, y, z, cell, nb, kVelocity, fin);
     double g[Q], lam[Q];
+    adj_lam_site<Q, T>(a, b, x, y, z, cell, nb, lam);
 #pragma unroll
-    for (int v = 0; v < Q; ++v) {
-        g[v] = double(fin[v]) + (P::kShift ? L::w(v) * a.rho0 : 0.0);
-        lam[v] = double(b.lam[(size_t)v * a.ncell + cell]);
-    }
+    for (int v = 0; v < Q; ++v) g[v] = double(fin[v]) + (P::kShift ? L::w(v) * a.rho0 : 0.0);
     const double d = adj_regularised_face<Q>(a, a.flags[cell], y, g, lam, s);
-    if (s < Q) b.gbar[(size_t)s * a.ncell + cell] = T(d);
+    if (s < Q) b.gbar[(size_t)s * b.ps + cell] = T(d);
     else fpart[(s - Q) * n + i] = d;
 }
 
@@ -251,10 +375,9 @@ __global__ __launch_bounds__(64) void k_adj_edges(StepArgs a, EdgeArgs e, AdjArg
     T fin[Q];
     gather_in<Q, P, ODD>(a, x, y, z, cell, nb, kVelocity, fin);
     double g[Q], lam[Q];
-    for (int v = 0; v < Q; ++v) {
-        g[v] = double(fin[v]) + (P::kShift ? L::w(v) * a.rho0 : 0.0);
-        lam[v] = double(b.lam[(size_t)v * a.ncell + cell]);
-    }
+    adj_lam_site<Q, T>(a, b, x, y, z, cell, nb, lam);
+#pragma unroll
+    for (int v = 0; v < Q; ++v) g[v] = double(fin[v]) + (P::kShift ? L::w(v) * a.rho0 : 0.0);
     const double *er1 = e.erho + 8 * (size_t)i, *er2 = er1 + 4;
     const bool pressure = (a.flags[cell] & kTypeMask) == kPressure;
     const int ncode = (a.flags[cell] >> kNormalShift) & 7;
@@ -284,7 +407,7 @@ __global__ __launch_bounds__(64) void k_adj_edges(StepArgs a, EdgeArgs e, AdjArg
 #pragma unroll
     for (int w = 0; w < Q; ++w) acc += lam[w] * fout[w].d;
     // every output of the site has one seed that writes it; the other kind's are zero
-    if (s < Q) b.gbar[(size_t)s * a.ncell + cell] = T(acc);
+    if (s < Q) b.gbar[(size_t)s * b.ps + cell] = T(acc);
     else if (s == Q) epart[i] = acc;
     else if (pressure) tbar[3 * (size_t)i + (s - Q - 1)] = acc;
     else if (s == Q + 1) dbar[i] = acc;
@@ -300,7 +423,7 @@ __global__ __launch_bounds__(64) void k_adj_edges(StepArgs a, EdgeArgs e, AdjArg
 // neighbour cell, its entries in a fixed order (no atomics).
 template <int Q, class T>
 __global__ void k_adj_edge_nbrs(int nn, const int *ncell, const int *ptr, const int *ent, const double *dbar,
-                                const double *tbar, const double *erho, size_t ncell_total, T *gbar) {
+                                const double *tbar, const double *erho, size_t ps, T *gbar) {
     using L = Lattice<Q>;
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= nn) return;
@@ -318,88 +441,41 @@ __global__ void k_adj_edge_nbrs(int nn, const int *ncell, const int *ptr, const 
         }
     }
     const size_t cell = (size_t)ncell[k];
-    for (int v = 0; v < Q; ++v) gbar[(size_t)v * ncell_total + cell] += T(s[v]);
+    for (int v = 0; v < Q; ++v) gbar[(size_t)v * ps + cell] += T(s[v]);
 }
 
-// Reverse streaming: lam_w(x) gathers the adjoint of every streamed population that read
-// f_w(x) -- the pull by x + c_w (a fluid or regularised boundary site), the bounce-back at
-// x itself when x + c_w is solid, and the pull through an ExtrapolateRight source two cells to
-// the right.  Also the derivative with
-// respect to a scale s of the inlet profile (u_in -> s u_in) of the forced-equilibrium
-// velocity sources, d feq_v(rho_in, s u_in) / ds at s = 1.
+// Reverse streaming alone, after the first step has been reversed: lam = dJ/df of the initial
+// populations (null: only that step's inlet derivative, part[nblk_all + block]).
 template <int Q, class P>
-__global__ __launch_bounds__(256) void k_adj_stream(StepArgs a, AdjArgs<typename P::T> b) {
-    using L = Lattice<Q>;
+__global__ __launch_bounds__(256) void k_adj_stream(StepArgs a, AdjArgs<typename P::T> b, typename P::T *out) {
     using T = typename P::T;
     const int x = blockIdx.x * blockDim.x + threadIdx.x;
     const int y = blockIdx.y, z = blockIdx.z;
     double in_site = 0.0;
     if (x < a.nx) {
-        const int nx = a.nx, ny = a.ny;
-        const size_t cell = cell_of(x, y, z, nx, ny);
-        // the site's flag, the plain-site bit and the flag two sites downstream in one round trip.
-        // A plain site (every neighbour fluid) is pulled by its neighbours alone and pulls from no
-        // velocity source: no neighbour flag to read
+        const size_t cell = cell_of(x, y, z, a.nx, a.ny);
         const bool pl = (a.plain[cell >> 5] >> (cell & 31)) & 1u;   // never null in the adjoint
-        const unsigned fx = a.flags[x + 2 < nx ? cell + 2 : cell];
-        const bool xr = (x + 2 < nx) && ((fx & kTypeMask) == kExtrapRight);
+        const unsigned fx = a.flags[x + 2 < a.nx ? cell + 2 : cell];
         const unsigned fl = a.flags[cell];
-        const int ty = fl & kTypeMask;
-        if (pl || ty == kFluid || regularised_boundary_site(a, fl)) {   // a plain site is a fluid site
+        T acc[Q];
+        if (pl || (fl & kTypeMask) == kFluid || regularised_boundary_site(a, fl)) {
             Nbr nb;
-            nb.init(x, y, z, nx, ny, a.nz);
-            Nbr ns;
-            if (xr) ns.init(x + 2, y, z, nx, ny, a.nz);
-            // every load before the first store: a store to lam would otherwise order the
-            // following loads (of gbar, and of flags, which may alias anything) behind it
-            T acc[Q];
-            if (pl) {
-                static_for<Q>([&](auto wc) {
-                    constexpr int w = decltype(wc)::value;
-                    acc[w] = b.gbar[(size_t)w * a.ncell + nb.at(L::c(w, 0), L::c(w, 1), L::c(w, 2), nx, ny)];
-                });
-            } else {
-#pragma unroll
-                for (int w = 0; w < Q; ++w) {
-                    const size_t yn = nb.at(L::c(w, 0), L::c(w, 1), L::c(w, 2), nx, ny);
-                    const unsigned fn = a.flags[yn];
-                    const int tn = fn & kTypeMask;
-                    acc[w] = T(0);
-                    if (tn == kFluid || regularised_boundary_site(a, fn)) acc[w] = b.gbar[(size_t)w * a.ncell + yn];
-                    else if (tn == kSolid) acc[w] = b.gbar[(size_t)L::opp(w) * a.ncell + cell];
-                }
-            }
-            if (xr) {
-#pragma unroll
-                for (int w = 0; w < Q; ++w) {
-                    const size_t yp = ns.at(L::c(w, 0), L::c(w, 1), L::c(w, 2), nx, ny);
-                    if ((a.flags[yp] & kTypeMask) == kFluid) acc[w] += b.gbar[(size_t)w * a.ncell + yp];
-                }
-            }
-            if (!a.regularised && !pl) {
-                for (int v = 0; v < Q; ++v) {
-                    const size_t src = nb.at(-L::c(v, 0), -L::c(v, 1), -L::c(v, 2), nx, ny);
-                    if ((a.flags[src] & kTypeMask) != kVelocity) continue;
-                    // the source's velocity as the step's gather_in takes it (with a velocity ramp,
-                    // the ramped profile of the pulling site's row)
-                    const int js = a.ramp_on ? y : nb.ys[1 - L::c(v, 1)];
-                    const double rf = a.ramp_feq;
-                    const double us[3] = {a.uin[js] * rf, a.uin[ny + js] * rf, (L::D == 3) ? a.uin[2 * ny + js] * rf : 0.0};
-                    const double cu = L::c(v, 0) * us[0] + L::c(v, 1) * us[1] + L::c(v, 2) * us[2];
-                    // d feq_v / du . u_in = w rho_in (3 c.u + 9 (c.u)^2 - 3 u.u)
-                    const double usq = us[0] * us[0] + us[1] * us[1] + us[2] * us[2];
-                    const double d = L::w(v) * a.rho_in * (3.0 * cu + 9.0 * cu * cu - 3.0 * usq);
-                    in_site += double(b.gbar[(size_t)v * a.ncell + cell]) * d;
-                }
-            }
-#pragma unroll
-            for (int w = 0; w < Q; ++w) b.lam[(size_t)w * a.ncell + cell] = acc[w];
+            nb.init(x, y, z, a.nx, a.ny, a.nz);
+            if (out) adj_lam<Q, T>(a, b, x, y, z, cell, nb, pl, fx, acc);
+            if (!a.regularised && !pl) in_site = adj_inlet<Q, T>(a, b, x, y, z, cell);
         } else {
-            for (int w = 0; w < Q; ++w) b.lam[(size_t)w * a.ncell + cell] = T(0);
+#pragma unroll
+            for (int w = 0; w < Q; ++w) acc[w] = T(0);
         }
+        if (out)
+#pragma unroll
+            for (int w = 0; w < Q; ++w) out[(size_t)w * b.ps + cell] = acc[w];
     }
     const double s = block_sum(in_site);
-    if (threadIdx.x == 0) b.part[b.nblk + block_linear()] = s;
+    if (threadIdx.x == 0) {
+        b.part[block_linear()] = 0.0;
+        b.part[b.nblk_all + block_linear()] = s;
+    }
 }
 
 // IB adjoint, marker side: the spread's adjoint gathers the site force adjoint to the
@@ -472,23 +548,43 @@ static __global__ __launch_bounds__(256) void k_adj_ibm_marker(IbmArgs ib, AdjIb
 // IB adjoint, site side: the interpolation's adjoint spread through the per-site gather lists
 // (no atomics): gbar_v(s) += rho_bar_s + c_v . j_bar_s at every fluid support site.
 template <int Q, class T>
-__global__ void k_adj_ibm_site(IbmArgs ib, const double *mbar, const uint8_t *flags, T *gbar) {
+__global__ void k_adj_ibm_site(IbmArgs ib, const double *mbar, const uint8_t *flags, size_t ps, T *gbar) {
     using L = Lattice<Q>;
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= ib.nsites) return;
     const size_t cell = (size_t)ib.sites[s];
     if ((flags[cell] & kTypeMask) != kFluid) return;
+    // every load of a step before its sums and stores: a chunk's entries, their weights and markers,
+    // and the site's Q adjoints (which a store between them would put behind it)
+    T old[Q];
+#pragma unroll
+    for (int v = 0; v < Q; ++v) old[v] = gbar[(size_t)v * ps + cell];
+    constexpr int CH = 6;
     double jb[3] = {0.0, 0.0, 0.0}, rb = 0.0;
-    for (int e = ib.sptr[s]; e < ib.sptr[s + 1]; ++e) {
-        const int code = ib.sent[e];
-        const int m = code / ib.S;
-        const double dl = ib.sdelta[code];
-        for (int d = 0; d < 3; ++d) jb[d] += dl * mbar[4 * m + d];
-        rb += dl * mbar[4 * m + 3];
+    const int e0 = ib.sptr[s], e1 = ib.sptr[s + 1];
+    for (int eb = e0; eb < e1; eb += CH) {
+        int code[CH];
+        double dl[CH], mb[CH][4];
+#pragma unroll
+        for (int k = 0; k < CH; ++k) code[k] = ib.sent[eb + k < e1 ? eb + k : eb];
+#pragma unroll
+        for (int k = 0; k < CH; ++k) {
+            dl[k] = ib.sdelta[code[k]];
+            const double *m = mbar + 4 * (code[k] / ib.S);
+#pragma unroll
+            for (int d = 0; d < 4; ++d) mb[k][d] = m[d];
+        }
+#pragma unroll
+        for (int k = 0; k < CH; ++k)
+            if (eb + k < e1) {
+#pragma unroll
+                for (int d = 0; d < 3; ++d) jb[d] += dl[k] * mb[k][d];
+                rb += dl[k] * mb[k][3];
+            }
     }
+#pragma unroll
     for (int v = 0; v < Q; ++v)
-        gbar[(size_t)v * ib.ncell + cell] +=
-            T(rb + L::c(v, 0) * jb[0] + L::c(v, 1) * jb[1] + L::c(v, 2) * jb[2]);
+        gbar[(size_t)v * ps + cell] = old[v] + T(rb + L::c(v, 0) * jb[0] + L::c(v, 1) * jb[1] + L::c(v, 2) * jb[2]);
 }
 
 // ---- positions through epsilon and ds -------------------------------------------------------
@@ -595,6 +691,7 @@ static __global__ void k_adj_objective(IbmArgs ib, double dx, double dy, double 
     const int lane = threadIdx.x;
     const double dir[3] = {dx, dy, dz};
     double s = 0.0;
+#pragma unroll 4
     for (int m = lane; m < ib.nm; m += 64) {
         const double w = ib.eps[m] * ((ib.D == 3) ? ib.ds[m] : 1.0) * ib.ds[m];
         double fd = 0.0;
@@ -605,23 +702,50 @@ static __global__ void k_adj_objective(IbmArgs ib, double dx, double dy, double 
     if (lane == 0) acc[0] += s * invT;
 }
 
+// A forced-equilibrium velocity site never steps: its slots hold what its neighbours pushed in the
+// last odd step, and a state reached along the tape by an even step has them in the state before.
+template <int Q, class S>
+__global__ __launch_bounds__(256) void k_adj_carry(StepArgs a, const S *from, S *to) {
+    using L = Lattice<Q>;
+    const size_t cell = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (cell >= a.ncell || (a.flags[cell] & kTypeMask) != kVelocity) return;
+    int x, y, z;
+    cell_coords(a, (uint32_t)cell, x, y, z);
+    Nbr nb;
+    nb.init(x, y, z, a.nx, a.ny, a.nz);
+    static_for<Q>([&](auto vc) {
+        constexpr int v = decltype(vc)::value;
+        const int t = a.flags[nb.at(-L::c(v, 0), -L::c(v, 1), -L::c(v, 2), a.nx, a.ny)] & kTypeMask;
+        if (t == kFluid || t == kExtrapRight) to[(size_t)v * a.ps + cell] = from[(size_t)v * a.ps + cell];
+    });
+}
+
 // The initial populations' adjoint in LUMA's layout f[v + Q*id], id = k + j*K + i*K*M, from
 // the [v][cell] array: one thread per cell, reads coalesced, each thread's Q values contiguous
 template <int Q, class T>
-__global__ void k_adj_to_luma(const T *lam, size_t nc, int N, int M, int K, double *out) {
+__global__ void k_adj_to_luma(const T *lam, size_t ps, size_t nc, int N, int M, int K, double *out) {
     const size_t cell = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (cell >= nc) return;
     const size_t i = cell % N, j = (cell / N) % M, k = cell / ((size_t)N * M);
     const size_t id = k + j * K + i * (size_t)K * M;
-    for (int v = 0; v < Q; ++v) out[v + Q * id] = double(lam[(size_t)v * nc + cell]);
+    for (int v = 0; v < Q; ++v) out[v + Q * id] = double(lam[(size_t)v * ps + cell]);
 }
 
-// acc[k] += sum of part[k*n .. k*n + n), k = 0..nk-1; one block of 1024, each thread with
-// four independent running sums (loads in flight), then a fixed tree: the order is fixed
-static __global__ __launch_bounds__(1024) void k_adj_sum_partials(const double *part, int n, int nk, double w0,
-                                                                   double *acc) {
+// Up to three pairs of partial sums in one launch, a block each: acc[0] += w0 * sum of part[0 .. n)
+// (omega, w0 this step's d omega_t / d omega, 1 without a ramp), acc[1] += sum of part[n .. 2n)
+// (inlet scale).  Each thread has four independent running sums (loads in flight), then a fixed
+// tree: the order is fixed.
+struct AdjSums {
+    const double *part[3];
+    int n[3];
+    double *acc[3];
+};
+static __global__ __launch_bounds__(1024) void k_adj_sum_partials(AdjSums sums, double w0) {
     __shared__ double sh[1024];
-    for (int k = 0; k < nk; ++k) {
+    const double *part = sums.part[blockIdx.x];
+    double *acc = sums.acc[blockIdx.x];
+    const int n = sums.n[blockIdx.x];
+    for (int k = 0; k < 2; ++k) {
         const double *p = part + (size_t)k * n;
         double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
         int i = threadIdx.x;
@@ -638,7 +762,6 @@ static __global__ __launch_bounds__(1024) void k_adj_sum_partials(const double *
             if ((int)threadIdx.x < st) sh[threadIdx.x] += sh[threadIdx.x + st];
             __syncthreads();
         }
-        // the first partial (omega) scaled by this step's d omega_t / d omega (1 without a ramp)
         if (threadIdx.x == 0) acc[k] += k == 0 ? w0 * sh[0] : sh[0];
         __syncthreads();
     }

@@ -69,9 +69,17 @@ void f2_give_back() {
             continue;
         }
         if (o->stream) (void)hipStreamSynchronize(o->stream);
-        (void)hipFree(o->f2);
-        o->f2 = nullptr;
+        if (o->f2_auto) {
+            (void)hipFree(o->f2);
+            o->f2 = nullptr;
+        }
         o->f2_auto = o->pair_synced = 0;
+        std::vector<lumagpu_grid::Block> kept;
+        for (auto &b : o->blocks) {
+            if (b.used) kept.push_back(b);
+            else (void)hipFree(b.p);
+        }
+        o->blocks = std::move(kept);
         o->f2_mu.unlock();
         g_f2_grids.erase(g_f2_grids.begin() + k);
     }
@@ -81,6 +89,15 @@ void f2_forget(lumagpu_grid *g) {
     std::lock_guard<std::mutex> lock(g_f2_grids_mu);
     g_f2_grids.erase(std::remove(g_f2_grids.begin(), g_f2_grids.end(), g), g_f2_grids.end());
 }
+
+}  // namespace
+namespace lumagpu {
+void scratch_listed(lumagpu_grid *g) {
+    std::lock_guard<std::mutex> lock(g_f2_grids_mu);
+    if (std::find(g_f2_grids.begin(), g_f2_grids.end(), g) == g_f2_grids.end()) g_f2_grids.push_back(g);
+}
+}  // namespace lumagpu
+namespace {
 
 // with g->f2_mu held: true when g->f2 is there
 bool f2_ensure(lumagpu_grid *g) {
@@ -94,8 +111,7 @@ bool f2_ensure(lumagpu_grid *g) {
     }
     g->f2_auto = 1;
     g->pair_synced = 0;
-    std::lock_guard<std::mutex> lock(g_f2_grids_mu);
-    g_f2_grids.push_back(g);
+    scratch_listed(g);
     return true;
 }
 
@@ -318,6 +334,7 @@ int begin_step(lumagpu_grid *g) {
 
 // after a step's kernels: the next step's outlet sources are in the other buffer if they wrote them
 void outlet_written(lumagpu_grid *g, const StepArgs &a) {
+    if (g->xr_tape) return;   // the caller moves along its tape
     if (a.xr_next) {
         g->xr_sel ^= 1;
         g->xr_ready = 1;
@@ -1036,6 +1053,7 @@ int lumagpu_grid_destroy(lumagpu_grid *g) {
     (void)hipFree(g->f);
     f2_forget(g);
     (void)hipFree(g->f2);
+    for (auto &b : g->blocks) (void)hipFree(b.p);
     (void)hipFree(g->pair_deep);
     (void)hipFree(g->pair_cells);
     (void)hipFree(g->pair_links);
@@ -1540,9 +1558,8 @@ int lumagpu_set_velocity_ramp(lumagpu_grid *g, double ramp_time) {
 
 int lumagpu_set_temporal_blocking(lumagpu_grid *g, int shape, int zchunk) {
     if (int r = check_grid(g)) return r;
-    std::lock_guard<std::mutex> lock(g->f2_mu);
+    std::lock_guard<std::recursive_mutex> lock(g->f2_mu);
     if (shape < 0) {
-        f2_forget(g);
         g->f2_auto = 0;
         g->fuse_off = 1;
         if (g->f2) {
@@ -1568,9 +1585,7 @@ int lumagpu_set_temporal_blocking(lumagpu_grid *g, int shape, int zchunk) {
         g->f2 = nullptr;
         return fail(LUMAGPU_ENOMEM, "second population array");
     }
-    // asked for: no longer one to give back
-    f2_forget(g);
-    g->f2_auto = 0;
+    g->f2_auto = 0;   // asked for: no longer one to give back
     g->pair_synced = 0;
     g->fuse_off = 0;
     g->fuse_shape = shape;
@@ -1687,7 +1702,7 @@ int lumagpu_reset_forces(lumagpu_grid *g) {
 
 int lumagpu_run(lumagpu_grid *g, int nsteps) {
     if (int r = check_grid(g)) return r;
-    std::lock_guard<std::mutex> lock(g->f2_mu);
+    std::lock_guard<std::recursive_mutex> lock(g->f2_mu);
     if (nsteps < 0) return fail(LUMAGPU_EINVAL, "negative step count");
     if (g->half) return fail(LUMAGPU_ESTATE, "a split step is open on this grid: finish it with lumagpu_force_collide_swap");
     int s = 0;

@@ -23,8 +23,20 @@ struct lumagpu_grid {
     size_t melem = 8;                 // bytes per element of the macro, force and side arrays
     void *f = nullptr;
     void *f2 = nullptr;               // second population array of the kernels that take several steps per launch
+    void *f_to = nullptr;             // a labelled step's destination when not f itself (the adjoint's tape)
+    double *xr_tape = nullptr;        // the adjoint's tape of outlet side buffers, one per step of a segment
     int f2_auto = 0;                  // it was allocated by a run, not asked for: given back when memory is short
-    std::mutex f2_mu;                 // held by whoever uses or frees f2
+    // held by whoever uses or frees f2 and blocks; an allocation inside a run takes back its own grid's
+    // unused blocks too, so it may be locked again by its holder
+    std::recursive_mutex f2_mu;
+    // blocks of the last adjoint run, kept for the next (adjoint.hip); freed with the grid or when
+    // memory is short
+    struct Block {
+        void *p;
+        size_t bytes;
+        int used;
+    };
+    std::vector<Block> blocks;
     int fuse_off = 0;                 // lumagpu_set_temporal_blocking turned several steps per launch off
     // two steps per launch on a large 3D grid (fused_kernels.hpp): the deep cells, the cells around the
     // others (S1) and the others (S) with their link words
@@ -110,6 +122,8 @@ namespace lumagpu {
 // thread-local message behind lumagpu_last_error()
 int fail(int code, const std::string &msg);
 
+// listed among the grids whose own arrays (f2, blocks) can be taken back while nothing runs on them
+void scratch_listed(lumagpu_grid *g);
 // hipMalloc that, short of memory, first takes back what runs allocated for themselves (api.hip)
 hipError_t dev_malloc(void **p, size_t bytes);
 
@@ -130,7 +144,7 @@ inline StepArgs make_args(const lumagpu_grid *g) {
     StepArgs a;
     std::memset(&a, 0, sizeof a);   // padding included: the bytes key the cached step graph
     a.f = g->f;
-    a.fo = g->f;
+    a.fo = g->f_to ? g->f_to : g->f;
     a.ps = g->ps;
     a.nx = g->d.N;
     a.ny = g->d.M;
@@ -187,9 +201,14 @@ inline StepArgs make_args(const lumagpu_grid *g) {
     }
     a.kids = g->d_kids;
     a.nkids = (int)g->kids.size();
-    a.xr = g->xr ? g->xr + (size_t)g->xr_sel * g->Q * g->d.M * g->d.K * (g->melem / sizeof(double)) : nullptr;
-    a.xr_next = (g->xr && g->xr_fold) ? g->xr + (size_t)(g->xr_sel ^ 1) * g->Q * g->d.M * g->d.K * (g->melem / sizeof(double))
-                                       : nullptr;
+    const size_t xr_size = (size_t)g->Q * g->d.M * g->d.K * (g->melem / sizeof(double));
+    if (g->xr_tape) {
+        a.xr = g->xr_tape;
+        a.xr_next = g->xr_tape + xr_size;
+    } else if (g->xr) {
+        a.xr = g->xr + (size_t)g->xr_sel * xr_size;
+        a.xr_next = g->xr_fold ? g->xr + (size_t)(g->xr_sel ^ 1) * xr_size : nullptr;
+    }
     a.stale = g->stale;
     a.stale_idx = g->stale_idx;
     a.nstale = g->nstale;
