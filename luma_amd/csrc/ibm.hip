@@ -634,8 +634,6 @@ int upload(lumagpu_grid *g) {
         q.off = total;
         total += (q.bytes + 255) & ~size_t(255);
     }
-    if (!s->pack_ev && hipEventCreateWithFlags(&s->pack_ev, hipEventDisableTiming) != hipSuccess)
-        return fail(LUMAGPU_EHIP, "IB staging event creation failed");
     if (total > s->pack_cap) {
         // kernels still queued may read the old arena
         HIP_TRY(hipStreamSynchronize(g->stream));
@@ -647,16 +645,17 @@ int upload(lumagpu_grid *g) {
         if (hipMalloc(&s->d_pack, cap) != hipSuccess || hipHostMalloc(&s->h_pack, cap, hipHostMallocDefault) != hipSuccess)
             return fail(LUMAGPU_ENOMEM, "IB buffer allocation failed");
         s->pack_cap = cap;
-    } else {
-        // the previous copy out of the staging buffer has finished
-        HIP_TRY(hipEventSynchronize(s->pack_ev));
+    } else if (s->pack_busy) {
+        // the previous copy out of the staging buffer has finished.  In an FSI sub-iteration the wait
+        // for the marker forces came after it: nothing to record or wait for here
+        HIP_TRY(hipStreamSynchronize(g->stream));
     }
     for (const Part &q : parts) {
         if (q.bytes) std::memcpy(static_cast<char *>(s->h_pack) + q.off, q.src, q.bytes);
         *q.dev = static_cast<char *>(s->d_pack) + q.off;
     }
     if (total) HIP_TRY(hipMemcpyAsync(s->d_pack, s->h_pack, total, hipMemcpyHostToDevice, g->stream));
-    HIP_TRY(hipEventRecord(s->pack_ev, g->stream));
+    s->pack_busy = 1;
     int r = 0;
     size_t *c = s->cap;
     if ((r = dev_resize(&s->d_interp, c + 9, (size_t)nm * 4 * w, g->stream)) ||
@@ -893,6 +892,7 @@ int move_bodies_tangent(lumagpu_grid *g) {
     std::vector<Dual> force((size_t)s->nm * 3);
     HIP_TRY(hipMemcpyAsync(force.data(), s->d_force, force.size() * sizeof(Dual), hipMemcpyDeviceToHost, g->stream));
     HIP_TRY(hipStreamSynchronize(g->stream));
+    s->pack_busy = 0;
     const FemBeamT<Dual>::Solver solver = [](int n, std::vector<Dual> &a, std::vector<Dual> &x) {
         return lu_solve_band(n, FemBeamT<Dual>::kBand, FemBeamT<Dual>::kBand, a, x);
     };
@@ -949,6 +949,7 @@ int move_bodies(lumagpu_grid *g) {
     }
     HIP_TRY(hipMemcpyAsync(s->h_force, s->d_force, nf * sizeof(double), hipMemcpyDeviceToHost, g->stream));
     HIP_TRY(hipStreamSynchronize(g->stream));
+    s->pack_busy = 0;
     const double *force = s->h_force;
     const FemBeam::Solver solver = [](int n, std::vector<double> &a, std::vector<double> &x) {
         return lu_solve_band(n, FemBeam::kBand, FemBeam::kBand, a, x);

@@ -72,7 +72,7 @@ struct IbmSystem {
     double *d_sdelta = nullptr, *d_vel = nullptr, *d_eps = nullptr, *d_ds = nullptr;
     void *d_pack = nullptr, *h_pack = nullptr;
     size_t pack_cap = 0;        // bytes of d_pack and h_pack
-    hipEvent_t pack_ev = nullptr;   // recorded after the last copy out of h_pack
+    int pack_busy = 0;          // a copy out of h_pack may be running: no stream wait since it was queued
     double *d_interp = nullptr, *d_force = nullptr, *d_out = nullptr;
     size_t cap[11] = {};        // element counts of d_interp (9) and d_force (10)
     double *h_force = nullptr;  // pinned download buffer of the marker forces
@@ -97,7 +97,6 @@ struct IbmSystem {
             if (p) (void)hipFree(p);
         for (void *p : {h_pack, (void *)h_force, (void *)h_gone})
             if (p) (void)hipHostFree(p);
-        if (pack_ev) (void)hipEventDestroy(pack_ev);
     }
 };
 
