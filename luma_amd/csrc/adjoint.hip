@@ -4,12 +4,13 @@
 //
 // Forward: T steps of the ordinary step (lumagpu_step semantics), the population array copied
 // to a checkpoint every K steps and the objective accumulated on the device.  Backward: for
-// each segment, newest first, the segment's K states are recomputed from its checkpoint and
-// kept in HBM; then every step of the segment is reversed from its stored input state (the
-// outlet side buffer and the IB forces are recomputed from that state, then the adjoint
-// kernels of adjoint_kernels.hpp run).  The marker-position gradient adds, on the host, the
-// dependence of epsilon (the RKPM system A eps = 1, ObjectManager_ops_ibm.cpp:773-920) and of
-// ds (nearest-marker spacing, :927-981) on the positions.
+// each segment, newest first, the segment's K states run from its checkpoint along a tape in
+// HBM, each step writing its successor there (the last segment in the forward run already); then
+// every step of the segment is reversed from its stored input state (the IB forces are recomputed
+// from it, the outlet side buffer is on the tape, then the adjoint kernels of
+// adjoint_kernels.hpp run).  The marker-position gradient adds the dependence of epsilon (the RKPM
+// system A eps = 1, ObjectManager_ops_ibm.cpp:773-920) and of ds (nearest-marker spacing,
+// :927-981) on the positions.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

@@ -34,6 +34,7 @@ CASES = {
     "walls": _walls,
     "sphere": _sphere,
     "corners": lambda: setups.velocity_corner_box(84, 80, 79, dims=3),
+    "ramp": lambda: setups.uniform_inflow_3d(121, 70, 66, 0.03, 0.6),
     "pressure": lambda: setups.pressure_outlet_duct(90, 80, 75, dims=3),
 }
 
@@ -43,6 +44,8 @@ def _grid(name, case):
     if name == "sphere":
         g.ibm_add_body(setups.sphere_markers((40.3, 35.1, 33.2), 6.0, 1.0))
         g.ibm_initialise()
+    if name == "ramp":
+        g.set_velocity_ramp(21.0)   # ends within the third run
     return g
 
 
