@@ -292,6 +292,8 @@ hipError_t launch_extrap(const lumagpu_grid *g) {
 // holding IB bodies (:53-57).  Sweep 1's stream, BC and macro happen in the step kernel, which
 // end_step launches; what the IB step reads of sweep 1 is recomputed at its supports.
 int begin_step(lumagpu_grid *g) {
+    if (g->masked && !g->sites_ok)
+        return fail(LUMAGPU_ESTATE, "the grid's labels or force were not set to the end: set them again");
     // the outlet side buffer reads this grid's own populations only (the children read them
     // too, but nobody writes them before this grid's step): it runs while the children step
     // the previous step wrote this step's outlet sources unless the state changed since
@@ -469,7 +471,7 @@ int run_fused_graph(lumagpu_grid *g, int reps) {
 bool multi_ok(const lumagpu_grid *g) {
     return !g->fuse_off && g->Q == 9 && (g->d.precision == LUMAGPU_FP64 || g->d.precision == LUMAGPU_FP32S) && !g->parent &&
            g->kids.empty() && ibm_marker_count(g) == 0 && !g->gravity_on && !(g->ramp_time > 0.0) &&
-           !(g->re_ramp > 0.0) && g->nedge == 0 && g->simple_types && g->ncell <= (size_t(1) << 18) && g->has_state;
+           !(g->re_ramp > 0.0) && g->nedge == 0 && g->simple_types && g->ncell <= (size_t(1) << 18) && g->has_state && (!g->masked || g->sites_ok);
 }
 
 // up to n steps from the post-local layout, as many as whole launches take; *done: steps run
@@ -480,7 +482,11 @@ int run_multi(lumagpu_grid *g, int n, int *done) {
     g->all_forced = g->sweep1_zero = 0;
     while (n - *done >= 2) {
         const int H = plan_multi2d(g->d.N, g->d.M, n - *done, g->d.precision == LUMAGPU_FP64);
-        const StepArgs a = make_args(g);
+        StepArgs a = make_args(g);
+        if (!g->masked) {   // flag bytes that other calls made are not this step's
+            a.flags = nullptr;
+            a.link = nullptr;
+        }
         const hipError_t e = g->d.precision == LUMAGPU_FP64 ? launch_multi2d_f64(a, g->f2, H, g->store_macro, g->stream)
                                                             : launch_multi2d_f32s(a, g->f2, H, g->store_macro, g->stream);
         if (e != hipSuccess) return fail(LUMAGPU_EHIP, std::string("multi-step launch: ") + hipGetErrorString(e));
@@ -504,7 +510,7 @@ bool pair_ok(const lumagpu_grid *g) {
         g->ps * g->elem >= (size_t(1) << 32))
         return false;
     if (g->has_outlet && !g->xr_fold) return false;
-    if (g->masked && !g->pair_types) return false;
+    if (g->masked && (!g->pair_types || !g->sites_ok)) return false;
     return !ibm_has_flexible(g) && !(g->host_forced && ibm_marker_count(g) > 0);
 }
 
@@ -808,7 +814,7 @@ int capture_stale(lumagpu_grid *g) {
 
 // refined sites read by a site that does not coalesce (anything but TL2F, solid or refined),
 // with the periodic wrap of the step kernels
-static int build_stale(lumagpu_grid *g) {
+static int build_stale(lumagpu_grid *g, bool *fresh) {
     const int N = g->d.N, M = g->d.M, K = g->d.K;
     auto ty = [&](int i, int j, int k) {
         i = (i + N) % N; j = (j + M) % M; k = (k + K) % K;
@@ -840,9 +846,9 @@ static int build_stale(lumagpu_grid *g) {
                             }
                         }
             }
-    // the same sites as before (a flag upload that changed only force bits): keep what was captured
-    if (cells == g->stale_list) return 0;
-    g->stale_list = cells;
+    // the same sites as before: keep what was captured
+    *fresh = cells != g->stale_list;
+    if (!*fresh) return 0;
     (void)hipStreamSynchronize(g->stream);
     (void)hipFree(g->stale);
     (void)hipFree(g->stale_idx);
@@ -850,6 +856,7 @@ static int build_stale(lumagpu_grid *g) {
     g->stale = nullptr;
     g->stale_idx = g->stale_cells = nullptr;
     g->nstale = 0;
+    g->stale_list.clear();
     if (cells.empty()) return 0;
     if (hipMalloc(&g->stale, (size_t)g->Q * cells.size() * g->elem) != hipSuccess ||
         hipMalloc(&g->stale_idx, g->ncell * sizeof(int)) != hipSuccess ||
@@ -858,7 +865,8 @@ static int build_stale(lumagpu_grid *g) {
     HIP_TRY(hipMemcpy(g->stale_idx, idx.data(), g->ncell * sizeof(int), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(g->stale_cells, cells.data(), cells.size() * sizeof(int), hipMemcpyHostToDevice));
     g->nstale = (int)cells.size();
-    return capture_stale(g);
+    g->stale_list = std::move(cells);
+    return 0;
 }
 
 // Large labelled grids step in two launches: k_aa_plain over the grid for the plain sites
@@ -866,26 +874,21 @@ static int build_stale(lumagpu_grid *g) {
 // kernel over the list of the other sites it steps.  Small grids, whose steps are launch-bound,
 // keep one launch.
 constexpr size_t kSplitMinCells = size_t(1) << 20;
+static bool split_sites(const lumagpu_grid *g) { return g->ncell >= kSplitMinCells && !g->zslab; }
 static int build_mlist(lumagpu_grid *g) {
-    if (g->ncell < kSplitMinCells || g->zslab) {
-        g->nmlist = -1;
-        return 0;
-    }
-    std::vector<uint8_t> types(g->ncell);
-    for (size_t c = 0; c < g->ncell; ++c) types[c] = g->hflags[c] & kTypeMask;
-    if (types == g->mlist_types && g->nmlist >= 0) return 0;   // only force bits changed
+    if (!split_sites(g)) return 0;
     const int N = g->d.N, M = g->d.M, K = g->d.K;
     auto ty = [&](int i, int j, int k) {
         i = (i + N) % N; j = (j + M) % M; k = (k + K) % K;
-        return (int)types[(size_t)i + (size_t)N * ((size_t)j + (size_t)M * k)];
+        return g->hflags[(size_t)i + (size_t)N * ((size_t)j + (size_t)M * k)] & kTypeMask;
     };
     std::vector<int> list;
     for (int k = 0; k < K; ++k)
         for (int j = 0; j < M; ++j)
             for (int i = 0; i < N; ++i) {
                 const size_t c = (size_t)i + (size_t)N * ((size_t)j + (size_t)M * k);
-                const int t = types[c];
                 const unsigned fl = g->hflags[c];
+                const int t = fl & kTypeMask;
                 // the sites k_aa_masked leaves alone
                 if (t == kSolid || t == kRefined || (!g->d.regularised && t == kVelocity)) continue;
                 if (t == kPressure || (t == kVelocity && ((fl >> kNormalShift) & 7) == kNormalEdge)) continue;
@@ -899,45 +902,69 @@ static int build_mlist(lumagpu_grid *g) {
                         }
                 if (!plain) list.push_back((int)c);
             }
-    (void)hipStreamSynchronize(g->stream);
-    (void)hipFree(g->mlist);
-    g->mlist = nullptr;
-    g->nmlist = -1;
-    g->mlist_types.clear();
     if (!list.empty()) {
         if (hipMalloc(&g->mlist, list.size() * sizeof(int)) != hipSuccess)
             return fail(LUMAGPU_ENOMEM, "site list allocation failed");
         HIP_TRY(hipMemcpy(g->mlist, list.data(), list.size() * sizeof(int), hipMemcpyHostToDevice));
     }
     g->nmlist = (int)list.size();
-    g->mlist_types = std::move(types);
     return 0;
 }
 
 // link words of the sites k_aa_masked or k_aa_masked_list steps, from the flags on the device
 static int build_links(lumagpu_grid *g) {
+    const size_t n = g->nmlist >= 0 ? (size_t)g->nmlist : g->ncell;
+    if (n == 0) return 0;
+    if (hipMalloc(&g->link, n * sizeof(uint64_t)) != hipSuccess) {
+        g->link = nullptr;
+        return fail(LUMAGPU_ENOMEM, "link word allocation failed");
+    }
+    const unsigned nb = (unsigned)((n + 255) / 256);
+    const int *cells = g->nmlist >= 0 ? g->mlist : nullptr;
+    if (g->Q == 9)
+        k_links<9><<<nb, 256, 0, g->stream>>>(g->flags, g->d.N, g->d.M, g->d.K, g->d.regularised, cells, n, g->link);
+    else
+        k_links<19><<<nb, 256, 0, g->stream>>>(g->flags, g->d.N, g->d.M, g->d.K, g->d.regularised, cells, n, g->link);
+    HIP_TRY(hipGetLastError());
+    return 0;
+}
+
+// The site list, its link words and the captured refined sites, from the flag bytes without the force
+// bit and from which of the two layouts the grid steps in (one link word per cell, or per entry of
+// the list).  Kept while both are the same.  sites_ok is 0 from here on until all of it is there:
+// a step would read a list of one state with the link words of another, so it is refused meanwhile.
+static int build_sites(lumagpu_grid *g, bool had) {
     std::vector<uint8_t> types(g->ncell);
     for (size_t c = 0; c < g->ncell; ++c) types[c] = g->hflags[c] & ~kForcedBit;
-    if (g->link && types == g->link_types) return 0;   // only force bits changed
-    const size_t n = g->nmlist >= 0 ? (size_t)g->nmlist : g->ncell;
-    (void)hipStreamSynchronize(g->stream);
-    (void)hipFree(g->link);
-    g->link = nullptr;
-    g->link_types.clear();
-    if (n > 0) {
-        if (hipMalloc(&g->link, n * sizeof(uint64_t)) != hipSuccess) {
-            g->link = nullptr;
-            return fail(LUMAGPU_ENOMEM, "link word allocation failed");
-        }
-        const unsigned nb = (unsigned)((n + 255) / 256);
-        const int *cells = g->nmlist >= 0 ? g->mlist : nullptr;
-        if (g->Q == 9)
-            k_links<9><<<nb, 256, 0, g->stream>>>(g->flags, g->d.N, g->d.M, g->d.K, g->d.regularised, cells, n, g->link);
-        else
-            k_links<19><<<nb, 256, 0, g->stream>>>(g->flags, g->d.N, g->d.M, g->d.K, g->d.regularised, cells, n, g->link);
-        HIP_TRY(hipGetLastError());
+    if (had && types == g->site_types && split_sites(g) == (g->nmlist >= 0)) {
+        g->sites_ok = 1;
+        return 0;
     }
-    g->link_types = std::move(types);
+    (void)hipStreamSynchronize(g->stream);
+    (void)hipFree(g->mlist);
+    (void)hipFree(g->link);
+    g->mlist = nullptr;
+    g->link = nullptr;
+    g->nmlist = -1;
+    if (int r = build_mlist(g)) return r;
+    if (int r = build_links(g)) return r;
+    bool fresh = false;
+    if (int r = build_stale(g, &fresh)) return r;
+    g->site_types = std::move(types);
+    g->sites_ok = 1;
+    return fresh ? capture_stale(g) : 0;
+}
+
+// the device's flag bytes and plain-site bitmap
+static int alloc_flags(lumagpu_grid *g) {
+    if (!g->flags && hipMalloc(&g->flags, g->ncell) != hipSuccess) {
+        g->flags = nullptr;
+        return fail(LUMAGPU_ENOMEM, "flag array allocation failed");
+    }
+    if (!g->plain && hipMalloc(&g->plain, (g->ncell + 31) / 32 * sizeof(uint32_t)) != hipSuccess) {
+        g->plain = nullptr;
+        return fail(LUMAGPU_ENOMEM, "plain-site bitmap allocation failed");
+    }
     return 0;
 }
 
@@ -945,11 +972,12 @@ int upload_flags(lumagpu_grid *g) {
     ++g->flags_version;
     g->pair_synced = 0;
     if (g->hflags.size() != g->ncell) return fail(LUMAGPU_ESTATE, "host flag array does not cover the grid");
-    if (!g->flags && hipMalloc(&g->flags, g->ncell) != hipSuccess)
-        return fail(LUMAGPU_ENOMEM, "flag array allocation failed");
+    if (int r = alloc_flags(g)) return r;
+    // from here until the list and the link words are whole a step would read parts of two states:
+    // begin_step refuses it
+    const bool had = g->sites_ok != 0;
+    g->sites_ok = 0;
     const size_t nw = (g->ncell + 31) / 32;
-    if (!g->plain && hipMalloc(&g->plain, nw * sizeof(uint32_t)) != hipSuccess)
-        return fail(LUMAGPU_ENOMEM, "plain-site bitmap allocation failed");
     HIP_TRY(hipMemcpyAsync(g->flags, g->hflags.data(), g->ncell, hipMemcpyHostToDevice, g->stream));
     g->simple_types = std::all_of(g->hflags.begin(), g->hflags.end(), [](uint8_t f) {
         const int t = f & kTypeMask;
@@ -964,9 +992,7 @@ int upload_flags(lumagpu_grid *g) {
     if (g->Q == 9) k_plain_bits<9><<<nb, 256, 0, g->stream>>>(g->flags, g->d.N, g->d.M, g->d.K, g->ncell, g->plain);
     else k_plain_bits<19><<<nb, 256, 0, g->stream>>>(g->flags, g->d.N, g->d.M, g->d.K, g->ncell, g->plain);
     HIP_TRY(hipGetLastError());
-    if (int r = build_mlist(g)) return r;
-    if (int r = build_links(g)) return r;
-    return build_stale(g);
+    return build_sites(g, had);
 }
 hipError_t outlet_prepass(const lumagpu_grid *g) { return launch_extrap(g); }
 }  // namespace lumagpu
@@ -1202,32 +1228,35 @@ int lumagpu_set_labels(lumagpu_grid *g, const int *lattyp, const double *xpos, c
         etab[2 * ne + e] = nb[0];
         etab[3 * ne + e] = nb[1];
     }
-    (void)hipFree(g->edge);
-    (void)hipFree(g->erho);
-    g->edge = nullptr;
-    g->erho = nullptr;
-    g->nedge = 0;
-    if (ne) {
-        if (hipMalloc(&g->edge, etab.size() * sizeof(int)) != hipSuccess ||
-            hipMalloc(&g->erho, 8 * (size_t)ne * g->melem) != hipSuccess)
-            return fail(LUMAGPU_ENOMEM, "edge site table allocation failed");
-        HIP_TRY(hipMemcpyAsync(g->edge, etab.data(), etab.size() * sizeof(int), hipMemcpyHostToDevice, g->stream));
-        g->nedge = ne;
-    }
-    g->hflags = std::move(nf);
-    if (int r = upload_flags(g)) return r;
-    if (outlet && !g->xr &&
-        hipMalloc(&g->xr, 2 * (size_t)g->Q * g->d.M * g->d.K * g->melem) != hipSuccess)
+    // the allocations before the first change: short of memory here, the grid stays as it was
+    struct Freed {
+        void *p = nullptr;
+        ~Freed() { (void)hipFree(p); }
+    } edge, erho;
+    if (ne && (hipMalloc(&edge.p, etab.size() * sizeof(int)) != hipSuccess ||
+               hipMalloc(&erho.p, 8 * (size_t)ne * g->melem) != hipSuccess))
+        return fail(LUMAGPU_ENOMEM, "edge site table allocation failed");
+    if (outlet && !g->xr && hipMalloc(&g->xr, 2 * (size_t)g->Q * g->d.M * g->d.K * g->melem) != hipSuccess) {
+        g->xr = nullptr;
         return fail(LUMAGPU_ENOMEM, "outlet buffer allocation failed");
-    HIP_TRY(hipStreamSynchronize(g->stream));
+    }
+    if (int r = alloc_flags(g)) return r;
+    if (ne) HIP_TRY(hipMemcpyAsync(edge.p, etab.data(), etab.size() * sizeof(int), hipMemcpyHostToDevice, g->stream));
+    // the old tables are freed on the way out
+    void *const old_edge = g->edge, *const old_erho = g->erho;
+    g->edge = static_cast<int *>(edge.p);
+    g->erho = static_cast<double *>(erho.p);
+    edge.p = old_edge;
+    erho.p = old_erho;
+    g->nedge = ne;
+    g->hflags = std::move(nf);
     g->has_outlet = outlet;
     // the step kernels can write the next step's outlet sources when every outlet row's source
     // two cells left is a site they step (collided, or streamed only for TL2C)
     g->xr_fold = 0;
     g->xr_ready = 0;
-    if (outlet && g->d.N >= 3) {
+    if (outlet) {
         bool ok = true;
-        const int N = g->d.N, M = g->d.M, K = g->d.K;
         for (int k = 0; k < K && ok; ++k)
             for (int j = 0; j < M && ok; ++j) {
                 const size_t row = (size_t)N * ((size_t)j + (size_t)M * k);
@@ -1241,6 +1270,8 @@ int lumagpu_set_labels(lumagpu_grid *g, const int *lattyp, const double *xpos, c
         g->xr_fold = ok ? 1 : 0;
     }
     g->masked = any || g->d.forced;
+    if (int r = upload_flags(g)) return r;
+    HIP_TRY(hipStreamSynchronize(g->stream));
     return 0;
 }
 

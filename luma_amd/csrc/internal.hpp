@@ -59,9 +59,9 @@ struct lumagpu_grid {
     int *mlist = nullptr;
     // link words (k_links): of the listed sites, or of every cell of a grid stepped in one launch
     uint64_t *link = nullptr;
-    std::vector<uint8_t> link_types;  // the flag bytes (without the force bit) they were built from
     int nmlist = -1;                  // < 0: one labelled launch over the grid
-    std::vector<uint8_t> mlist_types; // the site types mlist was built from
+    std::vector<uint8_t> site_types;  // the flag bytes (without the force bit) list and words were built from
+    int sites_ok = 0;                 // they are whole: a labelled grid steps only then
     // the captured two-step graph of this hierarchy (root grids), reused while its key holds
     int ib_fold = 0;                  // the step kernel does this step's IB spread
     hipGraphExec_t gexec = nullptr;

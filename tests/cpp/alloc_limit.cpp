@@ -1,0 +1,113 @@
+// A stand-in for the allocation calls of the HIP runtime that libluma_amd.so makes, loaded before it
+// with RTLD_GLOBAL: each goes on to the runtime's own unless a limit set here refuses it.  So a test
+// can run the library short of device memory without filling the device.
+#include <dlfcn.h>
+
+#include <cstddef>
+#include <cstdio>
+#include <cstdlib>
+#include <map>
+#include <mutex>
+#include <thread>
+
+namespace {
+constexpr int kOutOfMemory = 2;   // hipErrorOutOfMemory
+std::mutex mu;
+std::map<void *, size_t> live;
+long long budget = -1;            // bytes that may still be allocated; < 0: no limit
+size_t refused_size = 0;          // allocations of exactly this many bytes fail
+size_t total_shown = 0;           // what hipMemGetInfo reports as the device's memory (0: the truth)
+int device_shown = -1;            // what hipGetDevice reports (< 0: the truth)
+size_t held = 0;
+int calls = 0, refusals = 0;
+std::thread::id watched;
+int watched_set_device = 0;
+
+void *runtime() {
+    static void *h = dlopen("libamdhip64.so.7", RTLD_NOW | RTLD_LOCAL);
+    if (!h) {
+        std::fprintf(stderr, "alloc_limit: %s\n", dlerror());
+        std::abort();
+    }
+    return h;
+}
+template <class F>
+F *own(const char *name) {
+    void *p = dlsym(runtime(), name);
+    if (!p) std::abort();
+    return reinterpret_cast<F *>(p);
+}
+}  // namespace
+
+extern "C" {
+int hipMalloc(void **p, size_t n) {
+    static auto *f = own<int(void **, size_t)>("hipMalloc");
+    std::lock_guard<std::mutex> lock(mu);
+    ++calls;
+    if ((budget >= 0 && n > (size_t)budget) || (refused_size && n == refused_size)) {
+        ++refusals;
+        return kOutOfMemory;
+    }
+    const int e = f(p, n);
+    if (e == 0) {
+        live[*p] = n;
+        held += n;
+        if (budget >= 0) budget -= (long long)n;
+    }
+    return e;
+}
+int hipFree(void *p) {
+    static auto *f = own<int(void *)>("hipFree");
+    std::lock_guard<std::mutex> lock(mu);
+    const auto it = live.find(p);
+    if (it != live.end()) {
+        held -= it->second;
+        if (budget >= 0) budget += (long long)it->second;
+        live.erase(it);
+    }
+    return f(p);
+}
+int hipMemGetInfo(size_t *avail, size_t *total) {
+    static auto *f = own<int(size_t *, size_t *)>("hipMemGetInfo");
+    const int e = f(avail, total);
+    std::lock_guard<std::mutex> lock(mu);
+    if (budget >= 0 && *avail > (size_t)budget) *avail = (size_t)budget;
+    if (total_shown) *total = total_shown;
+    return e;
+}
+int hipGetDevice(int *d) {
+    static auto *f = own<int(int *)>("hipGetDevice");
+    const int e = f(d);
+    if (device_shown >= 0) *d = device_shown;
+    return e;
+}
+int hipSetDevice(int d) {
+    static auto *f = own<int(int)>("hipSetDevice");
+    std::lock_guard<std::mutex> lock(mu);
+    if (std::this_thread::get_id() == watched) ++watched_set_device;
+    return f(d);
+}
+
+void limit_budget(long long bytes) {
+    std::lock_guard<std::mutex> lock(mu);
+    budget = bytes;
+}
+void limit_refuse_size(size_t bytes) {
+    std::lock_guard<std::mutex> lock(mu);
+    refused_size = bytes;
+}
+void limit_show_total(size_t bytes) {
+    std::lock_guard<std::mutex> lock(mu);
+    total_shown = bytes;
+}
+void limit_show_device(int d) { device_shown = d; }
+void limit_watch_this_thread() {
+    std::lock_guard<std::mutex> lock(mu);
+    watched = std::this_thread::get_id();
+    watched_set_device = 0;
+}
+int limit_set_device_calls() { return watched_set_device; }
+size_t limit_held() { return held; }
+int limit_calls() { return calls; }
+int limit_refusals() { return refusals; }
+}

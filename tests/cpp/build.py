@@ -1,5 +1,6 @@
-"""Builds the C++ facade driver (facade_run.cpp) against libluma_amd.so with g++, into
-tests/cpp/_build/.  Called by __graft_entry__.build() after the library."""
+"""Builds the C++ facade driver (facade_run.cpp) against libluma_amd.so and the allocation limiter of
+the memory tests (alloc_limit.cpp) with g++, into tests/cpp/_build/.  Called by
+__graft_entry__.build() after the library."""
 from __future__ import annotations
 
 import subprocess
@@ -9,6 +10,7 @@ from pathlib import Path
 HERE = Path(__file__).resolve().parent
 ROOT = HERE.parents[1]
 OUT = HERE / "_build" / "facade_run"
+LIMIT = HERE / "_build" / "alloc_limit.so"
 
 
 def build_driver(verbose: bool = False) -> Path:
@@ -19,6 +21,8 @@ def build_driver(verbose: bool = False) -> Path:
     if verbose:
         print(" ".join(cmd), flush=True)
     subprocess.run(cmd, check=True)
+    subprocess.run(["g++", "-std=c++17", "-O2", "-Wall", "-shared", "-fPIC", str(HERE / "alloc_limit.cpp"), "-ldl",
+                    "-o", str(LIMIT)], check=True)
     return OUT
 
 

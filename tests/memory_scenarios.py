@@ -1,0 +1,84 @@
+"""Programs that run the library short of device memory, one per name, each in a process of its own
+(test_gpu_memory.py): the limiter has to be loaded before the library.  A scenario raises where it
+fails and prints its name at the end."""
+import ctypes as C
+import sys
+from pathlib import Path
+
+import numpy as np
+
+HERE = Path(__file__).resolve().parent
+sys.path.insert(0, str(HERE.parent))
+limit = C.CDLL(str(HERE / "cpp" / "_build" / "alloc_limit.so"), mode=C.RTLD_GLOBAL)
+limit.limit_budget.argtypes = [C.c_longlong]
+limit.limit_refuse_size.argtypes = [C.c_size_t]
+limit.limit_show_total.argtypes = [C.c_size_t]
+limit.limit_held.restype = C.c_size_t
+
+from luma_amd import setups  # noqa: E402
+from luma_amd._abi import LumaGpuError  # noqa: E402
+from luma_amd.grid import GpuGrid  # noqa: E402
+
+MB = 1 << 20
+
+
+def walls(n=70):
+    """FP32-shifted labelled box of n^3 cells with a set force: run() takes two steps per launch."""
+    case = setups.body_force_channel(n, n, n, 3, g=1e-5)
+    case.u[..., 0] = 0.02 * np.sin(np.arange(n))[None, :, None]
+    case.u[case.lattyp == setups.SOLID] = 0.0
+    return case
+
+
+def grid(case, form="fp32s"):
+    return GpuGrid.from_case(case, form, store_macro=True)
+
+
+def state(g):
+    return (g.download_f(),) + g.download_macro()
+
+
+def single_steps(case, n, form="fp32s"):
+    with grid(case, form) as g:
+        for _ in range(n):
+            g.LBM_multi_opt()
+        return state(g)
+
+
+def same(a, b):
+    assert all(np.array_equal(x, y) for x, y in zip(a, b))
+
+
+def labels_cut_short():
+    # the link words of the new labels do not fit: the call fails and steps are refused, until the
+    # labels have been set; nothing reads a part of them
+    case = setups.lid_driven_cavity(40, re=200.0)
+    lt = case.lattyp.copy()
+    lt[10:15, 12:20] = setups.SOLID
+    with grid(case) as g, grid(case) as h:
+        g.run(4)
+        h.run(4)
+        limit.limit_refuse_size(8 * 40 * 40)
+        try:
+            g.set_labels(lt, case.xpos, case.ypos, case.zpos)
+            raise AssertionError("link words allocated")
+        except LumaGpuError as e:
+            assert "allocation" in str(e)
+        for step in (lambda: g.run(6), lambda: g.run(1), g.LBM_multi_opt, g.stream_bc_macro):
+            try:
+                step()
+                raise AssertionError("stepped")
+            except LumaGpuError as e:
+                assert "set them again" in str(e)
+        limit.limit_refuse_size(0)
+        for x in (g, h):
+            x.set_labels(lt, case.xpos, case.ypos, case.zpos)
+            x.run(6)
+        same(state(g), state(h))
+
+
+if __name__ == "__main__":
+    print(f"[memory] {sys.argv[1]}", flush=True)
+    globals()[sys.argv[1]]()
+    assert limit.limit_calls() > 0, "the library's allocations do not come through the limiter"
+    print(f"done {sys.argv[1]}", flush=True)
