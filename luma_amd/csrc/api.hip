@@ -514,9 +514,11 @@ bool pair_ok(const lumagpu_grid *g) {
     return !ibm_has_flexible(g) && !(g->host_forced && ibm_marker_count(g) > 0);
 }
 
-// the deep cells and the lists around them, from the flags on the device
+// the deep cells and the lists around them, from the flags on the device; LUMAGPU_ENOMEM where they do
+// not fit
 int pair_sets(lumagpu_grid *g) {
     if (!g->masked || g->pair_version == g->flags_version) return 0;
+    g->pair_version = 0;
     const size_t nw = (g->ncell + 31) / 32 + 1;   // a whole pair of words at the end
     struct Buf {
         uint32_t *p = nullptr;
@@ -602,7 +604,11 @@ int pair_half(lumagpu_grid *g, bool odd, PairPlan plan) {
 int run_pairs(lumagpu_grid *g, int n, int *done) {
     *done = 0;
     if (!f2_ensure(g)) return 0;
-    if (int r = pair_sets(g)) return r;
+    if (const int r = pair_sets(g)) {
+        if (r != LUMAGPU_ENOMEM) return r;
+        (void)hipGetLastError();
+        return 0;   // single steps need no sets
+    }
     if (g->masked && !g->pair_synced)
         HIP_TRY(hipMemcpyAsync(g->f2, g->f, g->ps * g->Q * g->elem, hipMemcpyDeviceToDevice, g->stream));
     g->pair_synced = 1;

@@ -77,6 +77,20 @@ def labels_cut_short():
         same(state(g), state(h))
 
 
+def sets_do_not_fit():
+    # two steps per launch need bitmaps and lists of sites; single steps do not
+    case = walls()
+    words = (70 ** 3 + 31) // 32 + 1
+    with grid(case) as g:
+        limit.limit_refuse_size(4 * words)
+        g.run(9)
+        assert limit.limit_refusals() > 0
+        same(state(g), single_steps(case, 9))
+        limit.limit_refuse_size(0)
+        g.run(9)
+        same(state(g), single_steps(case, 18))
+
+
 if __name__ == "__main__":
     print(f"[memory] {sys.argv[1]}", flush=True)
     globals()[sys.argv[1]]()
