@@ -59,7 +59,8 @@ hipError_t launch_aux(const lumagpu_grid *g, int op, const double *p0, const dou
 std::mutex g_f2_grids_mu;
 std::vector<lumagpu_grid *> g_f2_grids;
 
-// the arrays of grids that no run holds, back to the device
+// the arrays of grids that no run holds, back to the device.  f2_mu is recursive: on the thread of a run
+// its own grid's lock is no obstacle, and f2_busy says that its second array is in use.
 void f2_give_back() {
     std::lock_guard<std::mutex> lock(g_f2_grids_mu);
     for (size_t k = 0; k < g_f2_grids.size();) {
@@ -69,11 +70,14 @@ void f2_give_back() {
             continue;
         }
         if (o->stream) (void)hipStreamSynchronize(o->stream);
-        if (o->f2_auto) {
-            (void)hipFree(o->f2);
-            o->f2 = nullptr;
+        const bool busy = o->f2_busy != 0;
+        if (!busy) {
+            if (o->f2_auto) {
+                (void)hipFree(o->f2);
+                o->f2 = nullptr;
+            }
+            o->f2_auto = o->pair_synced = 0;
         }
-        o->f2_auto = o->pair_synced = 0;
         std::vector<lumagpu_grid::Block> kept;
         for (auto &b : o->blocks) {
             if (b.used) kept.push_back(b);
@@ -81,7 +85,8 @@ void f2_give_back() {
         }
         o->blocks = std::move(kept);
         o->f2_mu.unlock();
-        g_f2_grids.erase(g_f2_grids.begin() + k);
+        if (busy) ++k;
+        else g_f2_grids.erase(g_f2_grids.begin() + k);
     }
 }
 
@@ -98,6 +103,15 @@ void scratch_listed(lumagpu_grid *g) {
 }
 }  // namespace lumagpu
 namespace {
+
+// the second array is being stepped from or into: no allocation meanwhile takes it back
+struct F2Use {
+    lumagpu_grid *g;
+    explicit F2Use(lumagpu_grid *grid) : g(grid) { ++g->f2_busy; }
+    F2Use(const F2Use &) = delete;
+    F2Use &operator=(const F2Use &) = delete;
+    ~F2Use() { --g->f2_busy; }
+};
 
 // with g->f2_mu held: true when g->f2 is there
 bool f2_ensure(lumagpu_grid *g) {
@@ -123,7 +137,7 @@ int ensure_stage(lumagpu_grid *g, size_t bytes) {
         g->stage = nullptr;
         g->stage_bytes = 0;
     }
-    if (dev_malloc((void **)&g->stage, bytes) != hipSuccess) return fail(LUMAGPU_ENOMEM, "staging allocation failed");
+    if (dev_malloc(&g->stage, bytes) != hipSuccess) return fail(LUMAGPU_ENOMEM, "staging allocation failed");
     g->stage_bytes = bytes;
     return 0;
 }
@@ -187,10 +201,11 @@ hipError_t launch_zslab(const lumagpu_grid *g, const StepArgs &a, int phase) {
 namespace lumagpu {
 hipError_t dev_malloc(void **p, size_t bytes) {
     hipError_t e = hipMalloc(p, bytes);
-    if (e != hipErrorOutOfMemory) return e;
-    (void)hipGetLastError();
-    f2_give_back();
-    e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        f2_give_back();
+        e = hipMalloc(p, bytes);
+    }
     if (e != hipSuccess) *p = nullptr;
     return e;
 }
@@ -478,6 +493,7 @@ bool multi_ok(const lumagpu_grid *g) {
 int run_multi(lumagpu_grid *g, int n, int *done) {
     *done = 0;
     if (!f2_ensure(g)) return 0;   // one step per launch needs no second array
+    const F2Use use(g);
     // begin_step's state for a grid without bodies
     g->all_forced = g->sweep1_zero = 0;
     while (n - *done >= 2) {
@@ -524,8 +540,8 @@ int pair_sets(lumagpu_grid *g) {
         uint32_t *p = nullptr;
         ~Buf() { (void)hipFree(p); }
     } rest, near;
-    if ((!g->pair_deep && hipMalloc(&g->pair_deep, nw * 4) != hipSuccess) || hipMalloc(&rest.p, nw * 4) != hipSuccess ||
-        hipMalloc(&near.p, nw * 4) != hipSuccess)
+    if ((!g->pair_deep && dev_malloc(&g->pair_deep, nw * 4) != hipSuccess) ||
+        dev_malloc(&rest.p, nw * 4) != hipSuccess || dev_malloc(&near.p, nw * 4) != hipSuccess)
         return fail(LUMAGPU_ENOMEM, "site set allocation failed");
     const StepArgs a = make_args(g);
     const unsigned nb = (unsigned)((g->ncell + 255) / 256);
@@ -551,8 +567,8 @@ int pair_sets(lumagpu_grid *g) {
     g->pair_cells = nullptr;
     g->pair_links = nullptr;
     if (!cells.empty()) {
-        if (hipMalloc(&g->pair_cells, cells.size() * sizeof(int)) != hipSuccess ||
-            hipMalloc(&g->pair_links, cells.size() * sizeof(uint64_t)) != hipSuccess)
+        if (dev_malloc(&g->pair_cells, cells.size() * sizeof(int)) != hipSuccess ||
+            dev_malloc(&g->pair_links, cells.size() * sizeof(uint64_t)) != hipSuccess)
             return fail(LUMAGPU_ENOMEM, "site list allocation failed");
         HIP_TRY(hipMemcpyAsync(g->pair_cells, cells.data(), cells.size() * sizeof(int), hipMemcpyHostToDevice, g->stream));
         k_links<19><<<(unsigned)((cells.size() + 255) / 256), 256, 0, g->stream>>>(
@@ -604,6 +620,7 @@ int pair_half(lumagpu_grid *g, bool odd, PairPlan plan) {
 int run_pairs(lumagpu_grid *g, int n, int *done) {
     *done = 0;
     if (!f2_ensure(g)) return 0;
+    const F2Use use(g);
     if (const int r = pair_sets(g)) {
         if (r != LUMAGPU_ENOMEM) return r;
         (void)hipGetLastError();
@@ -1053,8 +1070,8 @@ int lumagpu_grid_create(const lumagpu_grid_desc *desc, lumagpu_grid **out) {
         return cleanup(LUMAGPU_EHIP, "hipEventCreate failed");
     if (dev_malloc(&g->f, g->ps * g->Q * g->elem) != hipSuccess)
         return cleanup(LUMAGPU_ENOMEM, "population array allocation failed");
-    if (dev_malloc((void **)&g->rho, g->ncell * g->melem) != hipSuccess ||
-        dev_malloc((void **)&g->u, g->ncell * g->D * g->melem) != hipSuccess)
+    if (dev_malloc(&g->rho, g->ncell * g->melem) != hipSuccess ||
+        dev_malloc(&g->u, g->ncell * g->D * g->melem) != hipSuccess)
         return cleanup(LUMAGPU_ENOMEM, "macro array allocation failed");
     if (hipMalloc(&g->uin, 3 * (size_t)d.M * sizeof(double)) != hipSuccess)
         return cleanup(LUMAGPU_ENOMEM, "inlet array allocation failed");
@@ -1066,7 +1083,7 @@ int lumagpu_grid_create(const lumagpu_grid_desc *desc, lumagpu_grid **out) {
         hipMalloc(&g->moments_out, kMomentCount * sizeof(double)) != hipSuccess)
         return cleanup(LUMAGPU_ENOMEM, "reduction buffers allocation failed");
     if (d.forced) {
-        if (dev_malloc((void **)&g->force, g->ncell * g->D * g->melem) != hipSuccess)
+        if (dev_malloc(&g->force, g->ncell * g->D * g->melem) != hipSuccess)
             return cleanup(LUMAGPU_ENOMEM, "force array allocation failed");
         if (hipMemsetAsync(g->force, 0, g->ncell * g->D * g->melem, g->stream) != hipSuccess)
             return cleanup(LUMAGPU_EHIP, "force array clear failed");
@@ -1331,8 +1348,8 @@ int lumagpu_checkpoint_save(lumagpu_grid *g, lumagpu_checkpoint **out) {
     ck->owner = g;
     ck->fbytes = g->ps * g->Q * g->elem;
     if (dev_malloc(&ck->f, ck->fbytes) != hipSuccess ||
-        dev_malloc((void **)&ck->rho, g->ncell * g->melem) != hipSuccess ||
-        dev_malloc((void **)&ck->u, g->ncell * g->D * g->melem) != hipSuccess) {
+        dev_malloc(&ck->rho, g->ncell * g->melem) != hipSuccess ||
+        dev_malloc(&ck->u, g->ncell * g->D * g->melem) != hipSuccess) {
         lumagpu_checkpoint_free(ck);
         return fail(LUMAGPU_ENOMEM, "checkpoint allocation failed");
     }

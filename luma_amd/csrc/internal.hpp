@@ -37,6 +37,7 @@ struct lumagpu_grid {
         int used;
     };
     std::vector<Block> blocks;
+    int f2_busy = 0;                  // a run is using f2 (see F2Use)
     int fuse_off = 0;                 // lumagpu_set_temporal_blocking turned several steps per launch off
     // two steps per launch on a large 3D grid (fused_kernels.hpp): the deep cells, the cells around the
     // others (S1) and the others (S) with their link words
@@ -126,6 +127,13 @@ int fail(int code, const std::string &msg);
 void scratch_listed(lumagpu_grid *g);
 // hipMalloc that, short of memory, first takes back what runs allocated for themselves (api.hip)
 hipError_t dev_malloc(void **p, size_t bytes);
+template <class T>
+hipError_t dev_malloc(T **p, size_t bytes) {
+    void *q = nullptr;
+    const hipError_t e = dev_malloc(&q, bytes);
+    *p = static_cast<T *>(q);
+    return e;
+}
 
 // device memory to the caller's, on g's stream (host_copy.hip); the pinned slots it uses live
 // while any grid does

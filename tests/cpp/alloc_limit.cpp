@@ -16,6 +16,7 @@ std::mutex mu;
 std::map<void *, size_t> live;
 long long budget = -1;            // bytes that may still be allocated; < 0: no limit
 size_t refused_size = 0;          // allocations of exactly this many bytes fail
+bool until_freed = false;         // ... until something of 1 MiB or more has been freed
 size_t total_shown = 0;           // what hipMemGetInfo reports as the device's memory (0: the truth)
 int device_shown = -1;            // what hipGetDevice reports (< 0: the truth)
 size_t held = 0;
@@ -63,6 +64,7 @@ int hipFree(void *p) {
     if (it != live.end()) {
         held -= it->second;
         if (budget >= 0) budget += (long long)it->second;
+        if (until_freed && it->second >= (size_t(1) << 20)) refused_size = 0;
         live.erase(it);
     }
     return f(p);
@@ -95,6 +97,12 @@ void limit_budget(long long bytes) {
 void limit_refuse_size(size_t bytes) {
     std::lock_guard<std::mutex> lock(mu);
     refused_size = bytes;
+    until_freed = false;
+}
+void limit_refuse_until_freed(size_t bytes) {
+    std::lock_guard<std::mutex> lock(mu);
+    refused_size = bytes;
+    until_freed = true;
 }
 void limit_show_total(size_t bytes) {
     std::lock_guard<std::mutex> lock(mu);

@@ -11,7 +11,7 @@ HERE = Path(__file__).resolve().parent
 sys.path.insert(0, str(HERE.parent))
 limit = C.CDLL(str(HERE / "cpp" / "_build" / "alloc_limit.so"), mode=C.RTLD_GLOBAL)
 limit.limit_budget.argtypes = [C.c_longlong]
-limit.limit_refuse_size.argtypes = [C.c_size_t]
+limit.limit_refuse_size.argtypes = limit.limit_refuse_until_freed.argtypes = [C.c_size_t]
 limit.limit_show_total.argtypes = [C.c_size_t]
 limit.limit_held.restype = C.c_size_t
 
@@ -89,6 +89,25 @@ def sets_do_not_fit():
         limit.limit_refuse_size(0)
         g.run(9)
         same(state(g), single_steps(case, 18))
+
+
+def sets_take_back():
+    # an allocation inside a run takes the arrays of other grids back, and spares the one in use
+    case = walls()
+    words = (70 ** 3 + 31) // 32 + 1
+    with grid(case) as a, grid(case) as b:
+        b.run(9)
+        limit.limit_refuse_until_freed(4 * words)
+        a.run(9)
+        assert limit.limit_refusals() == 1
+        want = single_steps(case, 9)
+        same(state(a), want)
+        same(state(b), want)
+        for g in (a, b):
+            g.run(8)
+        want = single_steps(case, 17)
+        same(state(a), want)
+        same(state(b), want)
 
 
 if __name__ == "__main__":
