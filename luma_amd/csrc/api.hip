@@ -794,7 +794,7 @@ int upload_kids(lumagpu_grid *g) {
         r.u = c->u;
         r.ncell = c->ncell;
     }
-    if (hipMalloc(&g->d_kids, h.size() * sizeof(ChildRef)) != hipSuccess)
+    if (dev_malloc(&g->d_kids, h.size() * sizeof(ChildRef)) != hipSuccess)
         return fail(LUMAGPU_ENOMEM, "refined-region table allocation failed");
     HIP_TRY(hipMemcpy(g->d_kids, h.data(), h.size() * sizeof(ChildRef), hipMemcpyHostToDevice));
     return 0;
@@ -881,9 +881,9 @@ static int build_stale(lumagpu_grid *g, bool *fresh) {
     g->nstale = 0;
     g->stale_list.clear();
     if (cells.empty()) return 0;
-    if (hipMalloc(&g->stale, (size_t)g->Q * cells.size() * g->elem) != hipSuccess ||
-        hipMalloc(&g->stale_idx, g->ncell * sizeof(int)) != hipSuccess ||
-        hipMalloc(&g->stale_cells, cells.size() * sizeof(int)) != hipSuccess)
+    if (dev_malloc(&g->stale, (size_t)g->Q * cells.size() * g->elem) != hipSuccess ||
+        dev_malloc(&g->stale_idx, g->ncell * sizeof(int)) != hipSuccess ||
+        dev_malloc(&g->stale_cells, cells.size() * sizeof(int)) != hipSuccess)
         return fail(LUMAGPU_ENOMEM, "refined-site buffer allocation failed");
     HIP_TRY(hipMemcpy(g->stale_idx, idx.data(), g->ncell * sizeof(int), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(g->stale_cells, cells.data(), cells.size() * sizeof(int), hipMemcpyHostToDevice));
@@ -926,7 +926,7 @@ static int build_mlist(lumagpu_grid *g) {
                 if (!plain) list.push_back((int)c);
             }
     if (!list.empty()) {
-        if (hipMalloc(&g->mlist, list.size() * sizeof(int)) != hipSuccess)
+        if (dev_malloc(&g->mlist, list.size() * sizeof(int)) != hipSuccess)
             return fail(LUMAGPU_ENOMEM, "site list allocation failed");
         HIP_TRY(hipMemcpy(g->mlist, list.data(), list.size() * sizeof(int), hipMemcpyHostToDevice));
     }
@@ -938,7 +938,7 @@ static int build_mlist(lumagpu_grid *g) {
 static int build_links(lumagpu_grid *g) {
     const size_t n = g->nmlist >= 0 ? (size_t)g->nmlist : g->ncell;
     if (n == 0) return 0;
-    if (hipMalloc(&g->link, n * sizeof(uint64_t)) != hipSuccess) {
+    if (dev_malloc(&g->link, n * sizeof(uint64_t)) != hipSuccess) {
         g->link = nullptr;
         return fail(LUMAGPU_ENOMEM, "link word allocation failed");
     }
@@ -980,11 +980,11 @@ static int build_sites(lumagpu_grid *g, bool had) {
 
 // the device's flag bytes and plain-site bitmap
 static int alloc_flags(lumagpu_grid *g) {
-    if (!g->flags && hipMalloc(&g->flags, g->ncell) != hipSuccess) {
+    if (!g->flags && dev_malloc(&g->flags, g->ncell) != hipSuccess) {
         g->flags = nullptr;
         return fail(LUMAGPU_ENOMEM, "flag array allocation failed");
     }
-    if (!g->plain && hipMalloc(&g->plain, (g->ncell + 31) / 32 * sizeof(uint32_t)) != hipSuccess) {
+    if (!g->plain && dev_malloc(&g->plain, (g->ncell + 31) / 32 * sizeof(uint32_t)) != hipSuccess) {
         g->plain = nullptr;
         return fail(LUMAGPU_ENOMEM, "plain-site bitmap allocation failed");
     }
@@ -1073,14 +1073,14 @@ int lumagpu_grid_create(const lumagpu_grid_desc *desc, lumagpu_grid **out) {
     if (dev_malloc(&g->rho, g->ncell * g->melem) != hipSuccess ||
         dev_malloc(&g->u, g->ncell * g->D * g->melem) != hipSuccess)
         return cleanup(LUMAGPU_ENOMEM, "macro array allocation failed");
-    if (hipMalloc(&g->uin, 3 * (size_t)d.M * sizeof(double)) != hipSuccess)
+    if (dev_malloc(&g->uin, 3 * (size_t)d.M * sizeof(double)) != hipSuccess)
         return cleanup(LUMAGPU_ENOMEM, "inlet array allocation failed");
     if (hipMemsetAsync(g->uin, 0, 3 * (size_t)d.M * sizeof(double), g->stream) != hipSuccess)
         return cleanup(LUMAGPU_EHIP, "inlet array clear failed");
     const dim3 gr = cell_grid(d.N, d.M, d.K);
     const size_t nblocks = (size_t)gr.x * gr.y * gr.z;
-    if (hipMalloc(&g->partials, nblocks * kMomentCount * sizeof(double)) != hipSuccess ||
-        hipMalloc(&g->moments_out, kMomentCount * sizeof(double)) != hipSuccess)
+    if (dev_malloc(&g->partials, nblocks * kMomentCount * sizeof(double)) != hipSuccess ||
+        dev_malloc(&g->moments_out, kMomentCount * sizeof(double)) != hipSuccess)
         return cleanup(LUMAGPU_ENOMEM, "reduction buffers allocation failed");
     if (d.forced) {
         if (dev_malloc(&g->force, g->ncell * g->D * g->melem) != hipSuccess)
@@ -1256,10 +1256,10 @@ int lumagpu_set_labels(lumagpu_grid *g, const int *lattyp, const double *xpos, c
         void *p = nullptr;
         ~Freed() { (void)hipFree(p); }
     } edge, erho;
-    if (ne && (hipMalloc(&edge.p, etab.size() * sizeof(int)) != hipSuccess ||
-               hipMalloc(&erho.p, 8 * (size_t)ne * g->melem) != hipSuccess))
+    if (ne && (dev_malloc(&edge.p, etab.size() * sizeof(int)) != hipSuccess ||
+               dev_malloc(&erho.p, 8 * (size_t)ne * g->melem) != hipSuccess))
         return fail(LUMAGPU_ENOMEM, "edge site table allocation failed");
-    if (outlet && !g->xr && hipMalloc(&g->xr, 2 * (size_t)g->Q * g->d.M * g->d.K * g->melem) != hipSuccess) {
+    if (outlet && !g->xr && dev_malloc(&g->xr, 2 * (size_t)g->Q * g->d.M * g->d.K * g->melem) != hipSuccess) {
         g->xr = nullptr;
         return fail(LUMAGPU_ENOMEM, "outlet buffer allocation failed");
     }

@@ -417,7 +417,7 @@ int lu_solve_device(const lumagpu_grid *g, int n, std::vector<double> &a, std::v
         ~Buf() { (void)hipFree(p); }
     } da, dp;
     std::vector<int> piv((size_t)n + 1);
-    if (hipMalloc(&da.p, a.size() * sizeof(double)) != hipSuccess || hipMalloc(&dp.p, piv.size() * sizeof(int)) != hipSuccess)
+    if (dev_malloc(&da.p, a.size() * sizeof(double)) != hipSuccess || dev_malloc(&dp.p, piv.size() * sizeof(int)) != hipSuccess)
         return fail(LUMAGPU_ENOMEM, "IB epsilon system allocation failed");
     double *ad = static_cast<double *>(da.p);
     int *pd = static_cast<int *>(dp.p);
@@ -642,7 +642,7 @@ int upload(lumagpu_grid *g) {
         s->d_pack = s->h_pack = nullptr;
         s->pack_cap = 0;
         const size_t cap = 2 * total;
-        if (hipMalloc(&s->d_pack, cap) != hipSuccess || hipHostMalloc(&s->h_pack, cap, hipHostMallocDefault) != hipSuccess)
+        if (dev_malloc(&s->d_pack, cap) != hipSuccess || hipHostMalloc(&s->h_pack, cap, hipHostMallocDefault) != hipSuccess)
             return fail(LUMAGPU_ENOMEM, "IB buffer allocation failed");
         s->pack_cap = cap;
     } else if (s->pack_busy) {
@@ -661,13 +661,13 @@ int upload(lumagpu_grid *g) {
     if ((r = dev_resize(&s->d_interp, c + 9, (size_t)nm * 4 * w, g->stream)) ||
         (r = dev_resize(&s->d_force, c + 10, (size_t)nm * 3 * w, g->stream)))
         return r;
-    if (!s->d_out && hipMalloc(&s->d_out, 6 * sizeof(double)) != hipSuccess)
+    if (!s->d_out && dev_malloc(&s->d_out, 6 * sizeof(double)) != hipSuccess)
         return fail(LUMAGPU_ENOMEM, "IB buffer allocation failed");
     if (order != s->sites) {
         s->sites_dirty = 1;
         s->site_map_ok = 0;
     }
-    if (!s->d_site_of && !ibm_has_flexible(g) && hipMalloc(&s->d_site_of, g->ncell * sizeof(int)) != hipSuccess)
+    if (!s->d_site_of && !ibm_has_flexible(g) && dev_malloc(&s->d_site_of, g->ncell * sizeof(int)) != hipSuccess)
         return fail(LUMAGPU_ENOMEM, "IB site map allocation failed");
     s->sites = order;
     s->nsites = (int)order.size();
@@ -706,7 +706,7 @@ int check_body(lumagpu_grid *g, int body) {
 
 int ensure_flags(lumagpu_grid *g) {
     if (g->hflags.size() != g->ncell) g->hflags.assign(g->ncell, (uint8_t)kFluid);
-    if (!g->flags && hipMalloc(&g->flags, g->ncell) != hipSuccess)
+    if (!g->flags && dev_malloc(&g->flags, g->ncell) != hipSuccess)
         return fail(LUMAGPU_ENOMEM, "flag array allocation failed");
     return 0;
 }
@@ -766,7 +766,7 @@ int clear_gone(lumagpu_grid *g) {
                 s->d_gone = s->h_gone = nullptr;
                 s->gone_cap = 0;
                 const size_t cap = 2 * gone.size();
-                if (hipMalloc(&s->d_gone, cap * sizeof(int)) != hipSuccess ||
+                if (dev_malloc(&s->d_gone, cap * sizeof(int)) != hipSuccess ||
                     hipHostMalloc(&s->h_gone, cap * sizeof(int), hipHostMallocDefault) != hipSuccess)
                     return fail(LUMAGPU_ENOMEM, "IB buffer allocation failed");
                 s->gone_cap = cap;

@@ -46,7 +46,7 @@ int dev_resize(T **d, size_t *cap, size_t n, hipStream_t s) {
     *d = nullptr;
     *cap = 0;
     if (n == 0) return 0;
-    if (hipMalloc(d, n * sizeof(T)) != hipSuccess) return fail(LUMAGPU_ENOMEM, "IB buffer allocation failed");
+    if (dev_malloc(d, n * sizeof(T)) != hipSuccess) return fail(LUMAGPU_ENOMEM, "IB buffer allocation failed");
     *cap = n;
     if (hipMemsetAsync(*d, 0, n * sizeof(T), s) != hipSuccess) return fail(LUMAGPU_EHIP, "IB buffer clear failed");
     return 0;

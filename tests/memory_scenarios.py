@@ -110,6 +110,38 @@ def sets_take_back():
         same(state(b), want)
 
 
+def others_give_way():
+    # with no memory left but another grid's second array: labels, outlet, bodies and their steps
+    case = setups.uniform_inflow_3d(60, 50, 44, 0.03, 0.6)
+    pos = setups.sphere_markers((20.3, 25.1, 22.2), 5.0, 1.0)
+
+    class Tight(GpuGrid):
+        def set_labels(self, *a):
+            limit.limit_budget(0)
+            super().set_labels(*a)
+
+    def flow(cls):
+        with cls.from_case(case, "fp64", store_macro=True) as g:
+            limit.limit_budget(-1)
+            if cls is Tight:
+                b2 = grid(walls())
+                b2.run(9)
+                limit.limit_budget(0)
+            g.ibm_add_body(pos)
+            g.ibm_initialise()
+            g.run(4)
+            limit.limit_budget(-1)
+            return state(g)
+
+    want = flow(GpuGrid)
+    with grid(walls()) as b:
+        b.run(9)
+        same(flow(Tight), want)
+        assert limit.limit_refusals() >= 2
+        b.run(8)
+        same(state(b), single_steps(walls(), 17))
+
+
 if __name__ == "__main__":
     print(f"[memory] {sys.argv[1]}", flush=True)
     globals()[sys.argv[1]]()
