@@ -17,7 +17,6 @@
 #include <memory>
 
 #include "ibm_system.hpp"
-#include "lu_device.hpp"
 
 namespace lumagpu {
 
@@ -410,27 +409,6 @@ int lu_solve_band(int n, int kl, int ku, std::vector<Dual> &a, std::vector<Dual>
 
 namespace {
 
-// lu_solve with the factorisation on the device (see lu_device.hip: the same factors)
-int lu_solve_device(const lumagpu_grid *g, int n, std::vector<double> &a, std::vector<double> &x) {
-    struct Buf {
-        void *p = nullptr;
-        ~Buf() { (void)hipFree(p); }
-    } da, dp;
-    std::vector<int> piv((size_t)n + 1);
-    if (dev_malloc(&da.p, a.size() * sizeof(double)) != hipSuccess || dev_malloc(&dp.p, piv.size() * sizeof(int)) != hipSuccess)
-        return fail(LUMAGPU_ENOMEM, "IB epsilon system allocation failed");
-    double *ad = static_cast<double *>(da.p);
-    int *pd = static_cast<int *>(dp.p);
-    HIP_TRY(hipMemcpyAsync(ad, a.data(), a.size() * sizeof(double), hipMemcpyHostToDevice, g->stream));
-    HIP_TRY(lu_factor_device(n, ad, pd, pd + n, g->stream));
-    HIP_TRY(hipMemcpyAsync(piv.data(), pd, piv.size() * sizeof(int), hipMemcpyDeviceToHost, g->stream));
-    if (int r = copy_to_host(g, a.data(), ad, a.size() * sizeof(double))) return r;
-    HIP_TRY(hipStreamSynchronize(g->stream));
-    if (piv[n]) return fail(LUMAGPU_EPHYS, "singular IB epsilon system");
-    lu_substitute(n, a.data(), piv.data(), x.data());
-    return 0;
-}
-
 // ibm_findEpsilon, :773-920: A_IJ = ds_J * sum_s delta_I(s) delta(x_J - x_s) A_I, A eps = 1.
 // On a tangent-form grid also d eps from A d(eps) = -dA eps, with dA from the marker, delta
 // and ds tangents.
@@ -507,13 +485,13 @@ int find_epsilon(const lumagpu_grid *g, Body &b) {
     std::vector<double> A0;
     if (tan) A0 = A;
     // a chain of markers (a filament) gives a matrix banded in marker order: the banded solver,
-    // which skips only the exact zeros outside the band, otherwise the dense one
+    // which skips only the exact zeros outside the band, otherwise the dense one, which passes over the
+    // zeros it meets.  Both on the host: the matrix is built here and sparse, and the device's chain of
+    // pivots with the copies both ways took longer (bodies of 200, 800, 1600 markers, ms for the whole
+    // of ibm_initialise, host / device: circle 0.9 / 1.8, 3.7 / 7.3, 10.6 / 35.8; sphere 3.7 / 4.5,
+    // 17.8 / 18.5, 45 / 57; a sphere of 3000 134 / 126)
     const bool band = 4 * (kl + ku) < n;
-    int r = 0;
-    if (band) r = lu_solve_band_t(n, kl, ku, A, rhs, "singular IB epsilon system");
-    else if (n >= kLuDeviceMin && n <= kLuDeviceMax) r = lu_solve_device(g, n, A, rhs);
-    else r = lu_solve(n, A, rhs);
-    if (r) return r;
+    if (int r = band ? lu_solve_band_t(n, kl, ku, A, rhs, "singular IB epsilon system") : lu_solve(n, A, rhs)) return r;
     for (int i = 0; i < n; ++i) b.m[i].eps = rhs[i];
     if (tan) {
         std::vector<double> drhs(n, 0.0);

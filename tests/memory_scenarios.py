@@ -142,6 +142,18 @@ def others_give_way():
         same(state(b), single_steps(walls(), 17))
 
 
+def epsilon_on_the_host():
+    # ibm_initialise needs no device memory for its marker system
+    n = 300
+    case = setups.uniform_inflow_3d(30, 26, 26, 0.03, 0.6)
+    pos = setups.sphere_markers((13.1, 13.2, 13.3), 5.0, 1.0, n=n)
+    limit.limit_refuse_size(8 * n * n)
+    with grid(case, "fp64") as g:
+        g.ibm_add_body(pos)
+        g.ibm_initialise()
+        assert np.isfinite(g.ibm_markers(0)["eps"]).all() and limit.limit_refusals() == 0
+
+
 if __name__ == "__main__":
     print(f"[memory] {sys.argv[1]}", flush=True)
     globals()[sys.argv[1]]()
