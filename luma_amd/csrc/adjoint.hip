@@ -284,7 +284,11 @@ int position_chains(lumagpu_grid *g, const double *sdd, const double *epsbar, co
         const double *eb = epsbar + first;
         double *db = dsbar.data() + first, *xb = xg + 3 * (size_t)first;
         const int n = (int)ms.size();
-        if (n >= kLuDeviceMin && n <= kLuDeviceMax) return epsilon_chain_device(g, ms, first, sdd, eb, db, xb);
+        if (n >= kLuDeviceMin && n <= kLuDeviceMax) {
+            const int r = epsilon_chain_device(g, ms, first, sdd, eb, db, xb);
+            if (r != LUMAGPU_ENOMEM) return r;
+            (void)hipGetLastError();   // no room for its matrix: nothing has been written yet
+        }
         return epsilon_chain(g, ms, eb, db, xb);
     };
     if (s->universal) {

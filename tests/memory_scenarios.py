@@ -154,6 +154,25 @@ def epsilon_on_the_host():
         assert np.isfinite(g.ibm_markers(0)["eps"]).all() and limit.limit_refusals() == 0
 
 
+def position_gradient_on_the_host():
+    # the same sums in another order: n markers' terms, each rounded at 1e-16 of the largest
+    n = 200
+    case = setups.uniform_inflow_3d(30, 26, 26, 0.03, 0.6)
+    pos = setups.sphere_markers((13.1, 13.2, 13.3), 4.0, 1.0, n=n)
+    out = []
+    for size in (0, 8 * n * n):
+        limit.limit_refuse_size(size)
+        with grid(case, "fp64") as g:
+            g.ibm_add_body(pos)
+            g.ibm_initialise()
+            out.append(g.adj_run(5, 3))
+        assert limit.limit_refusals() == (2 if size else 0)      # tried again after taking back
+    a, b = out
+    assert a["J"] == b["J"]
+    g = np.abs(a["dJ_dpos"]).max()
+    assert g > 0 and np.abs(a["dJ_dpos"] - b["dJ_dpos"]).max() <= 1e-11 * g
+
+
 if __name__ == "__main__":
     print(f"[memory] {sys.argv[1]}", flush=True)
     globals()[sys.argv[1]]()
