@@ -238,12 +238,12 @@ int epsilon_chain_device(lumagpu_grid *g, const std::vector<const Marker *> &ms,
         for (int k = 0; k < ms[i]->ns; ++k)
             for (int a = 0; a < 3; ++a) h[5 * n + 3 * (i * S + k) + a] = ms[i]->sxyz[k][a];
     }
-    // markers; then mu, xg and dsbar; the matrix; pivots and info
+    // markers; then mu, xg and dsbar; the matrix; pivots, info and its shape
     DevBuf geo, vec, mat, piv;
     if (int r = geo.alloc(g, h.size() * sizeof(double))) return r;
     if (int r = vec.alloc(g, 5 * n * sizeof(double))) return r;
     if (int r = mat.alloc(g, n * n * sizeof(double))) return r;
-    if (int r = piv.alloc(g, (n + 1) * sizeof(int))) return r;
+    if (int r = piv.alloc(g, (n + 4) * sizeof(int))) return r;
     double *gd = static_cast<double *>(geo.p), *vd = static_cast<double *>(vec.p), *a = static_cast<double *>(mat.p);
     int *pd = static_cast<int *>(piv.p);
     HIP_TRY(hipMemcpyAsync(gd, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice, g->stream));
@@ -251,18 +251,30 @@ int epsilon_chain_device(lumagpu_grid *g, const std::vector<const Marker *> &ms,
                       gd,           gd + 3 * n,     gd + 4 * n,    gd + 5 * n,
                       s->d_ns + first, s->d_sdelta + (size_t)first * S, sdd + (size_t)first * S * 3, s->d_eps + first,
                       s->d_ds + first};
-    k_eps_matrix<<<dim3((unsigned)((n + 255) / 256), (unsigned)n), 256, 0, g->stream>>>(e, a);
+    HIP_TRY(hipMemsetAsync(pd + n + 1, 0, 3 * sizeof(int), g->stream));
+    k_eps_matrix<<<dim3((unsigned)((n + 255) / 256), (unsigned)n), 256, 0, g->stream>>>(e, a, pd + n + 1);
     HIP_TRY(hipGetLastError());
-    HIP_TRY(lu_factor_device((int)n, a, pd, pd + n, g->stream));
-    std::vector<double> lu(n * n);
+    int shape[3];   // the band of A^T's column-major view, as in epsilon_chain, and the nonzeros
+    HIP_TRY(hipMemcpyAsync(shape, pd + n + 1, sizeof shape, hipMemcpyDeviceToHost, g->stream));
+    HIP_TRY(hipStreamSynchronize(g->stream));
+    const bool sparse = (size_t)shape[2] <= kLuSparse * n;
+    if (!sparse) HIP_TRY(lu_factor_device((int)n, a, pd, pd + n, g->stream));
+    // the host's pages while the device factors
+    std::vector<double> lu(n * n), v(epsbar, epsbar + n);
     std::vector<int> hp(n + 1);
     HIP_TRY(hipMemcpyAsync(hp.data(), pd, hp.size() * sizeof(int), hipMemcpyDeviceToHost, g->stream));
     if (int r = copy_to_host(g, lu.data(), a, lu.size() * sizeof(double))) return r;
     HIP_TRY(hipStreamSynchronize(g->stream));
-    if (hp[n]) return fail(LUMAGPU_EPHYS, "singular IB epsilon system");
-    std::vector<double> v(5 * n);
-    std::copy(epsbar, epsbar + n, v.begin());
-    lu_substitute((int)n, lu.data(), hp.data(), v.data());
+    if (sparse) {
+        const int kl = shape[0], ku = shape[1];
+        if (int r = kl + ku < (int)n - 1 ? lu_solve_band((int)n, kl, ku, lu, v, "singular IB epsilon system")
+                                         : lu_solve((int)n, lu, v))
+            return r;
+    } else {
+        if (hp[n]) return fail(LUMAGPU_EPHYS, "singular IB epsilon system");
+        lu_substitute((int)n, lu.data(), hp.data(), v.data());
+    }
+    v.resize(5 * n);
     std::copy(xg, xg + 3 * n, v.begin() + n);
     std::copy(dsbar, dsbar + n, v.begin() + 4 * n);
     HIP_TRY(hipMemcpyAsync(vd, v.data(), v.size() * sizeof(double), hipMemcpyHostToDevice, g->stream));

@@ -631,15 +631,27 @@ __device__ __forceinline__ double eps_delta_at(const EpsSystem &e, int J, const 
     return v;
 }
 
-// A_IJ = ds_J sum_k delta_I(s_k) delta(x_J; s_k) area_I into a[J * n + I]; one thread per pair
-static __global__ __launch_bounds__(256) void k_eps_matrix(EpsSystem e, double *a) {
+// A_IJ = ds_J sum_k delta_I(s_k) delta(x_J; s_k) area_I into a[J * n + I], one thread per pair, and
+// how far the nonzero ones lie below and above the diagonal (I - J, J - I) and how many they are into shape[3]
+static __global__ __launch_bounds__(256) void k_eps_matrix(EpsSystem e, double *a, int *shape) {
     const int I = blockIdx.x * blockDim.x + threadIdx.x, J = blockIdx.y;
-    if (I >= e.n) return;
-    double acc = 0.0;
-    if (!eps_far(e, I, J))
-        for (int k = 0; k < e.ns[I]; ++k)
-            acc += e.sdelta[(size_t)I * e.S + k] * eps_delta_at(e, J, e.sxyz + ((size_t)I * e.S + k) * 3) * e.area[I];
-    a[(size_t)J * e.n + I] = acc * e.ds[J];
+    double v = 0.0;
+    if (I < e.n) {
+        double acc = 0.0;
+        if (!eps_far(e, I, J))
+            for (int k = 0; k < e.ns[I]; ++k)
+                acc += e.sdelta[(size_t)I * e.S + k] * eps_delta_at(e, J, e.sxyz + ((size_t)I * e.S + k) * 3) * e.area[I];
+        v = acc * e.ds[J];
+        a[(size_t)J * e.n + I] = v;
+    }
+    // atomics of a wave that holds a nonzero: its first and last lane with one, and their number
+    const uint64_t m = __ballot(v != 0.0);
+    if (m && (threadIdx.x & 63) == 0) {
+        const int lo = I + __ffsll((unsigned long long)m) - 1, hi = I + 63 - __clzll((long long)m);
+        atomicMax(shape, hi - J);
+        atomicMax(shape + 1, J - lo);
+        atomicAdd(shape + 2, __popcll(m));
+    }
 }
 
 // With A^T mu = epsbar: dJ/dA_IJ = -mu_I eps_J, and A's entries depend on both markers' positions and

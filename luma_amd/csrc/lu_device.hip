@@ -1,4 +1,5 @@
-// lu_device.hip -- LU factorisation with row pivoting of the marker systems (A eps = 1) on the device.
+// lu_device.hip -- LU factorisation with row pivoting of the marker systems (A eps = 1) on the device, for the
+// position gradient of large bodies (adjoint.hip).
 //
 // The systems are dense in storage and a few hundred to a few thousand markers large.  lu_solve on the
 // host takes its rank-1 updates one column after another; here the same operations run column

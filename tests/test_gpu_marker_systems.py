@@ -76,3 +76,28 @@ def test_singular_system_is_refused():
             g.ibm_initialise()
             g.adj_run(2, 2, initial=False)
             raise RuntimeError("epsilon system accepted")
+
+
+# a chain of markers couples to its neighbours alone: its matrix is made on the device and solved in the
+# band, up to the length where a panel of the dense factorisation takes two rows per thread and beyond
+@pytest.mark.parametrize("n", [192, 1030])
+def test_position_gradient_of_a_chain(n):
+    case = setups.channel_2d(n + 40, 34, 12.0, 0.04, 20.0)
+    dh = case.info["dh"]
+    r = np.random.default_rng(n)
+    pos = np.zeros((n, 3))
+    pos[:, 0] = (20.2 + np.arange(n) + r.uniform(-0.2, 0.2, n)) * dh
+    pos[:, 1] = (17.3 + r.uniform(-0.2, 0.2, n)) * dh
+
+    def run(p, **kw):
+        with GpuGrid.from_case(case, "fp64") as g:
+            g.ibm_add_body(p)
+            g.ibm_initialise()
+            return g.adj_run(6, 3, **kw)
+    print(f"[eps] chain {n}", flush=True)
+    grad = run(pos, initial=False)["dJ_dpos"]
+    d = np.zeros((n, 3))
+    d[:, :2] = r.standard_normal((n, 2)) * dh
+    h = 1e-5
+    fd = (run(pos + h * d, backward=False)["J"] - run(pos - h * d, backward=False)["J"]) / (2.0 * h)
+    assert abs((grad * d).sum() - fd) <= 1e-4 * abs(fd) + 1e-9
