@@ -10,8 +10,8 @@ namespace lumagpu {
 // registers, and the host solves.
 constexpr int kLuDeviceMin = 192, kLuDeviceMax = 4096;
 // Nonzeros per marker up to which the host solves the matrix that the device made: chains and rings of
-// markers a cell apart have 7, and their factors stay sparse, where the device's work grows with n^3;
-// surfaces of such markers have 30.  A gradient over 4 steps, dense on the device -> on the host: chain of
+// markers a cell apart have about 7, and their factors stay sparse, where the device's work grows with n^3;
+// surfaces of such markers about 30.  A gradient over 4 steps, dense on the device -> on the host: chain of
 // 200 / 800 / 1600 markers 1.8 -> 1.0, 6.6 -> 2.7, 32 -> 8 ms, ring of 1600 33 -> 13; all on the host
 // 1.9, 7.3, 26, 32; a sphere of 1600 is 35 ms on the device, 176 on the host.
 constexpr int kLuSparse = 12;

@@ -2,10 +2,12 @@
 gradient against central differences of the forward, as in the other gradient tests, for body
 sizes around the device's lower limit, multiples of the factorisation's 16-column panels and its
 1024 rows per block; and a singular system's refusal."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
-from luma_amd import setups
+from luma_amd import _abi, setups
 from luma_amd.grid import GpuGrid
 from oracle.oracle import OracleGrid, OracleIBM
 
@@ -101,3 +103,55 @@ def test_position_gradient_of_a_chain(n):
     h = 1e-5
     fd = (run(pos + h * d, backward=False)["J"] - run(pos - h * d, backward=False)["J"]) / (2.0 * h)
     assert abs((grad * d).sum() - fd) <= 1e-4 * abs(fd) + 1e-9
+
+
+# ---- the factorisation itself --------------------------------------------------------------------
+# lu_factor_device is no entry of the C ABI: it is called by its C++ name, in buffers of the runtime that
+# the library links
+def _factor(a):
+    lib, hip = _abi.load(), C.CDLL("libamdhip64.so.7")
+    n = a.shape[0]
+    f = lib["_ZN7lumagpu16lu_factor_deviceEiPdPiS1_P12ihipStream_t"]
+    f.argtypes = [C.c_int, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]
+    da, dp = C.c_void_p(), C.c_void_p()
+    assert hip.hipMalloc(C.byref(da), C.c_size_t(8 * n * n)) == 0
+    assert hip.hipMalloc(C.byref(dp), C.c_size_t(4 * (n + 1))) == 0
+    m = np.asfortranarray(a, dtype=np.float64)     # column-major
+    piv = np.full(n + 1, -1, np.int32)
+    ptr = lambda x: C.c_void_p(x.ctypes.data)
+    try:
+        assert hip.hipMemcpy(da, ptr(m), C.c_size_t(m.nbytes), 1) == 0
+        assert f(n, da, dp, C.c_void_p(dp.value + 4 * n), None) == 0
+        assert hip.hipDeviceSynchronize() == 0
+        assert hip.hipMemcpy(ptr(m), da, C.c_size_t(m.nbytes), 2) == 0
+        assert hip.hipMemcpy(ptr(piv), dp, C.c_size_t(piv.nbytes), 2) == 0
+    finally:
+        hip.hipFree(da)
+        hip.hipFree(dp)
+    return m, piv[:n], int(piv[n])
+
+
+# one column, a panel of 16 and its neighbours, several panels, two rows per thread
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 200, 1030])
+def test_factors_in_the_order_of_dgetf2(n):
+    a = np.random.default_rng(n).standard_normal((n, n))
+    print(f"[eps] factors {n}", flush=True)
+    got, piv, info = _factor(a)
+    m, want = a.copy(order="F"), np.empty(n, int)
+    for j in range(n):
+        p = j + int(np.argmax(np.abs(m[j:, j])))
+        want[j] = p
+        m[[j, p]] = m[[p, j]]
+        m[j + 1:, j] *= 1.0 / m[j, j]
+        m[j + 1:, j + 1:] -= m[j + 1:, j, None] * m[j, j + 1:]
+    assert info == 0 and np.array_equal(piv, want) and np.array_equal(got, m)
+
+
+# a column of zeros stays one under every update: the pivot of that column is exactly zero, in the first
+# panel, at a panel's first and last column, in the last panel, with one, two and four rows per thread
+@pytest.mark.parametrize("n,col", [(1, 0), (40, 0), (40, 15), (40, 16), (40, 39), (1100, 700), (2100, 8), (2100, 2099)])
+def test_zero_pivot_is_reported(n, col):
+    a = np.random.default_rng(n + col).standard_normal((n, n))
+    a[:, col] = 0.0
+    print(f"[eps] zero pivot {n} {col}", flush=True)
+    assert _factor(a)[2] == col + 1
