@@ -533,8 +533,10 @@ bool pair_ok(const lumagpu_grid *g) {
 // the deep cells and the lists around them, from the flags on the device; LUMAGPU_ENOMEM where they do
 // not fit
 int pair_sets(lumagpu_grid *g) {
-    if (!g->masked || g->pair_version == g->flags_version) return 0;
-    g->pair_version = 0;
+    // deep are cells by their types and, with bodies, by which sites these flag
+    const uint64_t key[2] = {g->types_version, ibm_marker_count(g) > 0 ? g->flags_version : 0};
+    if (!g->masked || (g->pair_key[0] == key[0] && g->pair_key[1] == key[1])) return 0;
+    g->pair_key[0] = 0;
     const size_t nw = (g->ncell + 31) / 32 + 1;   // a whole pair of words at the end
     struct Buf {
         uint32_t *p = nullptr;
@@ -576,7 +578,8 @@ int pair_sets(lumagpu_grid *g) {
         HIP_TRY(hipGetLastError());
         HIP_TRY(hipStreamSynchronize(g->stream));
     }
-    g->pair_version = g->flags_version;
+    g->pair_key[0] = key[0];
+    g->pair_key[1] = key[1];
     return 0;
 }
 
@@ -963,6 +966,8 @@ static int build_sites(lumagpu_grid *g, bool had) {
         g->sites_ok = 1;
         return 0;
     }
+    ++g->types_version;
+    g->pair_synced = 0;   // other cells may be the ones that never step
     (void)hipStreamSynchronize(g->stream);
     (void)hipFree(g->mlist);
     (void)hipFree(g->link);
@@ -993,7 +998,6 @@ static int alloc_flags(lumagpu_grid *g) {
 
 int upload_flags(lumagpu_grid *g) {
     ++g->flags_version;
-    g->pair_synced = 0;
     if (g->hflags.size() != g->ncell) return fail(LUMAGPU_ESTATE, "host flag array does not cover the grid");
     if (int r = alloc_flags(g)) return r;
     // from here until the list and the link words are whole a step would read parts of two states:

@@ -45,7 +45,9 @@ struct lumagpu_grid {
     int *pair_cells = nullptr;
     uint64_t *pair_links = nullptr;
     int n_near = 0, n_rest = 0;
-    uint64_t flags_version = 1, pair_version = 0;   // of the flag bytes; those the sets were built from
+    uint64_t flags_version = 1;       // of the flag bytes, force bits included
+    uint64_t types_version = 1;       // of the flag bytes without them
+    uint64_t pair_key[2] = {0, 0};    // types and, with bodies, flags version that the sets were built from
     int pair_synced = 0;              // slots that no step writes are the same in f and f2
     int fuse_shape = -1, fuse_zc = 0; // its tile shape (FusedShape, -1: off) and z planes per block
     uint8_t *flags = nullptr;

@@ -173,6 +173,24 @@ def position_gradient_on_the_host():
     assert g > 0 and np.abs(a["dJ_dpos"] - b["dJ_dpos"]).max() <= 1e-11 * g
 
 
+def force_set_again():
+    # other forces leave the site types, and with them the sets of two steps per launch, as they are
+    case = walls()
+    force = [case.force, 2.0 * case.force, case.force.copy()]
+    force[2][20:40, 10:30] = 0.0                # other force bits
+    with grid(case) as a, grid(case) as b:
+        for f in force:
+            calls = limit.limit_calls()
+            for g in (a, b):
+                g.set_force(f)
+            a.run(9)
+            if f is not force[0]:
+                assert limit.limit_calls() == calls, "sets or arrays made again"
+            for _ in range(9):
+                b.LBM_multi_opt()
+            same(state(a), state(b))
+
+
 if __name__ == "__main__":
     print(f"[memory] {sys.argv[1]}", flush=True)
     globals()[sys.argv[1]]()
