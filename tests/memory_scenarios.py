@@ -2,6 +2,7 @@
 (test_gpu_memory.py): the limiter has to be loaded before the library.  A scenario raises where it
 fails and prints its name at the end."""
 import ctypes as C
+import dataclasses
 import sys
 from pathlib import Path
 
@@ -50,17 +51,16 @@ def same(a, b):
 
 
 def labels_cut_short():
-    # the link words of the new labels do not fit: the call fails and steps are refused, until the
-    # labels have been set; nothing reads a part of them
+    # the link words of new labels do not fit: the call fails and steps are refused, until the labels
+    # have been set; nothing reads a part of them
     case = setups.lid_driven_cavity(40, re=200.0)
-    lt = case.lattyp.copy()
-    lt[10:15, 12:20] = setups.SOLID
-    with grid(case) as g, grid(case) as h:
+    box = dataclasses.replace(case, lattyp=None)
+    with grid(box) as g, grid(box) as h:
         g.run(4)
         h.run(4)
         limit.limit_refuse_size(8 * 40 * 40)
         try:
-            g.set_labels(lt, case.xpos, case.ypos, case.zpos)
+            g.set_labels(case.lattyp, case.xpos, case.ypos, case.zpos)
             raise AssertionError("link words allocated")
         except LumaGpuError as e:
             assert "allocation" in str(e)
@@ -72,7 +72,7 @@ def labels_cut_short():
                 assert "set them again" in str(e)
         limit.limit_refuse_size(0)
         for x in (g, h):
-            x.set_labels(lt, case.xpos, case.ypos, case.zpos)
+            x.set_labels(case.lattyp, case.xpos, case.ypos, case.zpos)
             x.run(6)
         same(state(g), state(h))
 
@@ -189,6 +189,23 @@ def force_set_again():
             for _ in range(9):
                 b.LBM_multi_opt()
             same(state(a), state(b))
+
+
+def labels_set_again():
+    # new labels of a small grid go into the arrays that it has
+    case = setups.lid_driven_cavity(40, re=200.0)
+    lt = [case.lattyp, case.lattyp.copy()]
+    lt[1][10:15, 12:20] = setups.SOLID
+    with grid(case, "fp64") as g:
+        calls = limit.limit_calls()
+        for k in (1, 0, 1):
+            g.set_labels(lt[k], case.xpos, case.ypos, case.zpos)
+        assert limit.limit_calls() == calls
+        for _ in range(5):
+            g.LBM_multi_opt()
+        got = state(g)
+    case.lattyp = lt[1]
+    same(got, single_steps(case, 5, "fp64"))
 
 
 if __name__ == "__main__":
