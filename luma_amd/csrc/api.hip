@@ -489,6 +489,17 @@ bool multi_ok(const lumagpu_grid *g) {
            !(g->re_ramp > 0.0) && g->nedge == 0 && g->simple_types && g->ncell <= (size_t(1) << 18) && g->has_state && (!g->masked || g->sites_ok);
 }
 
+// Fewer steps than these go one per launch: the first launches of a run follow each other every 3 us, and
+// a window's start (its loads, 9 planes through LDS) costs 2 to 9 of them.  run(n) with the wait after it,
+// single / several per launch, us: box FP32 48^2 n = 2 16.6 / 17.5, 4 22.1 / 18.9, 512^2 n = 2 22.7 / 26.5, 4
+// 35.4 / 31.6; box FP64 256^2 n = 2 19.7 / 24.5, 4 29.3 / 29.5, 512^2 n = 2 30 / 38, 4 51 / 49; lid FP64 320^2
+// n = 2 25.0 / 26.3, 4 39.8 / 33.1.  FP64 windows of a small box, whose single steps are launches and little
+// else: 48^2 n = 4 22.4 / 25.6, 6 28.3 / 29.8, 128^2 n = 4 24.0 / 26.9, 6 30.8 / 30.4; from 8 steps on single
+// ones are replayed as a graph, 48^2 54 / 33.
+int multi_min(const lumagpu_grid *g) {
+    return g->d.precision == LUMAGPU_FP64 && !g->masked && multi2d_blocks(g->d.N, g->d.M, 6) <= 64 ? 8 : 4;
+}
+
 // up to n steps from the post-local layout, as many as whole launches take; *done: steps run
 int run_multi(lumagpu_grid *g, int n, int *done) {
     *done = 0;
@@ -496,7 +507,7 @@ int run_multi(lumagpu_grid *g, int n, int *done) {
     const F2Use use(g);
     // begin_step's state for a grid without bodies
     g->all_forced = g->sweep1_zero = 0;
-    while (n - *done >= 2) {
+    while (n - *done >= multi_min(g)) {
         const int H = plan_multi2d(g->d.N, g->d.M, n - *done, g->d.precision == LUMAGPU_FP64);
         StepArgs a = make_args(g);
         if (!g->masked) {   // flag bytes that other calls made are not this step's
@@ -1798,7 +1809,7 @@ int lumagpu_run(lumagpu_grid *g, int nsteps) {
             if (int r = run_pairs(g, nsteps - s, &done)) return r;
         s += done;
     }
-    if (nsteps - s >= 2 && multi_ok(g)) {
+    if (nsteps - s >= multi_min(g) && multi_ok(g)) {
         if (g->parity != 0) {
             if (int r = apply_step(g, 0, nullptr, nullptr)) return r;
             ++s;
@@ -1810,7 +1821,7 @@ int lumagpu_run(lumagpu_grid *g, int nsteps) {
     // Long runs of a hierarchy without host work per step replay a captured pair of steps: the
     // step alternates between the two AA kernels, so two steps are the period (the child's
     // four sub-steps included).  One eager step first settles the IB support flags.
-    if (nsteps >= 8 && graph_ok(g)) {
+    if (nsteps - s >= 8 && graph_ok(g)) {
         while (s < nsteps && (s == 0 || g->parity != 0)) {
             if (int r = apply_step(g, 0, nullptr, nullptr)) return r;
             ++s;

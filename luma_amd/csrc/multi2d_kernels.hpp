@@ -113,6 +113,12 @@ __global__ __launch_bounds__(kMultiWindow *kMultiWindow) void k_multi2d(StepArgs
     }
 }
 
+// blocks of a launch of H steps
+inline long multi2d_blocks(int nx, int ny, int H) {
+    const int tile = kMultiWindow - 2 * H;
+    return (long)((nx + tile - 1) / tile) * ((ny + tile - 1) / tile);
+}
+
 // Steps per launch for up to n (even) steps: the H whose launch, rounds of blocks over the
 // 256 CUs and window steps cost least per step.  The two constants are what launches of H = 8
 // (256 x 256, one block per CU) and H = 12 (64 x 64) take together with their lids.
@@ -121,9 +127,7 @@ inline int plan_multi2d(int nx, int ny, int n, bool fp64) {
     int best = 0;
     double cost = 0.0;
     for (int H = 2; H <= 12 && H <= n; H += 2) {
-        const int tile = kMultiWindow - 2 * H;
-        const long blocks = (long)((nx + tile - 1) / tile) * ((ny + tile - 1) / tile);
-        const double c = (launch_us + H * step_us * ((blocks + 255) / 256)) / H;
+        const double c = (launch_us + H * step_us * ((multi2d_blocks(nx, ny, H) + 255) / 256)) / H;
         if (best == 0 || c < cost) {
             best = H;
             cost = c;

@@ -208,6 +208,18 @@ def labels_set_again():
     same(got, single_steps(case, 5, "fp64"))
 
 
+def short_runs_step_singly():
+    # too short for several steps per launch: no second array for them
+    for n, form, steps in ((48, "fp64", 7), (400, "fp64", 3), (48, "fp32s", 3)):
+        with GpuGrid.from_case(setups.taylor_green((n, n, 1), u0=0.04, tau=0.6, dims=2), form) as g:
+            calls = limit.limit_calls()
+            for _ in range(3):
+                g.run(steps)
+            assert limit.limit_calls() == calls, (n, form)
+            g.run(40)
+            assert limit.limit_calls() == calls + 1, (n, form)
+
+
 if __name__ == "__main__":
     print(f"[memory] {sys.argv[1]}", flush=True)
     globals()[sys.argv[1]]()

@@ -81,3 +81,20 @@ def test_new_state_and_labels_between_runs():
         for _ in range(10):
             b.LBM_multi_opt()
         assert np.array_equal(a.download_f(), b.download_f())
+
+
+# runs on both sides of the least counts (4, and 8 for small FP64 boxes), from both layouts, with the steps
+# that are left over one at a time
+@pytest.mark.parametrize("kind", ["periodic", "regularised"])
+@pytest.mark.parametrize("n", [40, 330])
+@pytest.mark.parametrize("form", ["fp64", "fp32s"])
+def test_short_runs(kind, n, form):
+    case = _case(kind, n, n)
+    print(f"[multi2d] short {kind} {n} {form}", flush=True)
+    with GpuGrid.from_case(case, form, store_macro=True) as a, GpuGrid.from_case(case, form, store_macro=True) as b:
+        for steps in (4, 6, 7, 8, 9, 1, 5, 10, 13, 3):
+            a.run(steps)
+            for _ in range(steps):
+                b.LBM_multi_opt()
+            for p, q in zip((a.download_f(),) + a.download_macro(), (b.download_f(),) + b.download_macro()):
+                assert np.array_equal(p, q), steps
