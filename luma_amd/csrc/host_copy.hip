@@ -39,13 +39,30 @@ int cpus() {
     return CPU_COUNT(&set);
 }
 
+// the grid's device current on this thread while the object lives: the caller's own thread, which copies
+// too, gets back the device it had
+struct DeviceGuard {
+    int had = -1;
+    hipError_t e;
+    explicit DeviceGuard(int device) {
+        e = hipGetDevice(&had);
+        if (e == hipSuccess && had == device) had = -1;
+        else if (e == hipSuccess) e = hipSetDevice(device);
+    }
+    DeviceGuard(const DeviceGuard &) = delete;
+    DeviceGuard &operator=(const DeviceGuard &) = delete;
+    ~DeviceGuard() {
+        if (had >= 0) (void)hipSetDevice(had);
+    }
+};
+
 // the pieces first, first + n, ... of one copy; each waits for its own DMA only
 hipError_t copy_pieces(const lumagpu_grid *g, char *dst, const char *src, size_t bytes, int first, int n, char *pin,
                        std::atomic<bool> &stop) {
-    hipError_t e = hipSetDevice(g->device);
-    if (e != hipSuccess) return e;
+    const DeviceGuard device(g->device);
+    if (device.e != hipSuccess) return device.e;
     hipEvent_t ev = nullptr;
-    e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+    hipError_t e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
     if (e != hipSuccess) return e;
     for (size_t off = (size_t)first * kPipeSlot; off < bytes && e == hipSuccess && !stop; off += (size_t)n * kPipeSlot) {
         const size_t len = std::min(kPipeSlot, bytes - off);

@@ -18,7 +18,7 @@ long long budget = -1;            // bytes that may still be allocated; < 0: no 
 size_t refused_size = 0;          // allocations of exactly this many bytes fail
 bool until_freed = false;         // ... until something of 1 MiB or more has been freed
 size_t total_shown = 0;           // what hipMemGetInfo reports as the device's memory (0: the truth)
-int device_shown = -1;            // what hipGetDevice reports (< 0: the truth)
+int device_shown = -1;            // a current device for the watched thread alone (< 0: the truth)
 size_t held = 0;
 int calls = 0, refusals = 0;
 std::thread::id watched;
@@ -80,13 +80,18 @@ int hipMemGetInfo(size_t *avail, size_t *total) {
 int hipGetDevice(int *d) {
     static auto *f = own<int(int *)>("hipGetDevice");
     const int e = f(d);
-    if (device_shown >= 0) *d = device_shown;
+    if (device_shown >= 0 && std::this_thread::get_id() == watched) *d = device_shown;
     return e;
 }
 int hipSetDevice(int d) {
     static auto *f = own<int(int)>("hipSetDevice");
-    std::lock_guard<std::mutex> lock(mu);
-    if (std::this_thread::get_id() == watched) ++watched_set_device;
+    if (std::this_thread::get_id() == watched) {
+        ++watched_set_device;
+        if (device_shown >= 0) {
+            device_shown = d;
+            return 0;
+        }
+    }
     return f(d);
 }
 
@@ -108,12 +113,13 @@ void limit_show_total(size_t bytes) {
     std::lock_guard<std::mutex> lock(mu);
     total_shown = bytes;
 }
-void limit_show_device(int d) { device_shown = d; }
-void limit_watch_this_thread() {
-    std::lock_guard<std::mutex> lock(mu);
+// the calling thread is watched from here on
+void limit_show_device(int d) {
     watched = std::this_thread::get_id();
     watched_set_device = 0;
+    device_shown = d;
 }
+int limit_shown_device() { return device_shown; }
 int limit_set_device_calls() { return watched_set_device; }
 size_t limit_held() { return held; }
 int limit_calls() { return calls; }

@@ -220,6 +220,18 @@ def short_runs_step_singly():
             assert limit.limit_calls() == calls + 1, (n, form)
 
 
+def current_device_stays():
+    # a large download copies on the caller's thread too: its current device is what it was
+    f = np.random.default_rng(1).standard_normal((60, 70, 64, 19))      # 40 MB: several pieces
+    with GpuGrid(3, 19, 60, 70, 64, precision="fp64", omega=1.2) as g:
+        g.upload_f(f)
+        limit.limit_show_device(-1)
+        assert np.array_equal(g.download_f(), f) and limit.limit_set_device_calls() == 0
+        limit.limit_show_device(1)
+        assert np.array_equal(g.download_f(), f) and limit.limit_shown_device() == 1
+        limit.limit_show_device(-1)
+
+
 if __name__ == "__main__":
     print(f"[memory] {sys.argv[1]}", flush=True)
     globals()[sys.argv[1]]()
