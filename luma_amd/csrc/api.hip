@@ -113,8 +113,14 @@ struct F2Use {
     ~F2Use() { --g->f2_busy; }
 };
 
-// with g->f2_mu held: true when g->f2 is there
+// with g->f2_mu held: true when g->f2 is there.  A run allocates on the device current in the caller; where
+// that is not the grid's, it steps as it can without.
 bool f2_ensure(lumagpu_grid *g) {
+    int device = -1;
+    if (hipGetDevice(&device) != hipSuccess || device != g->device) {
+        (void)hipGetLastError();
+        return false;
+    }
     if (g->f2) return true;
     const size_t bytes = g->ps * g->Q * g->elem;
     size_t avail = 0, total = 0;

@@ -232,6 +232,22 @@ def current_device_stays():
         limit.limit_show_device(-1)
 
 
+def run_from_another_device():
+    # what a run takes for itself would lie on the caller's device: single steps need nothing there
+    case, box = walls(), setups.taylor_green((64, 50, 1), u0=0.04, tau=0.6, dims=2)
+    want = single_steps(case, 18), single_steps(box, 40)
+    with grid(case) as g, grid(box) as h:
+        g.run(9)
+        calls = limit.limit_calls()
+        limit.limit_show_device(1)
+        g.run(9)
+        h.run(40)
+        assert limit.limit_calls() == calls
+        limit.limit_show_device(-1)
+        same(state(g), want[0])
+        same(state(h), want[1])
+
+
 if __name__ == "__main__":
     print(f"[memory] {sys.argv[1]}", flush=True)
     globals()[sys.argv[1]]()
