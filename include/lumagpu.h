@@ -184,11 +184,13 @@ int lumagpu_set_velocity_ramp(lumagpu_grid *g, double ramp_time);
  * reads one and writes the other); shape < 0 frees it and turns the two-step kernel off.
  * Without this call lumagpu_run itself takes several steps per launch where it is faster: two on
  * FP32-shifted D3Q19 grids (labelled ones too), up to twelve on small D2Q9 grids, bit for bit the
- * single steps, in a second array that it allocates when at least half of the free memory
- * stays free and gives back when this library runs short of memory; shape < 0 turns that off
- * as well.  Grids that stop qualifying for the shape asked for (labels or a force set later)
- * step that way or one step at a time.  Long lumagpu_run calls replay a captured graph of two
- * two-step launches. */
+ * single steps, in a second array.  It allocates that when at least half of the free memory stays free
+ * and all grids of the device together keep at most a sixteenth of its memory that way (blocks of
+ * adjoint runs included), and gives it back when this library runs short of memory; otherwise,
+ * or when the current device is not the grid's, it steps singly.  shape < 0 turns that off as
+ * well.  Grids that stop qualifying for the shape asked for (labels or a force set later) step
+ * that way or one step at a time.  Long lumagpu_run calls replay a captured graph of two two-step
+ * launches. */
 int lumagpu_set_temporal_blocking(lumagpu_grid *g, int shape, int zchunk);
 /* L_REYNOLDS_RAMP (definitions.h:204): at the start of every step of this grid and of each grid
  * below it (LBM_multi_opt, GridObj_ops_lbm_optimised.cpp:39-42, before the children's
@@ -381,9 +383,9 @@ int lumagpu_checkpoint_free(lumagpu_checkpoint *ck);
  * ramp, a Reynolds ramp.  Refused (LUMAGPU_EUNSUPPORTED): refinement, z-slabs, gravity,
  * flexible bodies.  Memory: at most ceil(T/K) + K + 1
  * population arrays plus two adjoint arrays (and, while lambda0 is written, one array of
- * Q FP64 values per cell for LUMA's layout).  The grid keeps them for its next run while they are
- * at most a sixteenth of the device's memory; an allocation of this library that would fail
- * without them takes them back. */
+ * Q FP64 values per cell for LUMA's layout).  The grid keeps them for its next run while all
+ * grids of the device together keep at most a sixteenth of its memory; an allocation of this
+ * library that would fail without them takes them back. */
 typedef struct lumagpu_adj_result {
     double J;
     double dJ_domega;

@@ -57,16 +57,13 @@ struct DevBuf {
     }
 };
 
-// The grid keeps its blocks while they are at most a sixteenth of the device's memory.
+// The grid keeps its blocks while there is room for them beside what other grids keep (api.hip).
 void trim_blocks(lumagpu_grid *g) {
-    size_t held = 0, avail = 0, total = 0;
-    for (const auto &b : g->blocks) held += b.bytes;
-    if (hipMemGetInfo(&avail, &total) == hipSuccess && held <= total / 16) {
-        if (held > 0) scratch_listed(g);
-        return;
+    if (!scratch_room(g, 0)) {
+        for (auto &b : g->blocks) (void)hipFree(b.p);
+        g->blocks.clear();
     }
-    for (auto &b : g->blocks) (void)hipFree(b.p);
-    g->blocks.clear();
+    scratch_note(g);
 }
 
 // nlist < 0: every site in one launch; else the plain sites and a list of the others (see AdjMode)

@@ -51,27 +51,42 @@ hipError_t launch_aux(const lumagpu_grid *g, int op, const double *p0, const dou
     }
 }
 
-// ---- the second population array ----------------------------------------------------------------
-// A run allocates it where its kernels take several steps per launch, if that leaves at least half of the
-// free memory free, and keeps it with the grid.  When an allocation of this library fails, the arrays of
-// grids that are not stepping at that moment are given back (g_f2_grids) and it is tried again, so
-// a program's grids fit as they would without them.
+// ---- what runs take for themselves --------------------------------------------------------------
+// A run allocates a second population array where its kernels take several steps per launch, if that leaves
+// at least half of the free memory free; an adjoint run keeps its blocks.  Both stay with the grid for its
+// next run, but all grids of a device together keep at most a sixteenth of its memory (18 GB here: second
+// arrays of 236 M FP32 D3Q19 cells), so that a program's other allocations find what they found without
+// them.  When an allocation of this library fails, the arrays of grids that are not stepping at that
+// moment are given back (g_f2_grids) and it is tried again.
 std::mutex g_f2_grids_mu;
-std::vector<lumagpu_grid *> g_f2_grids;
+std::vector<lumagpu_grid *> g_f2_grids;   // the grids that keep any; their `scratch` says how much
+
+size_t f2_bytes(const lumagpu_grid *g) { return g->ps * g->Q * g->elem; }
+
+// what g keeps, with its f2_mu held
+size_t scratch_of(const lumagpu_grid *g) {
+    size_t n = g->f2_auto ? f2_bytes(g) : 0;
+    for (const auto &b : g->blocks) n += b.bytes;
+    return n;
+}
+
+// with g_f2_grids_mu held: g is to keep n bytes
+void scratch_set(lumagpu_grid *g, size_t n) {
+    g->scratch = n;
+    const auto it = std::find(g_f2_grids.begin(), g_f2_grids.end(), g);
+    if (n > 0 && it == g_f2_grids.end()) g_f2_grids.push_back(g);
+    if (n == 0 && it != g_f2_grids.end()) g_f2_grids.erase(it);
+}
 
 // the arrays of grids that no run holds, back to the device.  f2_mu is recursive: on the thread of a run
 // its own grid's lock is no obstacle, and f2_busy says that its second array is in use.
 void f2_give_back() {
     std::lock_guard<std::mutex> lock(g_f2_grids_mu);
-    for (size_t k = 0; k < g_f2_grids.size();) {
-        lumagpu_grid *o = g_f2_grids[k];
-        if (!o->f2_mu.try_lock()) {
-            ++k;
-            continue;
-        }
+    const std::vector<lumagpu_grid *> grids = g_f2_grids;
+    for (lumagpu_grid *o : grids) {
+        if (!o->f2_mu.try_lock()) continue;
         if (o->stream) (void)hipStreamSynchronize(o->stream);
-        const bool busy = o->f2_busy != 0;
-        if (!busy) {
+        if (!o->f2_busy) {
             if (o->f2_auto) {
                 (void)hipFree(o->f2);
                 o->f2 = nullptr;
@@ -84,22 +99,31 @@ void f2_give_back() {
             else (void)hipFree(b.p);
         }
         o->blocks = std::move(kept);
+        scratch_set(o, scratch_of(o));
         o->f2_mu.unlock();
-        if (busy) ++k;
-        else g_f2_grids.erase(g_f2_grids.begin() + k);
     }
-}
-
-void f2_forget(lumagpu_grid *g) {
-    std::lock_guard<std::mutex> lock(g_f2_grids_mu);
-    g_f2_grids.erase(std::remove(g_f2_grids.begin(), g_f2_grids.end(), g), g_f2_grids.end());
 }
 
 }  // namespace
 namespace lumagpu {
-void scratch_listed(lumagpu_grid *g) {
+void scratch_note(lumagpu_grid *g) {
     std::lock_guard<std::mutex> lock(g_f2_grids_mu);
-    if (std::find(g_f2_grids.begin(), g_f2_grids.end(), g) == g_f2_grids.end()) g_f2_grids.push_back(g);
+    scratch_set(g, scratch_of(g));
+}
+
+bool scratch_room(lumagpu_grid *g, size_t more) {
+    size_t avail = 0, total = 0;
+    if (hipMemGetInfo(&avail, &total) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    std::lock_guard<std::mutex> lock(g_f2_grids_mu);
+    size_t n = scratch_of(g) + more;
+    for (const lumagpu_grid *o : g_f2_grids)
+        if (o != g && o->device == g->device) n += o->scratch;
+    if (n > total / 16 || more > avail / 2) return false;
+    scratch_set(g, scratch_of(g) + more);
+    return true;
 }
 }  // namespace lumagpu
 namespace {
@@ -122,16 +146,15 @@ bool f2_ensure(lumagpu_grid *g) {
         return false;
     }
     if (g->f2) return true;
-    const size_t bytes = g->ps * g->Q * g->elem;
-    size_t avail = 0, total = 0;
-    if (hipMemGetInfo(&avail, &total) != hipSuccess || bytes > avail / 2 || hipMalloc(&g->f2, bytes) != hipSuccess) {
+    if (!scratch_room(g, f2_bytes(g))) return false;
+    if (hipMalloc(&g->f2, f2_bytes(g)) != hipSuccess) {
         (void)hipGetLastError();
         g->f2 = nullptr;
+        scratch_note(g);
         return false;
     }
     g->f2_auto = 1;
     g->pair_synced = 0;
-    scratch_listed(g);
     return true;
 }
 
@@ -1128,7 +1151,10 @@ int lumagpu_grid_destroy(lumagpu_grid *g) {
     if (g->counted) host_copy_grid_gone();
     (void)hipHostFree(g->pin);
     (void)hipFree(g->f);
-    f2_forget(g);
+    {
+        std::lock_guard<std::mutex> lock(g_f2_grids_mu);
+        scratch_set(g, 0);
+    }
     (void)hipFree(g->f2);
     for (auto &b : g->blocks) (void)hipFree(b.p);
     (void)hipFree(g->pair_deep);
@@ -1650,6 +1676,7 @@ int lumagpu_set_temporal_blocking(lumagpu_grid *g, int shape, int zchunk) {
         }
         g->f2 = nullptr;
         g->fuse_shape = -1;
+        scratch_note(g);
         return 0;
     }
     int tx, ty;
@@ -1668,6 +1695,7 @@ int lumagpu_set_temporal_blocking(lumagpu_grid *g, int shape, int zchunk) {
         return fail(LUMAGPU_ENOMEM, "second population array");
     }
     g->f2_auto = 0;   // asked for: no longer one to give back
+    scratch_note(g);
     g->pair_synced = 0;
     g->fuse_off = 0;
     g->fuse_shape = shape;

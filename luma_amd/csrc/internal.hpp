@@ -37,6 +37,7 @@ struct lumagpu_grid {
         int used;
     };
     std::vector<Block> blocks;
+    size_t scratch = 0;               // bytes of f2 (f2_auto) and blocks, as last noted (api.hip)
     int f2_busy = 0;                  // a run is using f2 (see F2Use)
     int fuse_off = 0;                 // lumagpu_set_temporal_blocking turned several steps per launch off
     // two steps per launch on a large 3D grid (fused_kernels.hpp): the deep cells, the cells around the
@@ -126,8 +127,10 @@ namespace lumagpu {
 // thread-local message behind lumagpu_last_error()
 int fail(int code, const std::string &msg);
 
-// listed among the grids whose own arrays (f2, blocks) can be taken back while nothing runs on them
-void scratch_listed(lumagpu_grid *g);
+// What runs of a grid take for themselves (f2, blocks; api.hip), with its f2_mu held: note what it keeps now;
+// and whether it may keep `more` bytes beyond that, which then count as kept
+void scratch_note(lumagpu_grid *g);
+bool scratch_room(lumagpu_grid *g, size_t more);
 // hipMalloc that, short of memory, first takes back what runs allocated for themselves (api.hip)
 hipError_t dev_malloc(void **p, size_t bytes);
 template <class T>

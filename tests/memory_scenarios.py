@@ -248,6 +248,49 @@ def run_from_another_device():
         same(state(h), want[1])
 
 
+def kept_memory_is_bounded():
+    # second arrays and adjoint blocks of all grids together: a sixteenth of the device's memory
+    case = walls()
+    f2 = (-(-70 ** 3 // 256) * 256) * 19 * 4          # and the planes' padding: below 1 % more
+    limit.limit_show_total(int(16 * 1.5 * f2))
+    want = single_steps(case, 9)
+    with grid(case) as a:
+        before = limit.limit_held()
+        a.run(9)
+        assert limit.limit_held() > before + f2, "no second array"
+        with grid(case) as b:
+            state(b)                                  # its staging
+            before = limit.limit_held()
+            b.run(9)
+            assert limit.limit_held() == before, "a second array beyond the bound"
+            same(state(b), want)
+            a.close()
+            b.init_equilibrium(case.rho, case.u)
+            before = limit.limit_held()
+            b.run(9)
+            assert limit.limit_held() > before + f2
+            same(state(b), want)
+    box = setups.channel_2d(90, 40, 10.0, 0.04, 20.0)
+    grads = []
+    for total in (1 << 40, 16 << 10):
+        limit.limit_show_total(total)
+        with grid(box, "fp64") as g:
+            g.ibm_add_body(setups.circle_markers((3.0, 2.0, 0.0), 0.5, box.info["dh"]))
+            g.ibm_initialise()
+            start = g.checkpoint()
+            state(g)
+            before = limit.limit_held()
+            for _ in range(2):
+                g.restore(start)
+                grads.append(g.adj_run(20, 6, initial=True))
+                if total < 1 << 40:
+                    assert limit.limit_held() == before, "blocks beyond the bound"
+            assert total < 1 << 40 or limit.limit_held() > before
+            GpuGrid.free_checkpoint(start)
+    for r in grads[1:]:
+        assert r["J"] == grads[0]["J"] and np.array_equal(r["lambda0"], grads[0]["lambda0"])
+
+
 if __name__ == "__main__":
     print(f"[memory] {sys.argv[1]}", flush=True)
     globals()[sys.argv[1]]()

@@ -14,7 +14,8 @@ HERE = Path(__file__).resolve().parent
 @pytest.mark.parametrize("name", ["labels_cut_short", "sets_do_not_fit", "sets_take_back", "others_give_way",
                                   "epsilon_on_the_host", "position_gradient_on_the_host",
                                   "force_set_again", "labels_set_again", "short_runs_step_singly",
-                                  "current_device_stays", "run_from_another_device"])
+                                  "current_device_stays", "run_from_another_device",
+                                  "kept_memory_is_bounded"])
 def test_scenario(name):
     assert (HERE / "cpp" / "_build" / "alloc_limit.so").exists(), "build it with __graft_entry__.build()"
     print(f"[memory] {name}", flush=True)
