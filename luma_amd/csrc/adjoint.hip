@@ -809,6 +809,9 @@ extern "C" int lumagpu_adj_run(lumagpu_grid *g, int nsteps, int checkpoint_every
     const int r = g->d.precision == LUMAGPU_FP64
                       ? adj_run<P64>(g, nsteps, checkpoint_every, dir, backward, res, dJ_dpos, lambda0)
                       : adj_run<P32S>(g, nsteps, checkpoint_every, dir, backward, res, dJ_dpos, lambda0);
+    // a run that ended early may have kernels queued on the blocks that the next one takes, and writes
+    // from the host without regard to this stream
+    if (r) (void)hipStreamSynchronize(g->stream);
     trim_blocks(g);
     return r;
 }

@@ -291,6 +291,37 @@ def kept_memory_is_bounded():
         assert r["J"] == grads[0]["J"] and np.array_equal(r["lambda0"], grads[0]["lambda0"])
 
 
+def gradient_cut_short():
+    # a gradient that runs out of memory between its forward and its reversed steps, then the same again
+    case = setups.channel_2d(90, 40, 10.0, 0.04, 20.0)
+    with grid(case, "fp64") as g:
+        g.ibm_add_body(setups.circle_markers((3.0, 2.0, 0.0), 0.5, case.info["dh"]))
+        g.ibm_initialise()
+        start = g.checkpoint()
+        limit.limit_refuse_size(3 * 8 * 90 * 40)      # the force adjoint
+        for _ in range(3):
+            g.restore(start)
+            try:
+                g.adj_run(20, 6, initial=True)
+                raise AssertionError("allocated")
+            except LumaGpuError as e:
+                assert "adjoint buffer" in str(e)
+        limit.limit_refuse_size(0)
+        got = []
+        for _ in range(2):
+            g.restore(start)
+            got.append(g.adj_run(20, 6, initial=True))
+        GpuGrid.free_checkpoint(start)
+    with grid(case, "fp64") as g:
+        g.ibm_add_body(setups.circle_markers((3.0, 2.0, 0.0), 0.5, case.info["dh"]))
+        g.ibm_initialise()
+        want = g.adj_run(20, 6, initial=True)
+    assert np.abs(want["lambda0"]).max() > 0
+    for r in got:
+        for k in want:
+            assert np.array_equal(r[k], want[k]), k
+
+
 if __name__ == "__main__":
     print(f"[memory] {sys.argv[1]}", flush=True)
     globals()[sys.argv[1]]()
