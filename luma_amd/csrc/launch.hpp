@@ -261,7 +261,7 @@ void with_bool(bool b, F &&f) {
 template <int Q, class P>
 hipError_t launch_list_p(const StepArgs &a, bool odd, bool store, const int *cells, const uint64_t *links, int n,
                          hipStream_t s) {
-    if (n <= 0) return hipSuccess;
+    if (n <= 0) return hipGetLastError();   // of the launches before it
     const dim3 g((unsigned)((n + 63) / 64));
     with_bool(odd, [&](auto o) {
         with_bool(store, [&](auto st) {

@@ -1,6 +1,7 @@
 // A stand-in for the allocation calls of the HIP runtime that libluma_amd.so makes, loaded before it
 // with RTLD_GLOBAL: each goes on to the runtime's own unless a limit set here refuses it.  So a test
-// can run the library short of device memory without filling the device.
+// can run the library short of device memory without filling the device.  And its launches: one can be
+// made to fail.
 #include <dlfcn.h>
 
 #include <cstddef>
@@ -21,6 +22,8 @@ size_t total_shown = 0;           // what hipMemGetInfo reports as the device's 
 int device_shown = -1;            // a current device for the watched thread alone (< 0: the truth)
 size_t held = 0;
 int calls = 0, refusals = 0;
+int failing_launch = 0;           // this launch from now fails (1: the next); 0: none
+int launch_error = 0;             // what hipGetLastError then reports, once
 std::thread::id watched;
 int watched_set_device = 0;
 
@@ -95,6 +98,22 @@ int hipSetDevice(int d) {
     return f(d);
 }
 
+struct Dim3 {
+    unsigned x, y, z;
+};
+int hipLaunchKernel(const void *fn, Dim3 grid, Dim3 block, void **args, size_t lds, void *stream) {
+    static auto *f = own<int(const void *, Dim3, Dim3, void **, size_t, void *)>("hipLaunchKernel");
+    if (failing_launch > 0 && --failing_launch == 0) return launch_error = 719;   // hipErrorLaunchFailure
+    return f(fn, grid, block, args, lds, stream);
+}
+int hipGetLastError() {
+    static auto *f = own<int()>("hipGetLastError");
+    const int e = f(), injected = launch_error;
+    launch_error = 0;
+    return injected ? injected : e;
+}
+
+void limit_fail_launch(int nth) { failing_launch = nth; }
 void limit_budget(long long bytes) {
     std::lock_guard<std::mutex> lock(mu);
     budget = bytes;

@@ -1,4 +1,4 @@
-"""Programs that run the library short of device memory, one per name, each in a process of its own
+"""Programs that run the library short of device memory, or with a failing launch, one per name, each in a process of its own
 (test_gpu_memory.py): the limiter has to be loaded before the library.  A scenario raises where it
 fails and prints its name at the end."""
 import ctypes as C
@@ -320,6 +320,22 @@ def gradient_cut_short():
     for r in got:
         for k in want:
             assert np.array_equal(r[k], want[k]), k
+
+
+def launch_errors_are_reported():
+    # a grid of plain sites alone steps in one launch, without a list after it
+    shape = (104, 101, 102)
+    case = setups.taylor_green(shape, u0=0.04, tau=0.7)
+    case.forced, case.force = True, np.full(shape + (3,), 1e-6)
+    with GpuGrid.from_case(case, "fp64") as g:
+        g.run(2)
+        limit.limit_fail_launch(1)
+        try:
+            g.LBM_multi_opt()
+            raise AssertionError("a failed launch was taken for a step")
+        except LumaGpuError as e:
+            assert "launch" in str(e)
+        assert g.t == 2
 
 
 if __name__ == "__main__":

@@ -15,7 +15,8 @@ HERE = Path(__file__).resolve().parent
                                   "epsilon_on_the_host", "position_gradient_on_the_host",
                                   "force_set_again", "labels_set_again", "short_runs_step_singly",
                                   "current_device_stays", "run_from_another_device",
-                                  "kept_memory_is_bounded", "gradient_cut_short"])
+                                  "kept_memory_is_bounded", "gradient_cut_short",
+                                  "launch_errors_are_reported"])
 def test_scenario(name):
     assert (HERE / "cpp" / "_build" / "alloc_limit.so").exists(), "build it with __graft_entry__.build()"
     print(f"[memory] {name}", flush=True)
