@@ -1,10 +1,12 @@
-"""Labels set again on a grid large enough for the site list (2^20 cells): the list and its link words
-are those of a grid that never had other labels, whatever the earlier calls left."""
+"""Grids large enough for the site list (2^20 cells): with labels set again, the list and its link words
+are those of a grid that never had other labels, whatever the earlier calls left; and the outlet's
+rows, which the list steps by their link words' outlet bits, against the oracle."""
 import numpy as np
 import pytest
 
 from luma_amd import setups
 from luma_amd.grid import GpuGrid
+from oracle.oracle import OracleGrid
 
 pytestmark = pytest.mark.gpu
 
@@ -60,3 +62,29 @@ def test_same_labels_at_other_positions():
         b.set_labels(lt, x, inside, z)
         for p, q in zip(_after(a, rho, u), _after(b, rho, u)):
             assert np.array_equal(p, q)
+
+
+def test_outlet_rows():
+    # every fluid and outlet site up to the last column, behind fluid rows as the flow has them and with
+    # a solid block on the way
+    case = setups.uniform_inflow_3d(131, 92, 88, 0.03, 0.6)
+    case.lattyp[60:67, 30:37, 20:31] = setups.SOLID
+    case.forced = False
+    case.u[..., 1] = 0.01 * np.sin(np.arange(92))[None, :, None]
+    case.u[..., 2] = 0.01 * np.cos(0.3 * np.arange(131))[:, None, None]
+    case.u[0] = (0.03, 0.0, 0.0)        # the inlet's, which is what its sites hold
+    case.u[case.lattyp == setups.SOLID] = 0.0
+    o = OracleGrid(3, 19, case.N, case.M, case.K, omega=case.omega, regularised=False, edges=case.edges)
+    o.set_labels(case.lattyp)
+    o.set_positions(case.xpos, case.ypos, case.zpos)
+    o.set_inlet(case.ux_in, case.uy_in, case.uz_in)
+    o.init_feq(case.rho, case.u)
+    o.run(5, 8)
+    print("[lists] outlet", flush=True)
+    with GpuGrid.from_case(case, "fp64", store_macro=True) as g:
+        g.run(5)
+        got = (g.download_f(),) + g.download_macro()
+    m = (case.lattyp == setups.FLUID) | (case.lattyp == setups.EXTRAP_RIGHT)
+    assert m[-1].any()
+    for a, b in zip(got, (o.get_f(),) + o.get_macro()):
+        assert np.array_equal(a[m], b[m])
