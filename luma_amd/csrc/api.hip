@@ -511,7 +511,8 @@ int run_fused_graph(lumagpu_grid *g, int reps) {
 
 // Small 2D grids take several steps per launch (k_multi2d): one level, no bodies, nothing that
 // changes from step to step, and site types whose sources the window holds.  2^18 cells: above,
-// a step fills the chip by itself, and the window's repeated cells cost more than launches.
+// a step fills the chip by itself, and the window's repeated cells cost more than launches.  FP64 and
+// FP32-shifted storage: the kernel is built for these two, FP16-shifted grids of this size step singly.
 bool multi_ok(const lumagpu_grid *g) {
     return !g->fuse_off && g->Q == 9 && (g->d.precision == LUMAGPU_FP64 || g->d.precision == LUMAGPU_FP32S) && !g->parent &&
            g->kids.empty() && ibm_marker_count(g) == 0 && !g->gravity_on && !(g->ramp_time > 0.0) &&
@@ -557,8 +558,11 @@ int run_multi(lumagpu_grid *g, int n, int *done) {
 // step that is the same kernels every time (no gravity reset, no Reynolds ramp), site types of the
 // list kernels, bodies rigid and settled (their supports flagged), outlet sources written by the
 // step.  us per step, single -> pairs: periodic boxes 32^3 10.7 -> 3.4, 64^3 9.4 -> 6.5, 128^3 53 -> 37,
-// 160^3 108 -> 77; walls with a set force 48^3 11.3 -> 13.1, 64^3 14.2 -> 14.9, 65^3 22.5 -> 20.2,
-// 96^3 42 -> 29, 160^3 129 -> 106: labelled grids, with three launches a pair, from 2^18 cells.
+// 160^3 108 -> 77.  Labelled grids have three launches a pair and gain later: walls with a set force
+// 48^3 11.3 -> 13.1, 64^3 14.2 -> 14.9, 65^3 22.9 -> 20.5, 96^3 42 -> 29, 160^3 129 -> 106.  Above 2^18 cells:
+// there both take the same on rows of whole 64s (64 x 64 x 66 15.9 -> 15.5, 128 x 64 x 33 15.8 -> 15.8,
+// 192 x 48 x 29 15.9 -> 16.3, 512 x 32 x 17 16.4 -> 16.5; rows of 1024, 15.9 -> 17.7, are the worst) and
+// pairs less on others (300 x 30 x 30 21.3 -> 17.5).
 constexpr size_t kPairMin = size_t(1) << 15, kPairMinLabelled = (size_t(1) << 18) + 1;
 bool pair_ok(const lumagpu_grid *g) {
     if (g->fuse_off || g->Q != 19 || g->d.precision != LUMAGPU_FP32S || g->parent || !g->kids.empty() || g->zslab ||

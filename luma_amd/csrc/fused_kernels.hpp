@@ -392,7 +392,7 @@ hipError_t launch_fused2_p(int shape, const StepArgs &a, void *dst, int zc, bool
 // leaves the even results of S1 in their cells' slots; step 2 writes the slots that deep cells own
 // in the odd layout, so it comes after 1 and spares every slot that step 3 reads, since those are
 // owned by S.  A slot of neither kind belongs to a solid, forced-equilibrium or other site that
-// never steps: it holds what it held (pair_sync copies those after a change of state or labels),
+// never steps: it holds what it held (run_pairs copies those after a change of state or labels),
 // or what S pushes there.
 
 // deep: plain, and every neighbour plain; with bodies, none of them a support (forced)

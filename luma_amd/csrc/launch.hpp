@@ -230,12 +230,16 @@ inline dim3 cell_grid(int nx, int ny, int nz) {
     return dim3((nx + b.x - 1) / b.x, ny, nz);
 }
 
-// How the grid kernels of a step take the cells.  Row blocks where one of cell_block's sizes
-// divides the row; else linear order, which leaves no lane idle and no line split between two
-// non-temporal accesses.  Even / odd kernel, us per step, by rows -> linear: 250 x 190 x 175 FP16
+// How the grid kernels of a step take the cells.  Linear order leaves no lane idle and no line split
+// between two non-temporal accesses.  Even / odd kernel, us per step, by rows -> linear: 250 x 190 x 175 FP16
 // 217 / 166 -> 102 / 146; 200 x 171 x 150 FP64 334 / 262 -> 279 / 268; labelled plain sites
 // 180 x 131 x 150 FP32 130 / 116 -> 95 / 114, 288 x 96 x 96 FP32 (aligned rows, a block of 32
-// lanes at the end of each) 105 / 107 -> 77 / 75.
+// lanes at the end of each) 105 / 107 -> 77 / 75.  Rows that one of cell_block's other sizes divides gain
+// little or nothing (4 M cells, both kernels' mean, FP64 / FP16: rows of 64 206 / 59 -> 197 / 54, of 192
+// 206 / 55 -> 202 / 56, of 320 263 / 77 -> 201 / 59, of 576 206 / 58 -> 202 / 58).  Rows of whole 128s stay
+// with blocks of 128 or 256: unlabelled, linear order is as fast or up to 5 % faster there (FP64 rows of 128
+// 199.5 -> 197.7, 256 199.2 -> 199.0, 384 210 -> 200), but labelled FP64 grids lose 2 % with it
+// (128 228 -> 233, 256 226 -> 231, 512 232 -> 238).
 template <class P>
 CellOrder cell_order(const StepArgs &a) {
     // 2^31 cells bound the linear index; the tangent forms step small grids

@@ -120,8 +120,10 @@ inline long multi2d_blocks(int nx, int ny, int H) {
 }
 
 // Steps per launch for up to n (even) steps: the H whose launch, rounds of blocks over the
-// 256 CUs and window steps cost least per step.  The two constants are what launches of H = 8
-// (256 x 256, one block per CU) and H = 12 (64 x 64) take together with their lids.
+// 256 CUs and window steps cost least per step.  The two constants lie between boxes and lids, whose
+// sites run after the fluid of their wave: a launch of H = 8 on 256 x 256 (one block per CU) takes 14.7 us
+// FP32 on a box and 23.5 with a lid (17.1 by the constants), 27.4 and 33.7 FP64 (31.5); of H = 12 on
+// 48 x 48 14.6 and 28.7 us FP32 (21.9), 28 and 39 FP64 (43.5).
 inline int plan_multi2d(int nx, int ny, int n, bool fp64) {
     const double launch_us = 7.5, step_us = fp64 ? 3.0 : 1.2;
     int best = 0;
