@@ -221,8 +221,9 @@ void ds_chain(const lumagpu_grid *g, const Body &b, const double *dsbar, double 
 
 // epsilon_chain on the device for a system of kLuDeviceMin markers and more: assembly, LU and the sums
 // over near pairs are O(n^2) and O(n^3) work that one host thread took 94 ms for at 804 markers
-// (here 6.5 ms); the O(n^2) substitutions stay on the host.  first: the system's first marker
-// in the grid's marker arrays; sdd: the gradients of the delta weights.
+// (here 6.5 ms); the O(n^2) substitutions stay on the host, and so does the whole solve of a sparse
+// matrix (kLuSparse).  first: the system's first marker in the grid's marker arrays; sdd: the gradients of
+// the delta weights.  LUMAGPU_ENOMEM before anything of the caller's has been written.
 int epsilon_chain_device(lumagpu_grid *g, const std::vector<const Marker *> &ms, int first, const double *sdd,
                          const double *epsbar, double *dsbar, double *xg) {
     const IbmSystem *s = g->ibm;
