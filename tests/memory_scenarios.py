@@ -291,6 +291,21 @@ def kept_memory_is_bounded():
         assert r["J"] == grads[0]["J"] and np.array_equal(r["lambda0"], grads[0]["lambda0"])
 
 
+def second_array_refused():
+    # a second array that would take more than half of what is free: single steps
+    case, box = walls(), setups.taylor_green((64, 50, 1), u0=0.04, tau=0.6, dims=2)
+    want = single_steps(case, 9), single_steps(box, 40)
+    with grid(case) as g, grid(box) as h:
+        for x, cells, q, steps in ((g, 70 ** 3, 19, 9), (h, 64 * 50, 9, 40)):
+            calls = limit.limit_calls()
+            limit.limit_budget(int(1.9 * cells * q * 4))
+            x.run(steps)
+            assert limit.limit_calls() == calls
+            limit.limit_budget(-1)
+        same(state(g), want[0])
+        same(state(h), want[1])
+
+
 def gradient_cut_short():
     # a gradient that runs out of memory between its forward and its reversed steps, then the same again
     case = setups.channel_2d(90, 40, 10.0, 0.04, 20.0)
