@@ -404,14 +404,15 @@ int adj_run(lumagpu_grid *g, int nsteps, int every, const double dir[3], int bac
         g->f_to = nullptr;
         g->xr_tape = nullptr;
         g->xr_ready = 0;
-        // the end state's sites that never step, when its last step (even) pushed nothing to them
-        if (forward && !g->d.regularised && len >= 2 && tpar[len - 1] != 0) {
+        // the end state's slots that no step wrote: those of forced-equilibrium sites
+        if (forward && !g->d.regularised && len >= 2) {
             using S = typename P::S;
             const S *from = static_cast<const S *>(state(seg, len - 1));
             const unsigned nb = (unsigned)((g->ncell + 255) / 256);
             const StepArgs a = make_args(g);
-            if (g->Q == 9) k_adj_carry<9, S><<<nb, 256, 0, g->stream>>>(a, from, static_cast<S *>(end));
-            else k_adj_carry<19, S><<<nb, 256, 0, g->stream>>>(a, from, static_cast<S *>(end));
+            const int odd = tpar[len - 1] == 0;
+            if (g->Q == 9) k_adj_carry<9, S><<<nb, 256, 0, g->stream>>>(a, from, static_cast<S *>(end), odd);
+            else k_adj_carry<19, S><<<nb, 256, 0, g->stream>>>(a, from, static_cast<S *>(end), odd);
             HIP_TRY(hipGetLastError());
         }
         return 0;

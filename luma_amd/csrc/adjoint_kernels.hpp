@@ -714,10 +714,12 @@ static __global__ void k_adj_objective(IbmArgs ib, double dx, double dy, double 
     if (lane == 0) acc[0] += s * invT;
 }
 
-// A forced-equilibrium velocity site never steps: its slots hold what its neighbours pushed in the
-// last odd step, and a state reached along the tape by an even step has them in the state before.
+// A forced-equilibrium velocity site never steps, so the slots it would write keep what stepping in place
+// leaves in them, and along the tape they are in the state before the last step.  After an even step: its own
+// slots that its neighbours pushed to in the odd step before.  After an odd step: the slots of its
+// neighbours that its pushes would fill, with what their even step wrote.
 template <int Q, class S>
-__global__ __launch_bounds__(256) void k_adj_carry(StepArgs a, const S *from, S *to) {
+__global__ __launch_bounds__(256) void k_adj_carry(StepArgs a, const S *from, S *to, int odd) {
     using L = Lattice<Q>;
     const size_t cell = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (cell >= a.ncell || (a.flags[cell] & kTypeMask) != kVelocity) return;
@@ -727,8 +729,11 @@ __global__ __launch_bounds__(256) void k_adj_carry(StepArgs a, const S *from, S 
     nb.init(x, y, z, a.nx, a.ny, a.nz);
     static_for<Q>([&](auto vc) {
         constexpr int v = decltype(vc)::value;
-        const int t = a.flags[nb.at(-L::c(v, 0), -L::c(v, 1), -L::c(v, 2), a.nx, a.ny)] & kTypeMask;
-        if (t == kFluid || t == kExtrapRight) to[(size_t)v * a.ps + cell] = from[(size_t)v * a.ps + cell];
+        const int s = odd ? 1 : -1;
+        const size_t n = nb.at(s * L::c(v, 0), s * L::c(v, 1), s * L::c(v, 2), a.nx, a.ny);
+        const int t = a.flags[n] & kTypeMask;
+        const size_t slot = (size_t)v * a.ps + (odd ? n : cell);
+        if (t == kFluid || t == kExtrapRight) to[slot] = from[slot];
     });
 }
 

@@ -93,3 +93,27 @@ def test_gradients_and_tape(build):
     pred = float((adj["lambda0"] * dirn).sum())
     print("dJ/df0 . d", pred, fd, flush=True)
     assert abs(pred - fd) <= 1e-4 * abs(fd)
+
+
+# the state a gradient leaves is that of plain steps at every site, those of a forced-equilibrium inlet (which
+# never step) included: last segments of one, two and more steps, ending on either kind of step, from either
+# layout
+@pytest.mark.parametrize("dims,form", [(2, "fp64"), (2, "fp32s"), (3, "fp64"), (3, "fp32s")])
+def test_state_at_sites_that_never_step(dims, form):
+    if dims == 2:
+        case = setups.channel_2d(60, 30, 10.0, 0.04, 20.0, regularised=False)
+        case.lattyp[20:24, 10:16] = setups.SOLID
+        case.lattyp[30:33, 4:9] = setups.VELOCITY
+    else:
+        case = setups.uniform_inflow_3d(24, 12, 11, 0.03, 0.6)
+        case.lattyp[10:13, 3:7, 2:5] = setups.VELOCITY
+    for before, t, every in ((0, 3, 4), (1, 2, 7), (0, 2, 2), (1, 3, 3), (0, 5, 2), (0, 6, 5), (1, 7, 4), (0, 1, 1)):
+        print(f"[adjoint] state {dims}D {form} {before} {t} {every}", flush=True)
+        with GpuGrid.from_case(case, form) as a, GpuGrid.from_case(case, form) as b:
+            for g in (a, b):
+                for _ in range(before):
+                    g.LBM_multi_opt()
+            a.adj_run(t, every, initial=True)
+            for _ in range(t):
+                b.LBM_multi_opt()
+            assert a.t == b.t and np.array_equal(a.download_f(), b.download_f()), (before, t, every)
