@@ -4,6 +4,7 @@ fails and prints its name at the end."""
 import ctypes as C
 import dataclasses
 import sys
+import threading
 from pathlib import Path
 
 import numpy as np
@@ -289,6 +290,46 @@ def kept_memory_is_bounded():
             GpuGrid.free_checkpoint(start)
     for r in grads[1:]:
         assert r["J"] == grads[0]["J"] and np.array_equal(r["lambda0"], grads[0]["lambda0"])
+
+
+def threads_short_of_memory():
+    # one thread steps while another's grids come, run and go in memory that holds one second array less
+    case = walls(66)
+    want = {n: single_steps(case, n) for n in (9, 18, 27)}
+    size = 66 ** 3 * 19 * 4
+    with grid(case) as a, grid(case) as b:
+        state(a)
+        limit.limit_budget(int(7.2 * size))       # b's grids (f, rho, u, force, staging): 5 x size, and two arrays
+        out, errors = {}, []
+
+        def stepping():
+            try:
+                for n in (9, 18, 27):
+                    a.run(9)
+                    out[n] = state(a)
+            except Exception as e:
+                errors.append(e)
+
+        def coming_and_going():
+            try:
+                for _ in range(4):
+                    b.init_equilibrium(case.rho, case.u)
+                    b.run(9)
+                    same(state(b), want[9])
+                    with grid(case) as c:
+                        c.run(9)
+                        same(state(c), want[9])
+            except Exception as e:
+                errors.append(e)
+        threads = [threading.Thread(target=t) for t in (stepping, coming_and_going)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        limit.limit_budget(-1)
+    assert not errors, errors
+    for n in out:
+        same(out[n], want[n])
 
 
 def second_array_refused():

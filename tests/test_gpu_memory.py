@@ -16,7 +16,8 @@ HERE = Path(__file__).resolve().parent
                                   "force_set_again", "labels_set_again", "short_runs_step_singly",
                                   "current_device_stays", "run_from_another_device",
                                   "kept_memory_is_bounded", "gradient_cut_short",
-                                  "launch_errors_are_reported", "second_array_refused"])
+                                  "launch_errors_are_reported", "second_array_refused",
+                                  "threads_short_of_memory"])
 def test_scenario(name):
     assert (HERE / "cpp" / "_build" / "alloc_limit.so").exists(), "build it with __graft_entry__.build()"
     print(f"[memory] {name}", flush=True)
