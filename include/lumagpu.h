@@ -89,7 +89,9 @@ int lumagpu_grid_destroy(lumagpu_grid *g);
 int lumagpu_grid_add_child(lumagpu_grid *parent, lumagpu_grid *child);
 
 /* ---- state upload / download --------------------------------------------------------- */
-/* LatTyp + XPos/YPos/ZPos (GridObj_init_grids.cpp:234-273; labels of LBM_initBoundLab) */
+/* LatTyp + XPos/YPos/ZPos (GridObj_init_grids.cpp:234-273; labels of LBM_initBoundLab).  After a call
+ * that failed half-way (LUMAGPU_ENOMEM) the grid's steps return LUMAGPU_ESTATE until labels or
+ * force have been set. */
 int lumagpu_set_labels(lumagpu_grid *g, const int *lattyp, const double *xpos, const double *ypos,
                        const double *zpos);
 /* ux_in/uy_in/uz_in, one value per j (GridObj_init_grids.cpp:1322-1360) */
